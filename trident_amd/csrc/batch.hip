@@ -967,18 +967,21 @@ __device__ __forceinline__ uint2 row_entry(float u, int row0) {
 // 2^-126 first, so it never sees a denormal (a larger E only raises the bound).  A_lo (1 + 2^-21)
 // >= A: vec_Ar holds A rounded down by 1e-13 and then to float32.
 //
-// Each lane keeps the M smallest bounds of its rows (M = 4 when K <= 16: a query's rows are
-// spread over 16 lanes, and the merged lists' K-th entry is the exact K-th smallest unless one
-// lane held more than M of them, in which case it is still an upper bound of it).
+// Each lane keeps the M smallest bounds of its rows (M = 4 when K <= 16, 8 when K <= 64, else 16:
+// a query's rows are spread over 16 lanes, and the merged lists' K-th entry is the exact K-th
+// smallest unless one lane held more than M of them, in which case it is still an upper bound
+// of it).
 template <int KS, int M>
 __global__ __launch_bounds__(256) void ub_scan_kernel(BatchArgs a) {
     // The code buffers double as the end-of-unit list exchange (after a barrier).
     constexpr int BV = block_vectors(KS);
     constexpr int NBC = BV == 64 ? 2 : kWideAhead + 1;  // code buffers
-    constexpr int kCodeU4 = NBC * KS * 4 * BV, kUblU4 = kWavesPerBlock * kWaveQ * kWave / 4;
+    // a query column's kept bounds of one wave (K > 16: one more float against bank conflicts)
+    constexpr int kUblRow = M <= 4 ? kUbList : 4 * M + 1;
+    constexpr int kCodeU4 = NBC * KS * 4 * BV, kUblU4 = kWavesPerBlock * kWaveQ * kUblRow / 4;
     __shared__ uint4 s_big[kCodeU4 > kUblU4 ? kCodeU4 : kUblU4];
     uint4(*s_codes)[KS * 4 * BV] = reinterpret_cast<uint4(*)[KS * 4 * BV]>(s_big);
-    float(*s_ubl)[kWaveQ * kWave] = reinterpret_cast<float(*)[kWaveQ * kWave]>(s_big);
+    float(*s_ubl)[kWaveQ * kUblRow] = reinterpret_cast<float(*)[kWaveQ * kUblRow]>(s_big);
     // Row scalars: double-buffered with the codes, or (wide layout) a ring of 8 that also
     // holds the block its replica waves finish one block late.  s_part: the replicas' partial
     // sums.
@@ -1240,14 +1243,17 @@ __global__ __launch_bounds__(256) void ub_scan_kernel(BatchArgs a) {
             }
         }
 
-        // ---- K-th smallest upper bound per query -> atomicMin into tau[q] ----
-        //  K <= 16: the four lane groups' lists are merged in registers (exact top 16 of the
-        //    kept bounds), replica waves exchange theirs through LDS and the group's first
+        // ---- the unit's K smallest kept bounds join each query's list ----
+        //  K <= 16 (M = 4): the four lane groups' lists are merged in registers (exact top 16 of
+        //    the kept bounds), replica waves exchange theirs through LDS and the group's first
         //    wave merges them the same way.
-        //  K > 16: all R x 64 lists go through a register bitonic list.
+        //  K > 16 (M = 8, or 16 past K = 64): the R waves' lists meet in LDS and every wave selects
+        //    for a quarter of the queries.  (One wave sorting 64-bit keys for all 16 queries,
+        //    with M = 16 throughout, left the other three waiting: 227 us against 55 at K = 33,
+        //    1237 queries of D = 100, 440 against 128 at K = 100, 5000 queries of D = 96.)
         // Either way the K-th entry is an upper bound of the K-th smallest distance bound.
         __syncthreads();  // every wave is done with the code buffers
-        if (a.K <= kUbList) {
+        if constexpr (M <= 4) {
             if (active) {
                 merge16_groups(ubl);
                 if (R > 1 && g == 0) {
@@ -1280,33 +1286,59 @@ __global__ __launch_bounds__(256) void ub_scan_kernel(BatchArgs a) {
                     atomicMin(&a.ub_best[q], __float_as_uint(uk));
             }
         } else {
+            // each wave lists every fourth query: the K-th smallest of the unit's 4 M R kept
+            // bounds by bisection on their bits (ballot counts), then the K smallest
+            // compacted -- in no order, which the query's list does not need
             if (active) {
-                float* s_ub = s_ubl[wid];
 #pragma unroll
-                for (int i = 0; i < kUbList; ++i) s_ub[j * 64 + g * kUbList + i] = ubl[i];
+                for (int i = 0; i < M; ++i) s_ubl[wid][j * kUblRow + g * M + i] = ubl[i];
             }
             __syncthreads();
-            if (active && rr == 0) {
-                for (int jj = 0; jj < nq; ++jj) {
-                    WaveList<64> L;
-                    L.init();
-                    for (int r2 = 0; r2 < R; ++r2)
-                        L.insert(key_of((double)s_ubl[wid + r2][jj * 64 + lane]), lane);
-                    // lane i holds the unit's i-th smallest kept bound: the first K join the
-                    // query's list
-                    const int qq = __shfl(q, jj, kWave);
-                    const int nl = ub_per_unit(a.K);
-                    int base = 0;
-                    if (lane == 0) base = atomicAdd(&a.ub_cnt[qq], nl);
-                    base = __shfl(base, 0, kWave);
-                    const float uv = L.k0 == kKeyInvalid ? INFINITY : (float)dist_of(L.k0);
-                    if (lane < nl && base + lane < a.ub_cap)
-                        a.ub_list[(size_t)qq * a.ub_cap + base + lane] =
-                            row_entry(uv, a.vec_off[cid] + vb);
-                    // K <= 64: the unit's own K-th bound, when its entries did not fit
-                    if (a.K <= 64 && lane == a.K - 1 && base + nl > a.ub_cap && uv < INFINITY)
-                        atomicMin(&a.ub_best[qq], __float_as_uint(uv));
+            const int nl = ub_per_unit(a.K);
+            const int row0 = v0 + vb;
+            for (int qi = wid; qi < cnt; qi += kWavesPerBlock) {
+                const int w0 = (qi / kWaveQ) * R, col = qi % kWaveQ;
+                constexpr int NV = kWavesPerBlock * 4 * M / kWave;  // values per lane (R = 4)
+                uint32_t v[NV];
+#pragma unroll
+                for (int i = 0; i < NV; ++i) {
+                    const int e = i * kWave + lane, r2 = e / (4 * M);
+                    v[i] = r2 < R ? __float_as_uint(s_ubl[w0 + r2][col * kUblRow + e % (4 * M)])
+                                  : 0x7f800000u;
                 }
+                // smallest x with count(v <= x) >= nl (v are non-negative floats or +inf)
+                uint32_t lo = 0u, hi = 0x7f800000u;
+                while (lo < hi) {
+                    const uint32_t mid = lo + ((hi - lo) >> 1);
+                    int c = 0;
+#pragma unroll
+                    for (int i = 0; i < NV; ++i) c += __popcll(__ballot(v[i] <= mid));
+                    if (c >= nl) hi = mid;
+                    else lo = mid + 1u;
+                    if (c == nl) break;  // exactly the nl smallest lie at or below hi
+                }
+                const int qq = a.pair_qid[start + qi];
+                int base = 0;
+                if (lane == 0) base = atomicAdd(&a.ub_cnt[qq], nl);
+                base = __builtin_amdgcn_readfirstlane(base);
+                uint2* dst = a.ub_list + (size_t)qq * a.ub_cap;
+                // values below hi first, then those equal to it, nl in all (+inf fills the rest)
+                int at = base;
+                const int end = min(base + nl, a.ub_cap);
+#pragma unroll
+                for (int eq = 0; eq < 2; ++eq) {
+#pragma unroll
+                    for (int i = 0; i < NV; ++i) {
+                        const bool take = eq ? v[i] == hi : v[i] < hi;
+                        const uint64_t m = __ballot(take);
+                        const int sl = at + mask_rank(m);
+                        if (take && sl < end) dst[sl] = row_entry(__uint_as_float(v[i]), row0);
+                        at += __popcll(m);
+                    }
+                }
+                // the unit's own K-th bound, when its entries did not fit
+                if (lane == 0 && base + nl > a.ub_cap && hi < 0x7f800000u)
+                    atomicMin(&a.ub_best[qq], hi);
             }
         }
         if (tid == 0) s_unit[(it + 1) & 1] = nblk > 0 ? nxt : atomicAdd(ctr, 1);
@@ -1315,39 +1347,55 @@ __global__ __launch_bounds__(256) void ub_scan_kernel(BatchArgs a) {
 }
 
 template __global__ void ub_scan_kernel<1, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<2, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<3, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<4, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<1, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<1, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<2, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<2, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<2, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<3, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<3, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<3, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<4, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<4, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<4, 16>(BatchArgs);
 template __global__ void ub_scan_kernel<5, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<6, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<7, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<8, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<9, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<10, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<11, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<12, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<13, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<14, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<15, 4>(BatchArgs);
-template __global__ void ub_scan_kernel<16, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<5, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<5, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<6, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<6, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<6, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<7, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<7, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<7, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<8, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<8, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<8, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<9, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<9, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<9, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<10, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<10, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<10, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<11, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<11, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<11, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<12, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<12, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<12, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<13, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<13, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<13, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<14, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<14, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<14, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<15, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<15, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<15, 16>(BatchArgs);
+template __global__ void ub_scan_kernel<16, 4>(BatchArgs);
+template __global__ void ub_scan_kernel<16, 8>(BatchArgs);
 template __global__ void ub_scan_kernel<16, 16>(BatchArgs);
 
-// Seeding threshold, one wave per query.  Its list holds each seeding unit's min(K, 64) smallest
+// Seeding threshold, one wave per query.  Its list holds each seeding unit's K smallest
 // bounds u with their rows (all distinct rows); the K smallest (u, position) entries are the
 // query's seeds:
 //   tau_ub = the K-th smallest u (K rows have distance <= it), also over ub_best (a unit's own
@@ -1374,22 +1422,71 @@ __global__ __launch_bounds__(256) void ub_kth_kernel(BatchArgs a) {
     double tau = ubest < INFINITY ? (double)ubest * ubest / a.rot_sq_min * (1.0 + 1e-6) : INFINITY;
     if (n >= K) {
         const uint2* lst = a.ub_list + (size_t)q * a.ub_cap;
-        WaveList<KP> L;
-        L.init();
-        for (int i0 = 0; i0 < n; i0 += kWave) {
-            const int i = i0 + lane;
-            const uint2 e = i < n ? lst[i] : make_uint2(0u, 0u);
-            L.insert(i < n ? key_of((double)__uint_as_float(e.x)) : kKeyInvalid,
-                     i < n ? (int32_t)e.y : kIdInvalid);
+        double u = INFINITY;  // the K-th smallest listed bound
+        constexpr int NV = 8;
+        if (n <= NV * kWave) {
+            // the whole list in registers: K-th smallest by bisection on the bits (ballot
+            // counts), the K seeds compacted in no order
+            uint32_t v[NV];
+            int32_t ps[NV];
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int e = i * kWave + lane;
+                const uint2 en = e < n ? lst[e] : make_uint2(0xffffffffu, 0xffffffffu);
+                v[i] = en.x;
+                ps[i] = (int32_t)en.y;
+            }
+            uint32_t lo = 0u, hi = 0x7f800000u;  // count(v <= hi) >= K: the n entries are <= +inf
+            while (lo < hi) {
+                const uint32_t mid = lo + ((hi - lo) >> 1);
+                int c = 0;
+#pragma unroll
+                for (int i = 0; i < NV; ++i) c += __popcll(__ballot(v[i] <= mid));
+                if (c >= K) hi = mid;
+                else lo = mid + 1u;
+                if (c == K) break;
+            }
+            uint32_t mx = 0u;
+            int at = 0;
+#pragma unroll
+            for (int eq = 0; eq < 2; ++eq) {
+#pragma unroll
+                for (int i = 0; i < NV; ++i) {
+                    const bool take = eq ? v[i] == hi : v[i] < hi;
+                    const uint64_t m = __ballot(take);
+                    const int sl = at + mask_rank(m);
+                    if (take && sl < K) {
+                        s_pos[wid][sl] = ps[i];
+                        mx = max(mx, v[i]);
+                    }
+                    at += __popcll(m);
+                }
+            }
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, kWave));
+            if (mx < 0x7f800000u) u = (double)__uint_as_float(mx);
+        } else {
+            WaveList<KP> L;
+            L.init();
+            for (int i0 = 0; i0 < n; i0 += kWave) {
+                const int i = i0 + lane;
+                const uint2 e = i < n ? lst[i] : make_uint2(0u, 0u);
+                L.insert(i < n ? key_of((double)__uint_as_float(e.x)) : kKeyInvalid,
+                         i < n ? (int32_t)e.y : kIdInvalid);
+            }
+            uint64_t kk;
+            int32_t ki;
+            L.at(K - 1, kk, ki);
+            if (kk != kKeyInvalid) u = dist_of(kk);
+            if (lane < K) s_pos[wid][lane] = L.i0;
+            if constexpr (KP > 64)
+                if (lane + kWave < K) s_pos[wid][kWave + lane] = L.i1;
         }
-        uint64_t kk;
-        int32_t ki;
-        L.at(K - 1, kk, ki);
-        const double u = kk != kKeyInvalid ? dist_of(kk) : INFINITY;
+        wave_sync();
         if (u < (double)INFINITY) tau = fmin(tau, u * u / a.rot_sq_min * (1.0 + 1e-6));
         // exact seeding: every one of the K smallest entries is finite and has its row
-        bool ok = lane >= K || (L.k0 != kKeyInvalid && L.i0 >= 0);
-        if constexpr (KP > 64) ok = ok && (lane + kWave >= K || (L.k1 != kKeyInvalid && L.i1 >= 0));
+        bool ok = lane >= K || s_pos[wid][lane] >= 0;
+        if constexpr (KP > 64) ok = ok && (lane + kWave >= K || s_pos[wid][kWave + lane] >= 0);
         if (u < (double)INFINITY && __ballot(!ok) == 0ull && a.fine_mode) {
             // fine codes: the K seeds' upper bounds from HBM; no row crosses PCIe here and
             // no seed is listed (the lower-bound pass lists every row with d64 <= tau)
@@ -1397,24 +1494,18 @@ __global__ __launch_bounds__(256) void ub_kth_kernel(BatchArgs a) {
             wave_sync();
             const double qe = sqrt(a.qep[q]) * (1.0 + 1e-12);
             double mx = 0.0;
-            for_chunks<KP>([&](auto cc) __attribute__((always_inline)) {
-                constexpr int h = decltype(cc)::value;
-                uint64_t hk;
-                int32_t pos;
-                list_chunk<h>(L, hk, pos);
+#pragma unroll
+            for (int h = 0; h < KP / kWave; ++h) {
                 if (h * kWave + lane < K) {
                     double lb, ub;
-                    fine_row_bounds(a, s_q64[wid], qe, pos, lb, ub);
+                    fine_row_bounds(a, s_q64[wid], qe, s_pos[wid][h * kWave + lane], lb, ub);
                     mx = fmax(mx, ub);
                 }
-            });
+            }
 #pragma unroll
             for (int o = 1; o < kWave; o <<= 1) mx = fmax(mx, shfl_f64(mx, lane ^ o));
             tau = fmin(tau, mx);
         } else if (u < (double)INFINITY && __ballot(!ok) == 0ull) {
-            if (lane < K) s_pos[wid][lane] = L.i0;
-            if constexpr (KP > 64)
-                if (lane + kWave < K) s_pos[wid][kWave + lane] = L.i1;
             for (int d = lane; d < a.D; d += kWave) s_q64[wid][d] = (double)a.xq[(size_t)q * a.D + d];
             wave_sync();
             double dv[KP / kWave];

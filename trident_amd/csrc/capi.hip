@@ -224,7 +224,7 @@ Workspace carve(const TridentIndexView* ix, void* base, int64_t B, int64_t nprob
     w.lbk = c.take<int2>(B * nprobe + 32);  // + 32: the scan reads whole 32-row groups
     w.cbound = c.take<double>(kCbStride * (int64_t)ix->nlist);
     w.qep = c.take<double>(B);
-    w.ub_cap = ub_cap_of(std::min<int64_t>(K, 64));
+    w.ub_cap = ub_cap_of(K);
     w.ub_list = c.take<uint2>(B * w.ub_cap);
     w.ub_cnt = c.take<int32_t>(B);
     w.ub_best = c.take<uint32_t>(B);
@@ -401,8 +401,7 @@ int dispatch_scan(const ScanArgs& a, int kind, hipStream_t st) {
 }
 
 // Route of a mode-2 search.  The batched route needs the per-vector scalars, K <= 128 (a
-// seeding unit lists at most 64 bounds per query; the threshold is the K-th over all of a
-// query's units and the merge keeps 128), D_pad <= 1024 (query weights
+// seeding unit lists K <= 128 bounds per query and the merge keeps 128), D_pad <= 1024 (query weights
 // held in registers: 8 VGPRs per 64 dims) and N < 2^27 (a queued survivor packs its index within the cluster
 // into 28 bits); AUTO takes it when clusters are shared by >= 8 queries on average, where
 // the contraction is dense enough for the matrix cores.
@@ -544,7 +543,7 @@ int launch_cm(const BatchArgs& b, hipStream_t st) {
     }
 }
 
-// Seeding pass: ub_scan_kernel<KS, M> (M = per-lane list length, 4 when K <= 16);
+// Seeding pass: ub_scan_kernel<KS, M> (M = per-lane list length: 4 while K <= 16, 8 while K <= 64);
 // lower-bound pass: lb_scan_kernel<KS> (D_pad <= 256) or lb_scan_wide_kernel<KS>.
 template <bool UB, int KS, int M>
 const void* batch_kernel_ptr() {
@@ -584,6 +583,8 @@ int launch_batch_ks(const BatchArgs& b, hipStream_t st) {
     if constexpr (UB) {
         if (b.K <= 16)
             ub_scan_kernel<KS, 4><<<persistent_grid<true, KS, 4>(), kBlock, 0, st>>>(b);
+        else if (b.K <= 64)
+            ub_scan_kernel<KS, 8><<<persistent_grid<true, KS, 8>(), kBlock, 0, st>>>(b);
         else
             ub_scan_kernel<KS, 16><<<persistent_grid<true, KS, 16>(), kBlock, 0, st>>>(b);
         return check_launch("ub_scan_kernel");

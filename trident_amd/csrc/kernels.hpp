@@ -473,13 +473,16 @@ __global__ void cm_seed_kernel(BatchArgs a, int B);
 __global__ void fine_bounds_kernel(BatchArgs a, const int32_t* __restrict__ qids,
                                   const int64_t* __restrict__ spos, int n, double* lb, double* ub);
 
-// Bounds a seeding unit lists per query: its K smallest, at most 64.
-__host__ __device__ constexpr int ub_per_unit(int K) { return K < 64 ? K : 64; }
+// Bounds a seeding unit lists per query: its K smallest (K <= 128).
+__host__ __device__ constexpr int ub_per_unit(int K) { return K < 128 ? K : 128; }
 
 // Seeding-list slots per query: at most 3 seeding probes (trident_p_init_rule) x kMaxSplit
-// slices, ub_per_unit(K) bounds each; a unit whose entries no longer fit offers its K-th bound
-// to ub_best instead.
-inline int64_t ub_cap_of(int64_t K) { return 3 * kMaxSplit * (int64_t)ub_per_unit((int)K); }
+// slices, K bounds each, up to K = 64; past it the seeding pass scans at most two slices of a
+// cluster (seed_slice_count), so the same 1536 slots hold at least 12 units' K bounds.  A unit whose entries no
+// longer fit offers its K-th bound to ub_best instead.
+inline int64_t ub_cap_of(int64_t K) {
+    return 3 * kMaxSplit * (K < 64 ? K : 64);
+}
 
 // Seeding bounds carry their row: the bound is rounded up to a multiple of 2^16 in its bit
 // pattern (at most 2^-7 of its value) and the low 16 bits hold the row's index in the unit's

@@ -112,6 +112,7 @@ struct Workspace {
     int32_t* pair_qids;
     float* pair_dqcs;
     int32_t* pair_rank;              // group_pairs past the LDS histogram: arrival ranks
+    int64_t cap;                     // candidate-list slots per query
     uint64_t* cand_key;
     int32_t* cand_id;
     int32_t* cand_cnt;
@@ -177,15 +178,27 @@ inline int64_t plane_bytes(int D_pad) { return 64 * (int64_t)((D_pad + 63) / 64)
 // K = 100: ~1 % of candidates pass, ~2,300 per query with a long tail), so those lists are 8x
 // deeper.  An index with a fine level keeps its base in host memory, where an overflow costs
 // most, so its lists are twice as deep again.
-inline int64_t cand_cap(int64_t nprobe, int64_t K, int64_t D_pad, bool fine) {
+inline int64_t cand_cap_min(int64_t nprobe, int64_t K, int64_t D_pad, bool fine) {
     return nprobe * std::max<int64_t>(K, 64) * (K > 64 && D_pad > 256 ? 8 : 1) * (fine ? 2 : 1);
 }
 
-Workspace carve(const TridentIndexView* ix, void* base, int64_t B, int64_t nprobe, int64_t K) {
+// A few probes of long clusters outrun those lists (nprobe 4 of 10,000-row clusters: 256 slots for
+// 40,000 rows, of which the 8-bit bounds leave ~1 %; 2 of 1,250 rows: 128 slots, and K = 100 keeps
+// every eighth row), so a list also holds twice the rows a query visits on average, up to 4096
+// slots (49 KB a query).  `deep` false keeps the smaller lists: a workspace sized without the floor
+// still serves its searches, with those.
+inline int64_t cand_cap(const TridentIndexView* ix, int64_t nprobe, int64_t K, bool deep) {
+    const int64_t least = cand_cap_min(nprobe, K, ix->D_pad, ix->fine_codes && ix->fine_qp);
+    const int64_t rows = (int64_t)((double)nprobe * ix->N / ix->nlist);
+    return deep ? std::max<int64_t>(least, std::min<int64_t>(2 * rows, 4096)) : least;
+}
+
+Workspace carve(const TridentIndexView* ix, void* base, int64_t B, int64_t nprobe, int64_t K,
+                bool deep = true) {
     Carver c{static_cast<char*>(base)};
     Workspace w;
     const int64_t KP = K <= 64 ? 64 : K <= 128 ? 128 : 256;
-    const int64_t cap = cand_cap(nprobe, K, ix->D_pad, ix->fine_codes && ix->fine_qp);
+    const int64_t cap = w.cap = cand_cap(ix, nprobe, K, deep);
     w.xq64 = c.take<double>(B * ix->D);
     w.xrot64 = c.take<double>(B * ix->D_pad);
     w.xrot32 = c.take<float>(B * ix->D_pad);
@@ -924,7 +937,7 @@ int trident_coarse_probe(const TridentIndexView* ix, const float* xq, int32_t B,
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "bad probe arguments B=%d nprobe=%d ld=%d", B,
                     nprobe, probe_ld);
     if (B == 0) return TRIDENT_OK;
-    Workspace w = carve(ix, workspace, B, nprobe, 1);
+    Workspace w = carve(ix, workspace, B, nprobe, 1, false);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);
@@ -1007,6 +1020,7 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
     if (!xq) return fail(TRIDENT_ERR_INVALID_ARGUMENT, "xq is NULL");
 
     Workspace w = carve(ix, workspace, B, nprobe, K_list);
+    if (workspace_bytes < w.bytes) w = carve(ix, workspace, B, nprobe, K_list, false);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);
@@ -1069,7 +1083,7 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
     if ((rc = mark(TRIDENT_EV_GROUPED))) return rc;
 
     const int KP = list_kp(K_list);
-    const int64_t cap = cand_cap(nprobe, K_list, ix->D_pad, ix->fine_codes && ix->fine_qp);
+    const int64_t cap = w.cap;
     if (out->stats) {
         if ((rc = fill(reinterpret_cast<int32_t*>(out->stats), 0, 8, st))) return rc;
         if ((rc = fill(reinterpret_cast<int32_t*>(w.stat_slots), 0, 2 * 4 * kStatSlots, st))) return rc;
@@ -1528,7 +1542,7 @@ int trident_search_noalloc(const TridentIndexView* ix, const TridentSearchParams
     // the size check comes before any HIP call, so an oversized request fails without touching
     // the device
     const size_t need =
-        carve(ix, nullptr, sp->B, sp->nprobe, merged_list_len(sp->mode, sp->K, sp->rerank_m)).bytes;
+        carve(ix, nullptr, sp->B, sp->nprobe, merged_list_len(sp->mode, sp->K, sp->rerank_m), false).bytes;
     if (need > (size_t)TRIDENT_NOALLOC_SCRATCH_BYTES)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL,
                     "trident_search_noalloc: B=%d nprobe=%d K=%d needs %zu bytes of scratch, more "
@@ -1559,7 +1573,7 @@ int trident_sq8_bounds(const TridentIndexView* ix, const float* xq, int32_t B,
     if ((rc = validate_cascade_index(ix))) return rc;
     if (B < 1 || n < 0 || !xq || !qids || !cids || !spos || !lb || !ub)
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "bad sq8_bounds arguments");
-    Workspace w = carve(ix, workspace, B, 1, 1);
+    Workspace w = carve(ix, workspace, B, 1, 1, false);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);
@@ -1604,7 +1618,7 @@ int trident_fine_bounds(const TridentIndexView* ix, const float* xq, int32_t B,
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "fine_bounds needs fine_codes and fine_qp");
     if (B < 1 || n < 0 || !xq || !qids || !spos || !lb || !ub)
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "bad fine_bounds arguments");
-    Workspace w = carve(ix, workspace, B, 1, 1);
+    Workspace w = carve(ix, workspace, B, 1, 1, false);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);

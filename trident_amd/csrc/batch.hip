@@ -76,69 +76,92 @@ __device__ __forceinline__ int splits_of(int n, int sv) {
 // probes; the threshold stays exact (the K-th exact distance of rows that exist), only looser.
 __device__ __forceinline__ int seed_slices(int S, int seed_sl) { return min(S, seed_sl); }
 
-// Entry e < nlist: the seeding units of cluster e (its pass-1 queries, or all of them when
-// seed_all, <= 16 per unit; the first seed_slices(S, seed_sl) slices); entry nlist + c: the
-// lower-bound units of cluster c (all its queries, <= uqB per unit, every slice).
-__device__ __forceinline__ int units_of_entry(const int32_t* seg, const int32_t* vec_off,
-                                              int nlist, int uqB, int seed_all, int seed_sl, int sv,
-                                              int svb, int e) {
-    const int p = e >= nlist ? 1 : 0, c = e - p * nlist;
-    const int q = (p || seed_all ? seg[c + 1] : seg[nlist + 1 + c]) - seg[c];
-    const int uq = p ? uqB : kUnitQ0;
-    const int S = splits_of(vec_off[c + 1] - vec_off[c], p ? svb : sv);
-    return q > 0 ? ((q + uq - 1) / uq) * (p ? S : seed_slices(S, seed_sl)) : 0;
-}
+// Work units of a cluster: u0 seeding units (its pass-1 queries, or all of them when seed_all, <=
+// 16 per unit; the first seed_slices(S, seed_sl) slices), u1 lower-bound units (all its queries, <=
+// uqB per unit, every slice).
+__device__ __forceinline__ int units_of(int q, int uq, int S) { return q > 0 ? (q + uq - 1) / uq * S : 0; }
 
-__device__ __forceinline__ int groups_of_cluster(const int32_t* seg, int c) {
-    return (seg[c + 1] - seg[c] + kGroupQ - 1) / kGroupQ;
-}
-
-// Exclusive scans of the unit counts of the 2 * nlist (pass, cluster) entries and of the
-// weight-group counts of the nlist cluster segments, in two launches of ceil(2 nlist / kBlock)
-// <= kBlock blocks, one entry (and one cluster) per thread: in-block offsets plus block totals
-// (blk_tot[b] units, blk_tot[kBlock + b] groups), then the carries of the blocks before.
-__global__ __launch_bounds__(256) void unit_scan_local_kernel(const int32_t* seg,
-                                                              const int32_t* vec_off, int nlist,
-                                                              int uqB, int seed_all, int seed_sl,
-                                                              int sv, int svb, int32_t* unit_off,
-                                                              int32_t* grp_off, int32_t* blk_tot) {
-    __shared__ uint32_t s_wtot[kWavesPerBlock];
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t nu =
-        i < 2 * nlist ? (uint32_t)units_of_entry(seg, vec_off, nlist, uqB, seed_all, seed_sl, sv, svb, i)
-                      : 0u;
-    const uint32_t ng = i < nlist ? (uint32_t)groups_of_cluster(seg, i) : 0u;
-    uint32_t tu = 0, tg = 0;
-    const uint32_t ru = block_exclusive_scan(nu, s_wtot, &tu);
-    const uint32_t rg = block_exclusive_scan(ng, s_wtot, &tg);
-    if (i < 2 * nlist) unit_off[i] = (int32_t)ru;
-    if (i < nlist) grp_off[i] = (int32_t)rg;
-    if (threadIdx.x == 0) {
-        blk_tot[blockIdx.x] = (int32_t)tu;
-        blk_tot[kBlock + blockIdx.x] = (int32_t)tg;
+// Offsets of the cluster-major layout from the counts, one block: exclusive scans over the
+// clusters of the pairs, the units of both kinds and the weight groups, 4 clusters a thread and
+// chunk of 4096.  One launch where two scans of two launches each ran (18.5 us; this takes 8 at
+// nlist 1024, 13 at 4096).
+__global__ __launch_bounds__(1024) void group_scan_kernel(GroupArgs a) {
+    constexpr int V = 4, NW = 16;
+    __shared__ uint32_t s_tot[4][NW];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nlist = a.nlist;
+    uint32_t carry[4] = {0u, 0u, 0u, 0u};  // pairs, seeding units, lower-bound units, groups
+    for (int c0 = 0; c0 < nlist; c0 += V * 1024) {
+        int n1[V];
+        uint32_t v[V][4], sum[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const int c = c0 + V * tid + i;
+            const bool in = c < nlist;
+            n1[i] = in ? a.counts[c] : 0;
+            const int n = n1[i] + (in ? a.counts[nlist + 1 + c] : 0);
+            const int len = in ? a.vec_off[c + 1] - a.vec_off[c] : 0;
+            v[i][0] = (uint32_t)n;
+            v[i][1] = (uint32_t)units_of(a.seed_all ? n : n1[i], kUnitQ0, seed_slices(splits_of(len, a.sv), a.seed_sl));
+            v[i][2] = (uint32_t)units_of(n, a.uqB, splits_of(len, a.svb));
+            v[i][3] = (uint32_t)((n + kGroupQ - 1) / kGroupQ);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sum[k] += v[i][k];
+        }
+        uint32_t inc[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) inc[k] = sum[k];
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t t = (uint32_t)__shfl_up((int)inc[k], o, kWave);
+                if (lane >= o) inc[k] += t;
+            }
+        }
+        __syncthreads();  // the previous chunk's totals are read
+        if (lane == kWave - 1) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s_tot[k][wid] = inc[k];
+        }
+        __syncthreads();
+        uint32_t run[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            uint32_t before = 0u, all = 0u;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const uint32_t t = s_tot[k][w];
+                before += w < wid ? t : 0u;
+                all += t;
+            }
+            run[k] = carry[k] + before + inc[k] - sum[k];
+            carry[k] += all;
+        }
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const int c = c0 + V * tid + i;
+            if (c < nlist) {
+                a.seg[c] = (int32_t)run[0];
+                a.seg[nlist + 1 + c] = (int32_t)run[0] + n1[i];
+                a.unit_off[c] = (int32_t)run[1];
+                a.unit_off[nlist + c] = (int32_t)run[2];  // the seeding units come on top below
+                a.grp_off[c] = (int32_t)run[3];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) run[k] += v[i][k];
+        }
     }
-}
-
-__global__ __launch_bounds__(256) void unit_scan_carry_kernel(int nlist, const int32_t* blk_tot,
-                                                              int nblk, int32_t* unit_off,
-                                                              int32_t* grp_off) {
-    __shared__ uint32_t s_wtot[kWavesPerBlock];
-    __shared__ uint32_t s_carry[2];
-    const int tid = threadIdx.x, i = blockIdx.x * kBlock + tid;
-    uint32_t tu = 0, tg = 0;
-    const uint32_t cu = block_exclusive_scan(tid < nblk ? (uint32_t)blk_tot[tid] : 0u, s_wtot, &tu);
-    const uint32_t cg =
-        block_exclusive_scan(tid < nblk ? (uint32_t)blk_tot[kBlock + tid] : 0u, s_wtot, &tg);
-    if (tid == (int)blockIdx.x) {
-        s_carry[0] = cu;
-        s_carry[1] = cg;
+    for (int c0 = 0; c0 < nlist; c0 += V * 1024) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const int c = c0 + V * tid + i;
+            if (c < nlist) a.unit_off[nlist + c] += (int32_t)carry[1];  // this thread wrote it
+        }
     }
-    __syncthreads();
-    if (i < 2 * nlist) unit_off[i] += (int32_t)s_carry[0];
-    if (i < nlist) grp_off[i] += (int32_t)s_carry[1];
-    if (blockIdx.x == 0 && tid == 0) {
-        unit_off[2 * nlist] = (int32_t)tu;
-        grp_off[nlist] = (int32_t)tg;
+    if (tid == 0) {
+        a.seg[nlist] = a.seg[2 * nlist + 1] = (int32_t)carry[0];
+        a.unit_off[2 * nlist] = (int32_t)(carry[1] + carry[2]);
+        a.grp_off[nlist] = (int32_t)carry[3];
     }
 }
 
@@ -153,42 +176,69 @@ __device__ __forceinline__ int seg_search(const int32_t* off, int n, int x) {
     return lo;
 }
 
-// One thread per weight group ({first pair, pair count}: kGroupQ consecutive pairs of a cluster's
-// segment), then one thread per unit: its segment by binary search over unit_off, then its
-// vector slice and query block.  Slices start on 64-vector blocks and are never empty (n > 64 S
-// (S - 1) whenever S = ceil(n / sv) > 1, for sv >= 512).
-__global__ __launch_bounds__(256) void unit_fill_kernel(const int32_t* seg, const int32_t* vec_off,
-                                                        int nlist, int uqB, int seed_all, int sv, int svb,
-                                                        const int32_t* unit_off,
-                                                        int4* units, int max_units,
-                                                        const int32_t* grp_off, int2* groups,
-                                                        int max_groups) {
-    const int ngrp = min(grp_off[nlist], max_groups);
-    for (int gi = blockIdx.x * blockDim.x + threadIdx.x; gi < ngrp;
-         gi += gridDim.x * blockDim.x) {
-        const int c = seg_search(grp_off, nlist, gi);
-        const int k = gi - grp_off[c];
-        groups[gi] = make_int2(seg[c] + k * kGroupQ, min(kGroupQ, seg[c + 1] - seg[c] - k * kGroupQ));
+// What follows from the offsets, in one launch, block ranges by role:
+//   nb_scatter: one thread per pair, placed at its bin's offset plus its rank;
+//   nb_fill:    one thread per weight group ({first pair, pair count}: kGroupQ consecutive pairs of a
+//               cluster's segment), then one per unit: its cluster by binary search over unit_off,
+//               then its vector slice and query block.  Slices start on 64-vector blocks and are
+//               never empty (n > 64 S (S - 1) whenever S = ceil(n / sv) > 1, for sv >= 512);
+//   the rest:   one wave per query, the sum of qerr^2 (the rotation error of q_rot, squared).
+__global__ __launch_bounds__(256) void group_fill_kernel(GroupArgs a) {
+    const int nlist = a.nlist;
+    int blk = (int)blockIdx.x;
+    if (blk < a.nb_scatter) {
+        const int total = a.B * a.nprobe;
+        for (int idx = blk * kBlock + (int)threadIdx.x; idx < total; idx += a.nb_scatter * kBlock) {
+            const int q = idx / a.nprobe, p = idx - q * a.nprobe;
+            const int cid = a.probe_cids[idx];
+            if ((unsigned)cid >= (unsigned)nlist) continue;
+            const int slot = a.seg[(p < a.p_init ? 0 : (nlist + 1)) + cid] + a.rank[idx];
+            a.pair_cid[slot] = cid;
+            a.pair_qid[slot] = q;
+            if (a.pair_dqc) a.pair_dqc[slot] = a.probe_dqcs[idx];
+        }
+        return;
     }
-    const int E = 2 * nlist;
-    const int total = min(unit_off[E], max_units);
-    for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < total; u += gridDim.x * blockDim.x) {
-        const int e = seg_search(unit_off, E, u);
-        const int p = e >= nlist ? 1 : 0, c = e - p * nlist;
-        const int n = vec_off[c + 1] - vec_off[c];
-        const int S = splits_of(n, p ? svb : sv);
-        const int local = u - unit_off[e];
-        const int q = (p || seed_all ? seg[c + 1] : seg[nlist + 1 + c]) - seg[c];
-        const int uq = p ? uqB : kUnitQ0;
-        // slice-major: a slice's query blocks are consecutive units, so the workgroups that
-        // take them together read the slice's codes while they are in the XCD's L2
-        const int QB = (q + uq - 1) / uq;
-        const int sp = local / QB, qb = local - sp * QB;
-        const int cnt = min(uq, q - qb * uq);
-        const int len = ((n + S - 1) / S + kBlkV - 1) & ~(kBlkV - 1);
-        const int vb = sp * len, ve = min(n, vb + len);
-        units[u] = make_int4(c | (cnt << 20), seg[c] + qb * uq, vb, ve);
+    blk -= a.nb_scatter;
+    const int32_t* seg = a.seg;
+    if (blk < a.nb_fill) {
+        const int i0 = blk * kBlock + (int)threadIdx.x, step = a.nb_fill * kBlock;
+        const int ngrp = min(a.grp_off[nlist], a.max_groups);
+        for (int gi = i0; gi < ngrp; gi += step) {
+            const int c = seg_search(a.grp_off, nlist, gi);
+            const int k = gi - a.grp_off[c];
+            a.groups[gi] = make_int2(seg[c] + k * kGroupQ, min(kGroupQ, seg[c + 1] - seg[c] - k * kGroupQ));
+        }
+        const int E = 2 * nlist;
+        const int total = min(a.unit_off[E], a.max_units);
+        for (int u = i0; u < total; u += step) {
+            const int e = seg_search(a.unit_off, E, u);
+            const int p = e >= nlist ? 1 : 0, c = e - p * nlist;
+            const int n = a.vec_off[c + 1] - a.vec_off[c];
+            const int S = splits_of(n, p ? a.svb : a.sv);
+            const int local = u - a.unit_off[e];
+            const int q = (p || a.seed_all ? seg[c + 1] : seg[nlist + 1 + c]) - seg[c];
+            const int uq = p ? a.uqB : kUnitQ0;
+            // slice-major: a slice's query blocks are consecutive units, so the workgroups that
+            // take them together read the slice's codes while they are in the XCD's L2
+            const int QB = (q + uq - 1) / uq;
+            const int sp = local / QB, qb = local - sp * QB;
+            const int cnt = min(uq, q - qb * uq);
+            const int len = ((n + S - 1) / S + kBlkV - 1) & ~(kBlkV - 1);
+            const int vb = sp * len, ve = min(n, vb + len);
+            a.units[u] = make_int4(c | (cnt << 20), seg[c] + qb * uq, vb, ve);
+        }
+        return;
     }
+    blk -= a.nb_fill;
+    const int lane = threadIdx.x & 63, q = blk * kWavesPerBlock + (int)(threadIdx.x >> 6);
+    if (q >= a.B) return;
+    const double* qe = a.qerr + (size_t)q * a.D_pad;
+    double ep = 0.0;
+    for (int d = lane; d < a.D_pad; d += kWave) ep = fma(qe[d], qe[d], ep);
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) ep += shfl_f64(ep, lane ^ o);
+    if (lane == 0) a.qep[q] = ep;
 }
 
 __global__ void fill_u64_kernel(unsigned long long* p, unsigned long long v, int64_t n) {
@@ -403,7 +453,8 @@ __global__ void fine_bounds_kernel(BatchArgs a, const int32_t* __restrict__ qids
 // spreads over many waves); each lane walks its own row in dimension order with 16-byte loads,
 // against the query row staged in LDS (DQ >= D floats per wave: 256, or 1024 for the wide
 // batched route).  An overflowed list (count > cap) is left alone: the merge rescans that
-// query's probes through the SQ8 bounds (merge_kernel).
+// query's probes through the SQ8 bounds (merge_kernel), in a slot of the parallel rescan taken
+// here while there are any.
 template <bool HOST, int DQ>
 __global__ __launch_bounds__(256) void refine_survivors_kernel(BatchArgs a, int B) {
     __shared__ __align__(16) float s_q[kWavesPerBlock][HOST ? 1 : DQ];  // host: float64 copy below
@@ -411,6 +462,18 @@ __global__ __launch_bounds__(256) void refine_survivors_kernel(BatchArgs a, int 
     const int q = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + wid);
     if (q >= B) return;
     const int cnt = a.cand_cnt[q], ns = a.seed_cnt[q];
+    if (a.ovf_max > 0 && blockIdx.y == 0 && lane == 0) {
+        int slot = -1;
+        if (cnt > a.cap) {
+            const int s = atomicAdd(a.ovf_n, 1);
+            if (s < a.ovf_max) {
+                slot = s;
+                a.ovf_q[s] = q;
+                a.ovf_done[s] = 0;
+            }
+        }
+        a.ovf_slot[q] = slot;
+    }
     if (cnt > a.cap || ns + (int)blockIdx.y * kWave >= cnt) return;
     const double tau = a.tau[q];
     const int D = a.D;  // <= DQ (the launch picks DQ from D)
@@ -536,23 +599,15 @@ __device__ __forceinline__ double sum16_f64(double v) {
     return v;
 }
 
-// Waves [0, ncl): per-cluster bounds of the f32 slack (ncl = nlist, or 0 when the index
-// carries them), A_max = 255^2 sum delta^2 (>= A_x,
+// One wave per cluster: the bounds of the f32 slack, A_max = 255^2 sum delta^2 (>= A_x,
 // codes <= 255) and r_max = max(2 sqrt(sum eps^2), the largest stored r_x) (the first term
 // bounds r_x = |a| + |b| <= 2 |a + b| for the non-negative per-dim error terms when eps bounds
 // them; the second holds for any eps, e.g. an index built with the reference's 0.5001 delta),
-// and r_lo = the smallest stored r_x of the cluster.  Waves [nlist, nlist + B): per-query sum of qerr^2 (the rotation error of q_rot,
-// squared).
-__global__ __launch_bounds__(256) void aux_bounds_kernel(BatchArgs a, int ncl, int B,
-                                                         double* cbound, double* qep,
-                                                         int32_t* unit_ctr) {
+// and r_lo = the smallest stored r_x of the cluster.
+__global__ __launch_bounds__(256) void cluster_bounds_kernel(BatchArgs a, int ncl, double* cbound) {
     const int lane = threadIdx.x & 63;
     const int wv = blockIdx.x * kWavesPerBlock + (int)(threadIdx.x >> 6);
     const int D_pad = a.D_pad;
-    // the per-launch state of both passes starts here (one launch instead of three fills):
-    // work counters, tau = +inf (pass A takes atomicMin), empty survivor lists (pass B)
-    if (blockIdx.x == 0 && unit_ctr)
-        for (int i = threadIdx.x; i < 2 * 8 * kCtrStride; i += blockDim.x) unit_ctr[i] = 0;
     if (wv < ncl) {
         const size_t off = a.per_cluster ? (size_t)wv * D_pad : 0;
         double dd = 0.0, ee = 0.0;
@@ -584,20 +639,6 @@ __global__ __launch_bounds__(256) void aux_bounds_kernel(BatchArgs a, int ncl, i
             cbound[kCbStride * wv] = 65025.0 * dd * (1.0 + 1e-12);
             cbound[kCbStride * wv + 1] = fmax(2.0 * sqrt(ee), (double)rhi) * (1.0 + 1e-12);
             cbound[kCbStride * wv + 2] = rlo < INFINITY ? (double)rlo : 0.0;
-        }
-    } else if (wv < ncl + B) {
-        const int q = wv - ncl;
-        const double* qe = a.qerr + (size_t)q * D_pad;
-        double ep = 0.0;
-        for (int d = lane; d < D_pad; d += kWave) ep = fma(qe[d], qe[d], ep);
-        ep = wave_sum_f64(ep);
-        if (lane == 0) {
-            qep[q] = ep;
-            a.tau[q] = INFINITY;
-            a.cand_cnt[q] = 0;
-            a.ub_cnt[q] = 0;
-            a.ub_best[q] = 0x7f800000u;  // +inf
-            a.seed_cnt[q] = 0;
         }
     }
 }

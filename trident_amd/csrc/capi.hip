@@ -3,10 +3,11 @@
 //
 // Launch sequence of trident_search (reference launch_trident_v4_search,
 // src/trident_v4_kernels.cu:1172-1604):
-//   prep_queries -> coarse_dist -> select_probes           (front end, :1233-1259)
+//   prologue (rotation, operands, cleared counters) -> coarse distances -> select_probes
+//                                                          (front end, :1233-1259)
 //   p_init rule                                            (:1264-1276)
-//   fill / count / scan / scatter pairs                    (:1279-1289)
-//   pass 1: fill cand_cnt, pair_scan, merge  -> tau        (:1451-1512)
+//   count / scan / scatter pairs                           (:1279-1289)
+//   pass 1: pair_scan, merge  -> tau                       (:1451-1512)
 //   pass 2: fill cand_cnt, pair_scan(tau), merge -> top-K  (:1514-1575)
 //   mode 0 with rerank_m > 0: merges keep the top M by acc_hat, rerank -> top-K
 //                                                          (:1487-1500, :1550-1566, :1044-1170)
@@ -106,12 +107,10 @@ struct Workspace {
     float* probe_dqcs;
     int32_t* counts;
     int32_t* seg_off;
-    int32_t* cursor;
-    int32_t* blk_tot;  // [2 * kBlock] block totals of the multi-block scans
     int32_t* pair_cids;
     int32_t* pair_qids;
     float* pair_dqcs;
-    int32_t* pair_rank;              // group_pairs past the LDS histogram: arrival ranks
+    int32_t* pair_rank;              // arrival ranks of the pairs in their (pass, cluster) bins
     int64_t cap;                     // candidate-list slots per query
     uint64_t* cand_key;
     int32_t* cand_id;
@@ -138,13 +137,11 @@ struct Workspace {
     uint32_t* ub_best;               // [B]
     int32_t* seed_cnt;               // [B]
     int64_t ub_cap;
-    float* qt32;                     // band front end (Dq > 128): queries, matrix-core tile layout
-    uint32_t* qtb;                   // band front end (Dq <= 128): queries, bfloat16 split layout
-    uint32_t* cmtb;                  // band front end (Dq <= 128): centroids, bfloat16 split layout
+    uint32_t* qtb;                   // band front end: queries, bfloat16 split layout
+    uint32_t* cmtb;                  // band front end: centroids, bfloat16 split layout
     float* tmin;                     // [B, ceil(nlist / 16)] tile minima (nlist >= kTileMinNlist)
     float* qn32;                     // [B] their squared norms
     float* cm32;                     // [nlist, Dq] centroid-major zero-padded centroids
-    float* cmt32;                    // the centroids in the matrix-core tile layout
     float* cn32;                     // [nlist] their squared norms
     unsigned long long* cmax2;       // largest centroid squared norm (float64 bits)
     // parallel rescan of overflowed candidate lists (batched route): slots for up to ovf_max
@@ -153,6 +150,7 @@ struct Workspace {
     int32_t* ovf_n;                  // [1]
     int32_t* ovf_q;                  // [ovf_max]
     int32_t* ovf_slot;               // [B]
+    int32_t* ovf_done;               // [ovf_max]
     double* ovf_t;                   // [ovf_max]
     uint64_t* ovf_key;               // [ovf_max, nprobe, KP <= 128]
     int32_t* ovf_id;
@@ -199,67 +197,69 @@ Workspace carve(const TridentIndexView* ix, void* base, int64_t B, int64_t nprob
     Workspace w;
     const int64_t KP = K <= 64 ? 64 : K <= 128 ? 128 : 256;
     const int64_t cap = w.cap = cand_cap(ix, nprobe, K, deep);
+    const int64_t Dq = band_dq(ix->D), row_words = 16 * band_steps_bf16((int)Dq) * band_parts((int)Dq);
     w.xq64 = c.take<double>(B * ix->D);
     w.xrot64 = c.take<double>(B * ix->D_pad);
     w.xrot32 = c.take<float>(B * ix->D_pad);
     w.qerr = c.take<double>(B * ix->D_pad);
-    // float64 coarse distances [B, nlist], or the band path's float32 approximations in rows of
-    // band_lda(nlist) floats (never more bytes: band_lda(n) <= n + 3 floats <= 2 n for n >= 3,
-    // and the rows of smaller n get the extra room here)
-    w.cd64 = c.take<double>(B * std::max<int64_t>(ix->nlist, (band_lda(ix->nlist) + 1) / 2));
     w.probe_cids = c.take<int32_t>(B * nprobe);
     w.probe_dqcs = c.take<float>(B * nprobe);
     w.counts = c.take<int32_t>(2 * ((int64_t)ix->nlist + 1));
     w.seg_off = c.take<int32_t>(2 * ((int64_t)ix->nlist + 1));
-    w.cursor = c.take<int32_t>(2 * ((int64_t)ix->nlist + 1));
-    w.blk_tot = c.take<int32_t>(2 * kBlock);
     w.pair_cids = c.take<int32_t>(B * nprobe);
     w.pair_qids = c.take<int32_t>(B * nprobe);
     w.pair_dqcs = c.take<float>(B * nprobe);
     w.pair_rank = c.take<int32_t>(B * nprobe);
-    w.cand_key = c.take<uint64_t>(B * cap);
-    w.cand_id = c.take<int32_t>(B * cap);
     w.cand_cnt = c.take<int32_t>(B);
     w.list_key = c.take<uint64_t>(B * KP);
     w.list_id = c.take<int32_t>(B * KP);
     w.tau64 = c.take<double>(B);
     w.stat_slots = c.take<unsigned long long>((size_t)kStatSlots * 4);
     w.max_units = max_units_of(B * nprobe, ix->nlist);
-    w.units = c.take<int4>(w.max_units);
     w.unit_off = c.take<int32_t>(2 * (int64_t)ix->nlist + 1);
     w.unit_ctr = c.take<int32_t>(2 * 8 * kCtrStride);
     w.max_groups = max_groups_of(B * nprobe, ix->nlist);
-    w.groups = c.take<int2>(w.max_groups);
     w.grp_off = c.take<int32_t>((int64_t)ix->nlist + 1);
-    w.pw = c.take<int8_t>(B * nprobe * 2 * plane_bytes(ix->D_pad));
-    w.prec = c.take<PairRec>(B * nprobe);
-    w.lbr = c.take<LbRec>(B * nprobe);
-    w.lbk = c.take<int2>(B * nprobe + 32);  // + 32: the scan reads whole 32-row groups
     w.cbound = c.take<double>(kCbStride * (int64_t)ix->nlist);
     w.qep = c.take<double>(B);
-    w.ub_cap = ub_cap_of(K);
-    w.ub_list = c.take<uint2>(B * w.ub_cap);
     w.ub_cnt = c.take<int32_t>(B);
     w.ub_best = c.take<uint32_t>(B);
     w.seed_cnt = c.take<int32_t>(B);
-    const int64_t Dq = band_dq(ix->D);
-    const int64_t Dpb = Dq <= 128 ? 32 * band_steps_bf16((int)Dq) : 0;  // bfloat16 split dims
-    w.qt32 = c.take<float>(Dq > 128 ? (B + 15) / 16 * 16 * Dq : 0);
-    w.qtb = c.take<uint32_t>((B + 15) / 16 * 16 * Dpb);
-    w.cmtb = c.take<uint32_t>(((int64_t)ix->nlist + 15) / 16 * 16 * Dpb);
-    w.tmin = c.take<float>(ix->nlist >= kTileMinNlist && Dq <= 128 ? B * (((int64_t)ix->nlist + 15) / 16) : 0);
-    w.qn32 = c.take<float>(B);
-    w.cm32 = c.take<float>((int64_t)ix->nlist * Dq);
-    w.cmt32 = c.take<float>(((int64_t)ix->nlist + 15) / 16 * 16 * Dq);
-    w.cn32 = c.take<float>(ix->nlist);
-    w.cmax2 = c.take<unsigned long long>(1);
     w.ovf_max = ovf_slots_of(B);
     w.ovf_n = c.take<int32_t>(1);
     w.ovf_q = c.take<int32_t>(w.ovf_max);
     w.ovf_slot = c.take<int32_t>(B);
+    w.ovf_done = c.take<int32_t>(w.ovf_max);
     w.ovf_t = c.take<double>(w.ovf_max);
+    // The front end's own buffers and those of the scans share their bytes: the former are dead
+    // once the probes are selected, the latter first written after that.
+    const size_t shared = c.off;
+    // float64 coarse distances [B, nlist], or, on the band path (nprobe <= 128), float32
+    // approximations in rows of band_lda(nlist) floats
+    const int64_t lda = band_lda(ix->nlist);
+    w.cd64 = c.take<double>(nprobe <= 128 ? (B * lda + 1) / 2 : B * std::max<int64_t>(ix->nlist, (lda + 1) / 2));
+    w.qtb = c.take<uint32_t>((B + 15) / 16 * 16 * row_words);
+    w.cmtb = c.take<uint32_t>(((int64_t)ix->nlist + 15) / 16 * 16 * row_words);
+    w.tmin = c.take<float>(ix->nlist >= kTileMinNlist && Dq <= 128 ? B * (((int64_t)ix->nlist + 15) / 16) : 0);
+    w.qn32 = c.take<float>(B);
+    w.cm32 = c.take<float>((int64_t)ix->nlist * Dq);
+    w.cn32 = c.take<float>(ix->nlist);
+    w.cmax2 = c.take<unsigned long long>(1);
+    const size_t front_end = c.off;
+    c.off = shared;
+    w.cand_key = c.take<uint64_t>(B * cap);
+    w.cand_id = c.take<int32_t>(B * cap);
+    w.units = c.take<int4>(w.max_units);
+    w.groups = c.take<int2>(w.max_groups);
+    w.pw = c.take<int8_t>(B * nprobe * 2 * plane_bytes(ix->D_pad));
+    w.prec = c.take<PairRec>(B * nprobe);
+    w.lbr = c.take<LbRec>(B * nprobe);
+    w.lbk = c.take<int2>(B * nprobe + 32);  // + 32: the scan reads whole 32-row groups
+    w.ub_cap = ub_cap_of(K);
+    w.ub_list = c.take<uint2>(B * w.ub_cap);
     w.ovf_key = c.take<uint64_t>(w.ovf_max * nprobe * std::min<int64_t>(KP, 128));
     w.ovf_id = c.take<int32_t>(w.ovf_max * nprobe * std::min<int64_t>(KP, 128));
+    c.off = std::max(c.off, front_end);
     w.bytes = c.off;
     return w;
 }
@@ -666,48 +666,86 @@ int fill(int32_t* p, int32_t v, int64_t n, hipStream_t st) {
     return check_launch("fill_i32_kernel");
 }
 
+// The query rotation of a front end: none, on the float64 matrix cores, or as one chain per
+// column in dimension order (modes 0 / 1, whose results are defined by that chain).
+enum Rotation { kRotNone, kRotMatrix, kRotChain };
+
+// front_prologue_kernel over B queries; coarse: also the matrix-core coarse pass's operands (from
+// the centroid rows cm, [nlist, Dq]).
+int launch_prologue(const TridentIndexView* ix, const float* xq, int B, Rotation rot, bool coarse,
+                    const float* cm, const Workspace& w, const ClearArgs& clear, hipStream_t st) {
+    const int ldw = ix->nlist + ix->D_pad;
+    PrologueArgs a{};
+    a.xq = xq;
+    a.B = B;
+    a.D = ix->D;
+    a.D_pad = ix->D_pad;
+    a.Dq = band_dq(ix->D);
+    a.W = ix->W_combined;
+    a.ldw = ldw;
+    a.nlist = ix->nlist;
+    a.bvec = ix->b_combined;
+    a.xq64 = w.xq64;
+    a.xrot64 = w.xrot64;
+    a.xrot32 = w.xrot32;
+    a.qerr = w.qerr;
+    a.NS = coarse ? band_steps_bf16(a.Dq) : 0;
+    a.NP = band_parts(a.Dq);
+    a.qtb = reinterpret_cast<uint16_t*>(w.qtb);
+    a.qn32 = w.qn32;
+    a.cm32 = cm;
+    a.cmtb = w.cmtb;
+    a.clear = clear;
+    // 64 columns a block, or 16 where that leaves the chip idle (a quarter of the products a wave)
+    const int64_t qt = (B + 15) / 16;
+    const bool wide = qt * ((ix->D_pad + 63) / 64) >= 256;
+    a.nb_rot = rot == kRotMatrix ? (int)(qt * (wide ? (ix->D_pad + 63) / 64 : (ix->D_pad + 15) / 16)) : 0;
+    a.nb_pad = (B + kWavesPerBlock - 1) / kWavesPerBlock;
+    const int64_t npair = ((int64_t)ix->nlist + 15) / 16 * 16 * 16 * a.NS;
+    a.nb_cent = (int)std::min<int64_t>((npair + kBlock - 1) / kBlock, 2048);
+    int64_t words = clear.tau ? B : 0;
+    for (int f = 0; f < kClears; ++f) words = std::max(words, clear.n[f]);
+    a.nb_clear = (int)std::min<int64_t>((words + kBlock - 1) / kBlock, 64);
+    const unsigned grid = (unsigned)(a.nb_rot + a.nb_pad + a.nb_cent + a.nb_clear);
+    if (wide) front_prologue_kernel<4><<<grid, kBlock, 0, st>>>(a);
+    else front_prologue_kernel<1><<<grid, kBlock, 0, st>>>(a);
+    int rc = check_launch("front_prologue_kernel");
+    if (rc || rot != kRotChain) return rc;
+    prep_queries_kernel<<<dim3((ix->D_pad + 127) / 128, (B + 4 * kPrepQB - 1) / (4 * kPrepQB)),
+                          dim3(64, 4), 0, st>>>(xq, B, ix->D, ix->D_pad, ix->W_combined, ldw, ix->nlist,
+                                                ix->b_combined, w.xrot64, w.xrot32, w.qerr);
+    return check_launch("prep_queries_kernel");
+}
+
 // Writes the probes to w.probe_cids / w.probe_dqcs (row stride nprobe) and, when non-null,
 // mirrors them into the caller's probe_cids / probe_dqcs (row stride ld).
-int run_front_end(const TridentIndexView* ix, const float* xq, int B, int nprobe, bool rotate,
-                  const Workspace& w, int32_t* probe_cids, float* probe_dqcs, int ld,
-                  hipStream_t st) {
+int run_front_end(const TridentIndexView* ix, const float* xq, int B, int nprobe, Rotation rot,
+                  const Workspace& w, const ClearArgs& clear, int32_t* probe_cids, float* probe_dqcs,
+                  int ld, hipStream_t st) {
     const int ldw = ix->nlist + ix->D_pad;
-    const int cols = std::max(ix->D, rotate ? ix->D_pad : 0);
-    prep_queries_kernel<<<dim3((cols + 127) / 128, (B + 4 * kPrepQB - 1) / (4 * kPrepQB)),
-                          dim3(64, 4), 0, st>>>(
-        xq, B, ix->D, ix->D_pad, ix->W_combined, ldw, ix->nlist, ix->b_combined, w.xq64,
-        w.xrot64, w.xrot32, w.qerr, rotate ? 1 : 0);
-    int rc = check_launch("prep_queries_kernel");
-    if (rc) return rc;
-    if (nprobe <= 128) {  // band front end
-        const int Dq = band_dq(ix->D);
-        const float *cm = ix->cent_rows, *cmt = ix->cent_tiles, *cn = ix->cent_norms;
-        const unsigned long long* cmax_dev = nullptr;
-        if (!cm) {  // derive the centroid layouts into the workspace
-            fill_u64_kernel<<<1, 64, 0, st>>>(w.cmax2, 0ull, 1);
-            if ((rc = check_launch("fill_u64_kernel"))) return rc;
-            pad_centroids_kernel<<<(unsigned)((ix->nlist + 63) / 64), 256, 0, st>>>(
-                ix->W_combined, ldw, ix->nlist, ix->D, Dq, w.cm32, w.cmt32, w.cn32, w.cmax2);
-            if ((rc = check_launch("pad_centroids_kernel"))) return rc;
-            cm = w.cm32;
-            cmt = w.cmt32;
-            cn = w.cn32;
-            cmax_dev = w.cmax2;
-        }
-        const bool split = Dq <= 128;  // bfloat16 split operands, else float32
-        const int NS = split ? band_steps_bf16(Dq) : 0;
-        pad_queries_kernel<<<(unsigned)((B + kWavesPerBlock - 1) / kWavesPerBlock), kBlock, 0,
-                             st>>>(xq, B, ix->D, Dq, split ? nullptr : w.qt32, w.qn32, NS,
-                                   split ? reinterpret_cast<uint16_t*>(w.qtb) : nullptr);
-        if ((rc = check_launch("pad_queries_kernel"))) return rc;
-        float* a32 = reinterpret_cast<float*>(w.cd64);  // [B, nlist] approximations
-        // the streaming selector's tile minima (bfloat16 pass, from kTileMinNlist centroids)
-        float* tmin = ix->nlist >= kTileMinNlist && split ? w.tmin : nullptr;
-        if (split) {
-            const int64_t npair = ((int64_t)ix->nlist + 15) / 16 * 16 * 16 * NS;
-            centroid_bf16_kernel<<<(unsigned)std::min<int64_t>((npair + 255) / 256, 4096), 256, 0,
-                                   st>>>(cm, ix->nlist, Dq, NS, w.cmtb);
-            if ((rc = check_launch("centroid_bf16_kernel"))) return rc;
+    int rc = TRIDENT_OK;
+    const bool band = nprobe <= 128;
+    const int Dq = band_dq(ix->D);
+    const float *cm = ix->cent_rows, *cn = ix->cent_norms;
+    const unsigned long long* cmax_dev = nullptr;
+    if (band && !cm) {  // derive the centroid layouts into the workspace
+        fill_u64_kernel<<<1, 64, 0, st>>>(w.cmax2, 0ull, 1);
+        if ((rc = check_launch("fill_u64_kernel"))) return rc;
+        pad_centroids_kernel<<<(unsigned)((ix->nlist + 63) / 64), 256, 0, st>>>(
+            ix->W_combined, ldw, ix->nlist, ix->D, Dq, w.cm32, w.cn32, w.cmax2);
+        if ((rc = check_launch("pad_centroids_kernel"))) return rc;
+        cm = w.cm32;
+        cn = w.cn32;
+        cmax_dev = w.cmax2;
+    }
+    if ((rc = launch_prologue(ix, xq, B, rot, band, cm, w, clear, st))) return rc;
+    if (band) {  // band front end
+        const bool two = band_parts(Dq) == 2;  // Dq <= 128
+        const int NS = band_steps_bf16(Dq);
+        float* a32 = reinterpret_cast<float*>(w.cd64);  // [B, band_lda(nlist)] approximations
+        // the streaming selector's tile minima (two-part pass, from kTileMinNlist centroids)
+        float* tmin = ix->nlist >= kTileMinNlist && two ? w.tmin : nullptr;
+        if (two) {
             const int64_t nst = ((ix->nlist + 15) / 16 + kStageTiles - 1) / kStageTiles;
             const int64_t spx = (nst + 7) / 8, nqb = (B + 63) / 64;
             const int64_t want = std::min<int64_t>(spx, std::max<int64_t>(1, kStreamBlocks / (8 * nqb)));
@@ -726,19 +764,26 @@ int run_front_end(const TridentIndexView* ix, const float* xq, int B, int nprobe
             }
             if ((rc = check_launch("coarse_gemm_bf16_kernel"))) return rc;
         } else {
-            const int64_t ncg = (ix->nlist + 16 * kGemmTiles - 1) / (16 * kGemmTiles);
-            coarse_gemm_kernel<<<(unsigned)(8 * ((B + 63) / 64) * ((ncg + 7) / 8)), kBlock, 0, st>>>(
-                w.qt32, w.qn32, B, cmt, cn, ix->nlist, Dq, a32);
-            if ((rc = check_launch("coarse_gemm_kernel"))) return rc;
+            // few queries (under four waves a CU of 64-centroid tiles): split the dimensions
+            const int64_t qt = (B + 15) / 16, ntl = (ix->nlist + 15) / 16;
+            const int64_t ncg = (ntl + kGemmTiles - 1) / kGemmTiles;
+            if (qt * ncg < 1024)
+                coarse_gemm_split3_kernel<1, true><<<(unsigned)(qt * ntl), kBlock, 0, st>>>(
+                    w.qtb, w.qn32, B, w.cmtb, cn, ix->nlist, NS, a32);
+            else
+                coarse_gemm_split3_kernel<kGemmTiles, false>
+                    <<<(unsigned)(8 * ((B + 63) / 64) * ((ncg + 7) / 8)), kBlock, 0, st>>>(
+                        w.qtb, w.qn32, B, w.cmtb, cn, ix->nlist, NS, a32);
+            if ((rc = check_launch("coarse_gemm_split3_kernel"))) return rc;
         }
-        const double kappa = split ? band_kappa_bf16(Dq) : band_kappa_f32(Dq);
-        const double kabs = split ? band_kabs_bf16(Dq) : 0.0;
+        const double kappa = two ? band_kappa_bf16(Dq) : band_kappa_split3(Dq);
+        const double kabs = band_kabs_bf16(Dq);
         const unsigned grid = (unsigned)((B + kWavesPerBlock - 1) / kWavesPerBlock);
         const int V = ix->nlist <= 1024 ? 16 : ix->nlist <= kBandMaxNlist ? 32 : 0;
 #define TRIDENT_BAND_LAUNCH(KPV, VV, SS)                                                         \
     select_band_kernel<KPV, VV, SS><<<grid, kBlock, 0, st>>>(                                   \
         a32, w.xq64, cm, cmax_dev, ix->cent_norm_max, B, ix->nlist, ix->D, Dq, kappa, kabs,     \
-        SS ? tmin : nullptr, split ? band_lda(ix->nlist) : ix->nlist, nprobe,                    \
+        SS ? tmin : nullptr, band_lda(ix->nlist), nprobe,                    \
         w.probe_cids,                                                                           \
         w.probe_dqcs, nprobe, probe_cids, probe_dqcs, ld)
         if (nprobe <= 64) {
@@ -825,48 +870,78 @@ int launch_scatter_pairs(const int32_t* probe_cids, const float* probe_dqcs, int
     return check_launch("scatter_pairs_kernel");
 }
 
-// joint = false: each pass's pairs grouped by cluster in its own array (p1*, p2*), seg_off =
-// [2, nlist + 1] per-pass segment offsets (the per-pair route).  With a rank buffer (B * nprobe)
-// and counters past the LDS histogram, the count keeps each pair's rank in its bin and the
-// scatter needs no atomics.  joint = true: one cluster-major
-// array (p1* and p2* the same array), each cluster's pass-1 pairs before its pass-2 pairs,
-// seg_off rows = cluster starts and pass-2 starts (the batched route).
-int group_pairs(const int32_t* probe_cids, const float* probe_dqcs, int ld, int B, int nprobe,
-                int p_init, int nlist, int32_t* counts, int32_t* seg_off, int32_t* cursor,
-                int32_t* p1c, int32_t* p1q, float* p1d, int32_t* p2c, int32_t* p2q, float* p2d,
-                bool joint, int32_t* blk_tot, int32_t* rank, hipStream_t st) {
-    int rc = fill(counts, 0, 2 * ((int64_t)nlist + 1), st);
-    if (rc) return rc;
-    const bool ranked = rank && group_lds_bytes(nlist) > 64 * 1024;
+// The pairs per pass and cluster (counts zero on entry) and each pair's arrival rank in its bin:
+// LDS histograms while 2 (nlist + 1) counters fit 64 KiB, one returning global atomic per pair past
+// that (at nlist 16,384 a chunk has about one pair per four counters: nothing to aggregate).
+int launch_count_ranks(const int32_t* probe_cids, int B, int nprobe, int p_init, int nlist,
+                       int32_t* counts, int32_t* rank, hipStream_t st) {
     const int64_t total = (int64_t)B * nprobe;
-    const unsigned gblocks = (unsigned)std::min<int64_t>((total + 255) / 256, 8192);
-    if (ranked) {
-        count_pairs_rank_kernel<<<gblocks, 256, 0, st>>>(probe_cids, ld, B, nprobe, p_init, nlist,
-                                                         counts, rank);
-        if ((rc = check_launch("count_pairs_rank_kernel"))) return rc;
-    } else if ((rc = launch_count_pairs(probe_cids, ld, B, nprobe, p_init, nlist, counts, st))) {
-        return rc;
+    if (group_lds_bytes(nlist) <= 64 * 1024) {
+        count_pairs_rank_lds_kernel<<<(unsigned)((total + kRankChunk - 1) / kRankChunk), 1024,
+                                      group_lds_bytes(nlist), st>>>(probe_cids, nprobe, B, nprobe, p_init,
+                                                                    nlist, counts, rank);
+        return check_launch("count_pairs_rank_lds_kernel");
     }
-    if (joint) {
-        // nlist <= kMaxBatchedNlist (choose_route), so the block totals fit one block's scan
-        const int nblk = (nlist + kBlock - 1) / kBlock;
-        scan_pairs_joint_local_kernel<<<nblk, kBlock, 0, st>>>(counts, nlist, seg_off, blk_tot);
-        if ((rc = check_launch("scan_pairs_joint_local_kernel"))) return rc;
-        scan_pairs_joint_carry_kernel<<<nblk, kBlock, 0, st>>>(counts, nlist, blk_tot, nblk,
-                                                               seg_off, cursor);
-        if ((rc = check_launch("scan_pairs_joint_carry_kernel"))) return rc;
-    } else {
-        scan_pairs_kernel<<<2, kBlock, 0, st>>>(counts, nlist, seg_off, cursor);
-        if ((rc = check_launch("scan_pairs_kernel"))) return rc;
-    }
-    if (ranked) {
-        scatter_pairs_rank_kernel<<<gblocks, 256, 0, st>>>(probe_cids, probe_dqcs, ld, B, nprobe,
-                                                           p_init, nlist, seg_off, rank, p1c, p1q,
-                                                           p1d, p2c, p2q, p2d);
-        return check_launch("scatter_pairs_rank_kernel");
-    }
-    return launch_scatter_pairs(probe_cids, probe_dqcs, ld, B, nprobe, p_init, nlist, cursor, p1c,
-                                p1q, p1d, p2c, p2q, p2d, st);
+    const unsigned blocks = (unsigned)std::min<int64_t>((total + 255) / 256, 8192);
+    count_pairs_rank_kernel<<<blocks, 256, 0, st>>>(probe_cids, nprobe, B, nprobe, p_init, nlist, counts, rank);
+    return check_launch("count_pairs_rank_kernel");
+}
+
+// The per-pair route's grouping: each pass's pairs by cluster in its own array (p1*, p2*).
+int group_pairs(const Workspace& w, int B, int nprobe, int p_init, int nlist, int32_t* p1c, int32_t* p1q,
+                float* p1d, int32_t* p2c, int32_t* p2q, float* p2d, hipStream_t st) {
+    int rc = launch_count_ranks(w.probe_cids, B, nprobe, p_init, nlist, w.counts, w.pair_rank, st);
+    if (rc) return rc;
+    scan_pairs_kernel<<<2, kBlock, 0, st>>>(w.counts, nlist, w.seg_off, w.seg_off);
+    if ((rc = check_launch("scan_pairs_kernel"))) return rc;
+    const unsigned blocks = (unsigned)std::min<int64_t>(((int64_t)B * nprobe + 255) / 256, 8192);
+    scatter_pairs_rank_kernel<<<blocks, 256, 0, st>>>(w.probe_cids, w.probe_dqcs, nprobe, B, nprobe, p_init,
+                                                      nlist, w.seg_off, w.pair_rank, p1c, p1q, p1d, p2c, p2q,
+                                                      p2d);
+    return check_launch("scatter_pairs_rank_kernel");
+}
+
+// The batched routes' grouping: the cluster-major pairs, work units and weight groups, and (with
+// the rotation's error bounds qerr) the queries' qep.
+int group_units(const TridentIndexView* ix, const Workspace& w, int B, int nprobe, int p_init, int uqB,
+                int seed_all, int seed_sl, int sv, int svb, bool dqc, bool rotated, hipStream_t st) {
+    int rc = launch_count_ranks(w.probe_cids, B, nprobe, p_init, ix->nlist, w.counts, w.pair_rank, st);
+    if (rc) return rc;
+    GroupArgs g{};
+    g.probe_cids = w.probe_cids;
+    g.probe_dqcs = w.probe_dqcs;
+    g.B = B;
+    g.nprobe = nprobe;
+    g.p_init = p_init;
+    g.nlist = ix->nlist;
+    g.counts = w.counts;
+    g.rank = w.pair_rank;
+    g.vec_off = ix->cluster_vec_off;
+    g.uqB = uqB;
+    g.seed_all = seed_all;
+    g.seed_sl = seed_sl;
+    g.sv = sv;
+    g.svb = svb;
+    g.seg = w.seg_off;
+    g.unit_off = w.unit_off;
+    g.grp_off = w.grp_off;
+    g.pair_cid = w.pair_cids;
+    g.pair_qid = w.pair_qids;
+    g.pair_dqc = dqc ? w.pair_dqcs : nullptr;
+    g.units = w.units;
+    g.max_units = (int)w.max_units;
+    g.groups = w.groups;
+    g.max_groups = (int)w.max_groups;
+    g.qerr = w.qerr;
+    g.D_pad = ix->D_pad;
+    g.qep = w.qep;
+    group_scan_kernel<<<1, 1024, 0, st>>>(g);
+    if ((rc = check_launch("group_scan_kernel"))) return rc;
+    g.nb_scatter = (int)std::min<int64_t>(((int64_t)B * nprobe + kBlock - 1) / kBlock, 4096);
+    g.nb_fill = (int)std::min<int64_t>((w.max_units + kBlock - 1) / kBlock, 512);
+    const int nb_qep = rotated ? (B + kWavesPerBlock - 1) / kWavesPerBlock : 0;
+    group_fill_kernel<<<(unsigned)(g.nb_scatter + g.nb_fill + nb_qep), kBlock, 0, st>>>(g);
+    return check_launch("group_fill_kernel");
 }
 
 }  // namespace
@@ -941,7 +1016,7 @@ int trident_coarse_probe(const TridentIndexView* ix, const float* xq, int32_t B,
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);
-    return run_front_end(ix, xq, B, nprobe, false, w, probe_cids, probe_dqcs, probe_ld,
+    return run_front_end(ix, xq, B, nprobe, kRotNone, w, ClearArgs{}, probe_cids, probe_dqcs, probe_ld,
                          static_cast<hipStream_t>(stream));
 }
 
@@ -1033,21 +1108,13 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
 
     // Probes always land in the workspace (row stride nprobe); the caller's buffers, when
     // given, receive a mirror copy from the same kernel.
-    int32_t* pc = w.probe_cids;
     float* pd = w.probe_dqcs;
-    const int ld = nprobe;
     auto mark = [&](int ev) -> int {
         if (!out->events || ev >= out->n_events || !out->events[ev]) return TRIDENT_OK;
         hipError_t e = hipEventRecord(static_cast<hipEvent_t>(out->events[ev]), st);
         return e == hipSuccess ? TRIDENT_OK
                                : fail(TRIDENT_ERR_HIP, "hipEventRecord: %s", hipGetErrorString(e));
     };
-    if ((rc = mark(TRIDENT_EV_START))) return rc;
-    if ((rc = run_front_end(ix, xq, B, nprobe, cascade || hat, w, out->probe_cids,
-                            out->probe_dqcs, out->probe_ld, st)))
-        return rc;
-    if ((rc = mark(TRIDENT_EV_PROBED))) return rc;
-
     // where the base lives: mapped host memory (out of core) changes the refine and, with
     // residual codes, the seeding; the PCIe telemetry counts rows read from there
     bool xb_host = false;
@@ -1065,35 +1132,72 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         return rc;
     // both batched routes group the pairs cluster-major in one array
     const bool batched = route == TRIDENT_ROUTE_BATCHED || cm;
+    // the prologue clears the counters and the telemetry, and the batched routes' per-query state
+    unsigned long long* host_rows =
+        out->host_rows && xb_host ? reinterpret_cast<unsigned long long*>(out->host_rows) : nullptr;
+    ClearArgs clear{};
+    {
+        int n = 0;
+        auto zero = [&](void* p, int64_t words) {
+            if (!p || words <= 0) return;
+            clear.p[n] = static_cast<int32_t*>(p);
+            clear.n[n++] = words;
+        };
+        static_assert(kClears >= 7, "one run of zero words each");
+        zero(w.counts, 2 * ((int64_t)ix->nlist + 1));
+        zero(out->stats, 8);
+        zero(out->stats ? w.stat_slots : nullptr, 2 * 4 * kStatSlots);
+        zero(out->host_rows, 2);
+        zero(out->host_rows_seed, 2);
+        zero(batched ? (void*)w.unit_ctr : (void*)w.cand_cnt, batched ? 2 * 8 * kCtrStride : B);
+        zero(w.ovf_n, 1);
+        if (batched) {
+            clear.tau = w.tau64;
+            clear.ub_best = w.ub_best;
+            clear.cand_cnt = w.cand_cnt;
+            clear.ub_cnt = w.ub_cnt;
+            clear.seed_cnt = w.seed_cnt;
+        }
+    }
+    if ((rc = mark(TRIDENT_EV_START))) return rc;
+    if ((rc = run_front_end(ix, xq, B, nprobe, hat ? kRotChain : cascade ? kRotMatrix : kRotNone, w, clear,
+                            out->probe_cids, out->probe_dqcs, out->probe_ld, st)))
+        return rc;
+    if ((rc = mark(TRIDENT_EV_PROBED))) return rc;
+
     // the matrix-core mode 10 first scans each query's nearest probe (p_init of them when the
     // caller sets it) for thresholds only, so that its other probes, scanned together, start
     // from a threshold instead of +inf
     if (cm) p_init = sp->p_init >= 0 ? std::min(sp->p_init, nprobe) : (nprobe > 1 ? 1 : 0);
     const int64_t M1 = (int64_t)B * p_init, M2 = (int64_t)B * (nprobe - p_init);
-    // per-pair route: the two passes' pairs in consecutive arrays; batched: one cluster-major
-    // array (group_pairs)
-    int32_t *p1c = w.pair_cids, *p1q = w.pair_qids;
-    float* p1d = w.pair_dqcs;
-    int32_t *p2c = batched ? p1c : w.pair_cids + M1, *p2q = batched ? p1q : w.pair_qids + M1;
-    float* p2d = batched ? p1d : w.pair_dqcs + M1;
-    if ((rc = group_pairs(pc, pd, ld, B, nprobe, p_init, ix->nlist, w.counts, w.seg_off, w.cursor,
-                          p1c, p1q, pd ? p1d : nullptr, p2c, p2q, pd ? p2d : nullptr, batched, w.blk_tot,
-                          w.pair_rank, st)))
-        return rc;
+    // per-pair route: the two passes' pairs in consecutive arrays; batched: one cluster-major array
+    int32_t *p1c = w.pair_cids, *p1q = w.pair_qids, *p2c = w.pair_cids + M1, *p2q = w.pair_qids + M1;
+    float *p1d = w.pair_dqcs, *p2d = w.pair_dqcs + M1;
+    // TRIDENT_UB_SEED 2 seeds from every probe, 0 and 1 from the first p_init
+    const int seed_all = cascade && sp->ub_seed == 2 ? 1 : 0;
+    const bool fine = ix->fine_codes && ix->fine_qp && xb_host;
+    if (cm) {
+        rc = group_units(ix, w, B, nprobe, p_init, kUnitQWide, 0, seed_slice_count(K, false, false), kSplitVec,
+                         kSplitVec, false, false, st);
+    } else if (batched) {
+        const int split_vec = ix->D_pad <= 256 ? kSplitVecNarrow : kSplitVec;
+        const int split_vec_b =
+            ix->D_pad <= 256 && (int64_t)ix->N >= (int64_t)kLongSliceRows * ix->nlist ? 2 * kSplitVecNarrow
+                                                                                  : split_vec;
+        // seeding slices: split_vec rows, or the index's seed_rows (at least 512, so that no
+        // slice is empty) when its rows within a cluster put the best seeds first
+        const int split_vec_a =
+            ix->seed_rows > 0 ? std::max(512, std::min(split_vec, (int)ix->seed_rows)) : split_vec;
+        rc = group_units(ix, w, B, nprobe, p_init, lb_unit_q(ix->D_pad), seed_all,
+                         seed_slice_count(K, xb_host, fine), split_vec_a, split_vec_b, sp->use_l1 != 0, true, st);
+    } else {
+        rc = group_pairs(w, B, nprobe, p_init, ix->nlist, p1c, p1q, p1d, p2c, p2q, p2d, st);
+    }
+    if (rc) return rc;
     if ((rc = mark(TRIDENT_EV_GROUPED))) return rc;
 
     const int KP = list_kp(K_list);
     const int64_t cap = w.cap;
-    if (out->stats) {
-        if ((rc = fill(reinterpret_cast<int32_t*>(out->stats), 0, 8, st))) return rc;
-        if ((rc = fill(reinterpret_cast<int32_t*>(w.stat_slots), 0, 2 * 4 * kStatSlots, st))) return rc;
-    }
-    unsigned long long* host_rows =
-        out->host_rows && xb_host ? reinterpret_cast<unsigned long long*>(out->host_rows) : nullptr;
-    if (out->host_rows && (rc = fill(reinterpret_cast<int32_t*>(out->host_rows), 0, 2, st))) return rc;
-    if (out->host_rows_seed &&
-        (rc = fill(reinterpret_cast<int32_t*>(out->host_rows_seed), 0, 2, st)))
-        return rc;
     // at the end of the seeding pass: the rows it read from host memory so far
     auto seed_rows = [&]() -> int {
         if (!out->host_rows_seed || !host_rows) return TRIDENT_OK;
@@ -1154,27 +1258,6 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         b.seed_cnt = w.seed_cnt;
         b.qep = w.qep;
         b.fine_mode = 1;  // the candidate keys hold (lb, ub): the refine skips lb > tau
-        // per-query state (tau, counts, thresholds) and the work counters
-        aux_bounds_kernel<<<(unsigned)((B + kWavesPerBlock - 1) / kWavesPerBlock), kBlock, 0,
-                            st>>>(b, 0, B, w.cbound, w.qep, w.unit_ctr);
-        if ((rc = check_launch("aux_bounds_kernel"))) return rc;
-        {
-            const int nblk = (2 * ix->nlist + kBlock - 1) / kBlock;
-            unit_scan_local_kernel<<<nblk, kBlock, 0, st>>>(w.seg_off, ix->cluster_vec_off,
-                                                            ix->nlist, b.unit_q, 0,
-                                                            seed_slice_count(K, false, false),
-                                                            kSplitVec, kSplitVec, w.unit_off, w.grp_off,
-                                                            w.blk_tot);
-            if ((rc = check_launch("unit_scan_local_kernel"))) return rc;
-            unit_scan_carry_kernel<<<nblk, kBlock, 0, st>>>(ix->nlist, w.blk_tot, nblk,
-                                                            w.unit_off, w.grp_off);
-            if ((rc = check_launch("unit_scan_carry_kernel"))) return rc;
-        }
-        unit_fill_kernel<<<(unsigned)std::min<int64_t>((w.max_units + 255) / 256, 2048), 256, 0,
-                           st>>>(w.seg_off, ix->cluster_vec_off, ix->nlist, b.unit_q, 0,
-                                 kSplitVec, kSplitVec, w.unit_off, w.units, (int)w.max_units, w.grp_off,
-                                 w.groups, (int)w.max_groups);
-        if ((rc = check_launch("unit_fill_kernel"))) return rc;
         const unsigned qg = (unsigned)((B + kWavesPerBlock - 1) / kWavesPerBlock);
         if (M1 > 0) {
             // warm-up over the first probes: for K <= 16 the scan's own thresholds (the K-th
@@ -1277,7 +1360,12 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         // then come from HBM, and only rows that can still enter the top-K are read)
         b.fine_codes = ix->fine_codes;
         b.fine_qp = ix->fine_qp;
-        b.fine_mode = ix->fine_codes && ix->fine_qp && b.xb_host ? 1 : 0;
+        b.fine_mode = fine ? 1 : 0;
+        b.ovf_max = KP <= 128 ? (int)w.ovf_max : 0;
+        b.ovf_n = w.ovf_n;
+        b.ovf_q = w.ovf_q;
+        b.ovf_slot = w.ovf_slot;
+        b.ovf_done = w.ovf_done;
         b.units = w.units;
         b.unit_off = w.unit_off;
         b.max_units = (int)w.max_units;
@@ -1303,37 +1391,11 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         b.groups = w.groups;
         b.grp_off = w.grp_off;
         b.max_groups = (int)w.max_groups;
-        const int ncl = ix->cluster_bounds ? 0 : ix->nlist;
-        aux_bounds_kernel<<<(unsigned)((ncl + B + kWavesPerBlock - 1) / kWavesPerBlock), kBlock,
-                            0, st>>>(b, ncl, B, w.cbound, w.qep, w.unit_ctr);
-        if ((rc = check_launch("aux_bounds_kernel"))) return rc;
-        // TRIDENT_UB_SEED 2 seeds from every probe, 0 and 1 from the first p_init
-        const int seed_all = sp->ub_seed == 2 ? 1 : 0;
-        const int split_vec = ix->D_pad <= 256 ? kSplitVecNarrow : kSplitVec;
-        const int split_vec_b =
-            ix->D_pad <= 256 && (int64_t)ix->N >= (int64_t)kLongSliceRows * ix->nlist ? 2 * kSplitVecNarrow
-                                                                                  : split_vec;
-        const int seed_sl = seed_slice_count(K, xb_host, b.fine_mode != 0);
-        // seeding slices: split_vec rows, or the index's seed_rows (at least 512, so that no
-        // slice is empty) when its rows within a cluster put the best seeds first
-        const int split_vec_a =
-            ix->seed_rows > 0 ? std::max(512, std::min(split_vec, (int)ix->seed_rows)) : split_vec;
-        {
-            const int nblk = (2 * ix->nlist + kBlock - 1) / kBlock;  // <= kBlock (kMaxBatchedNlist)
-            unit_scan_local_kernel<<<nblk, kBlock, 0, st>>>(w.seg_off, ix->cluster_vec_off,
-                                                            ix->nlist, b.unit_q, seed_all, seed_sl,
-                                                            split_vec_a, split_vec_b, w.unit_off, w.grp_off,
-                                                            w.blk_tot);
-            if ((rc = check_launch("unit_scan_local_kernel"))) return rc;
-            unit_scan_carry_kernel<<<nblk, kBlock, 0, st>>>(ix->nlist, w.blk_tot, nblk,
-                                                            w.unit_off, w.grp_off);
-            if ((rc = check_launch("unit_scan_carry_kernel"))) return rc;
+        if (!ix->cluster_bounds) {
+            cluster_bounds_kernel<<<(unsigned)((ix->nlist + kWavesPerBlock - 1) / kWavesPerBlock), kBlock, 0,
+                                    st>>>(b, ix->nlist, w.cbound);
+            if ((rc = check_launch("cluster_bounds_kernel"))) return rc;
         }
-        unit_fill_kernel<<<(unsigned)std::min<int64_t>((w.max_units + 255) / 256, 2048), 256, 0,
-                           st>>>(w.seg_off, ix->cluster_vec_off, ix->nlist, b.unit_q, seed_all,
-                                 split_vec_a, split_vec_b, w.unit_off, w.units, (int)w.max_units, w.grp_off,
-                                 w.groups, (int)w.max_groups);
-        if ((rc = check_launch("unit_fill_kernel"))) return rc;
         if ((rc = launch_pair_prep(b, st))) return rc;
         if (M1 > 0 || seed_all) {
             // pass A: per-query upper bounds from the seeding probes, then the exact distances of
@@ -1428,22 +1490,17 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
             m.ovf_q = w.ovf_q;
             m.ovf_slot = w.ovf_slot;
             m.ovf_t = w.ovf_t;
+            m.ovf_done = w.ovf_done;
             m.ovf_key = w.ovf_key;
             m.ovf_id = w.ovf_id;
-            if ((rc = fill(w.ovf_n, 0, 1, st))) return rc;
-            ovf_collect_kernel<<<(unsigned)((B + 255) / 256), 256, 0, st>>>(m);
-            if ((rc = check_launch("ovf_collect_kernel"))) return rc;
             const size_t odyn = (size_t)kWavesPerBlock * 3 * ix->D_pad * sizeof(float);
             const unsigned og = (unsigned)std::min<int64_t>(
                 (w.ovf_max * nprobe + kWavesPerBlock - 1) / kWavesPerBlock, 2048);
-            const unsigned kg = (unsigned)((w.ovf_max + kWavesPerBlock - 1) / kWavesPerBlock);
             if (KP == 64) {
                 ovf_scan_kernel<64, true><<<og, kBlock, odyn, st>>>(m);
-                ovf_kth_kernel<64><<<kg, kBlock, 0, st>>>(m);
                 ovf_scan_kernel<64, false><<<og, kBlock, odyn, st>>>(m);
             } else {
                 ovf_scan_kernel<128, true><<<og, kBlock, odyn, st>>>(m);
-                ovf_kth_kernel<128><<<kg, kBlock, 0, st>>>(m);
                 ovf_scan_kernel<128, false><<<og, kBlock, odyn, st>>>(m);
             }
             if ((rc = check_launch("ovf_scan_kernel"))) return rc;
@@ -1467,8 +1524,7 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
                               : kind1;
     // mode 0 with a rerank: the merges only build the top-M list; rerank_kernel writes the outputs
     const bool rerank = eff_rr > 0;
-    if (M1 > 0) {
-        if ((rc = fill(w.cand_cnt, 0, B, st))) return rc;
+    if (M1 > 0) {  // cand_cnt is zero
         a.pair_cid = p1c;
         a.pair_qid = p1q;
         a.pair_dqc = pd ? p1d : nullptr;
@@ -1489,7 +1545,7 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
     if ((rc = seed_rows())) return rc;
     if ((rc = mark(TRIDENT_EV_P1_MERGE))) return rc;
     if (M2 > 0) {
-        if ((rc = fill(w.cand_cnt, 0, B, st))) return rc;
+        if (M1 > 0 && (rc = fill(w.cand_cnt, 0, B, st))) return rc;
         a.pair_cid = p2c;
         a.pair_qid = p2q;
         a.pair_dqc = pd ? p2d : nullptr;
@@ -1579,13 +1635,7 @@ int trident_sq8_bounds(const TridentIndexView* ix, const float* xq, int32_t B,
                     w.bytes);
     if (n == 0) return TRIDENT_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const int ldw = ix->nlist + ix->D_pad;
-    const int cols = std::max(ix->D, ix->D_pad);
-    prep_queries_kernel<<<dim3((cols + 127) / 128, (B + 4 * kPrepQB - 1) / (4 * kPrepQB)),
-                          dim3(64, 4), 0, st>>>(
-        xq, B, ix->D, ix->D_pad, ix->W_combined, ldw, ix->nlist, ix->b_combined, w.xq64,
-        w.xrot64, w.xrot32, w.qerr, 1);
-    if ((rc = check_launch("prep_queries_kernel"))) return rc;
+    if ((rc = launch_prologue(ix, xq, B, kRotMatrix, false, nullptr, w, ClearArgs{}, st))) return rc;
     ScanArgs a = make_scan_args(ix, w, 1, 1, 0, nullptr);
     sq8_bounds_kernel<<<(n + 255) / 256, 256, 0, st>>>(a, qids, cids, spos, n, lb, ub);
     return check_launch("sq8_bounds_kernel");
@@ -1603,10 +1653,9 @@ int trident_cluster_bounds(const TridentIndexView* ix, double* cluster_bounds, v
     b.eps = ix->eps_dim;
     b.vec_off = ix->cluster_vec_off;
     b.vec_Ar = reinterpret_cast<const float2*>(ix->vec_Ar);
-    aux_bounds_kernel<<<(unsigned)((ix->nlist + kWavesPerBlock - 1) / kWavesPerBlock), kBlock, 0,
-                        static_cast<hipStream_t>(stream)>>>(b, ix->nlist, 0, cluster_bounds,
-                                                            nullptr, nullptr);
-    return check_launch("aux_bounds_kernel");
+    cluster_bounds_kernel<<<(unsigned)((ix->nlist + kWavesPerBlock - 1) / kWavesPerBlock), kBlock, 0,
+                            static_cast<hipStream_t>(stream)>>>(b, ix->nlist, cluster_bounds);
+    return check_launch("cluster_bounds_kernel");
 }
 
 int trident_fine_bounds(const TridentIndexView* ix, const float* xq, int32_t B,
@@ -1624,13 +1673,7 @@ int trident_fine_bounds(const TridentIndexView* ix, const float* xq, int32_t B,
                     w.bytes);
     if (n == 0) return TRIDENT_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const int ldw = ix->nlist + ix->D_pad;
-    const int cols = std::max(ix->D, ix->D_pad);
-    prep_queries_kernel<<<dim3((cols + 127) / 128, (B + 4 * kPrepQB - 1) / (4 * kPrepQB)),
-                          dim3(64, 4), 0, st>>>(
-        xq, B, ix->D, ix->D_pad, ix->W_combined, ldw, ix->nlist, ix->b_combined, w.xq64,
-        w.xrot64, w.xrot32, w.qerr, 1);
-    if ((rc = check_launch("prep_queries_kernel"))) return rc;
+    if ((rc = launch_prologue(ix, xq, B, kRotMatrix, false, nullptr, w, ClearArgs{}, st))) return rc;
     BatchArgs b{};
     b.D = ix->D;
     b.D_pad = ix->D_pad;

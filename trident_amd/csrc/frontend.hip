@@ -25,19 +25,20 @@ __global__ void fill_i32_kernel(int32_t* p, int32_t v, int64_t n) {
         p[i] = v;
 }
 
-// grid (ceil(max(D, D_pad) / 128), ceil(B / (4 kPrepQB))), block (64, 4): each wave takes
+// The rotation as one float64 chain per (query, column), in dimension order: modes 0 / 1, whose
+// results are defined by it (every other mode takes front_prologue_kernel's rotation).
+// grid (ceil(D_pad / 128), ceil(B / (4 kPrepQB))), block (64, 4): each wave takes
 // kPrepQB queries (wave-uniform rows, scalar loads) x 128 columns (two per lane), so every
 // converted query value feeds two chains and every rotation value kPrepQB.
-// xq64[b, d] = (double)xq[b, d]; xrot64[b, j] = sum_d xq[b, d] * R[d, j] + bvec[j] evaluated
+// xrot64[b, j] = sum_d xq[b, d] * R[d, j] + bvec[j] evaluated
 // in float64 (fma, dimension order), xrot32 = xrot64 rounded to float32, and qerr[b, j] bounds
 // the distance of xrot64 from the exact value: |fl(sum) - sum| <= (D + 1) 2^-53 sum_d |x_d R_dj|
 // <= (D + 1) 2^-53 |x| |R_j| (Cauchy-Schwarz; both norms from float64 sums), taken with a
 // factor two (and the bias) for the roundings of the norms.
 __global__ __launch_bounds__(256) void prep_queries_kernel(
     const float* __restrict__ xq, int B, int D, int D_pad, const float* __restrict__ W, int ldw,
-    int nlist, const float* __restrict__ bvec, double* __restrict__ xq64,
-    double* __restrict__ xrot64, float* __restrict__ xrot32, double* __restrict__ qerr,
-    int do_rot) {
+    int nlist, const float* __restrict__ bvec, double* __restrict__ xrot64,
+    float* __restrict__ xrot32, double* __restrict__ qerr) {
     constexpr int QB = kPrepQB;
     const int lane = threadIdx.x;
     const int j0 = blockIdx.x * 128 + lane, j1 = j0 + 64;
@@ -46,13 +47,7 @@ __global__ __launch_bounds__(256) void prep_queries_kernel(
     const float* qr[QB];
 #pragma unroll
     for (int i = 0; i < QB; ++i) qr[i] = xq + (size_t)min(b0 + i, B - 1) * D;
-#pragma unroll
-    for (int i = 0; i < QB; ++i) {
-        if (b0 + i >= B) break;
-        if (j0 < D) xq64[(size_t)(b0 + i) * D + j0] = (double)qr[i][j0];
-        if (j1 < D) xq64[(size_t)(b0 + i) * D + j1] = (double)qr[i][j1];
-    }
-    if (!do_rot || j0 >= D_pad) return;
+    if (j0 >= D_pad) return;
     // squared norms of the wave's queries, dims split over the lanes
     double nx[QB];
 #pragma unroll
@@ -380,50 +375,6 @@ __global__ __launch_bounds__(256) void scan_pairs_kernel(const int32_t* counts, 
     }
 }
 
-// The cluster-major layout (each cluster's pass-1 pairs, then its pass-2 pairs) from counts
-// [2, nlist + 1]: seg_off row 0 = cluster starts, row 1 = pass-2 starts; the cursor rows are the
-// same offsets, so the scatter kernels place pass p's pair of cluster c at cursor[p][c]++ in one
-// array.  Two launches over ceil(nlist / kBlock) blocks of one cluster per thread (coalesced):
-// the first scans each block's clusters and writes the in-block offsets and the block's total,
-// the second adds the totals of the blocks before it (at most kBlock blocks).
-__global__ __launch_bounds__(256) void scan_pairs_joint_local_kernel(const int32_t* counts,
-                                                                     int nlist, int32_t* seg_off,
-                                                                     int32_t* blk_tot) {
-    __shared__ uint32_t s_wtot[kWavesPerBlock];
-    const int c = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t n = c < nlist ? (uint32_t)(counts[c] + counts[nlist + 1 + c]) : 0u;
-    uint32_t total = 0;
-    const uint32_t run = block_exclusive_scan(n, s_wtot, &total);
-    if (c < nlist) seg_off[c] = (int32_t)run;
-    if (threadIdx.x == 0) blk_tot[blockIdx.x] = (int32_t)total;
-}
-
-__global__ __launch_bounds__(256) void scan_pairs_joint_carry_kernel(const int32_t* counts,
-                                                                     int nlist,
-                                                                     const int32_t* blk_tot,
-                                                                     int nblk, int32_t* seg_off,
-                                                                     int32_t* cursor) {
-    __shared__ uint32_t s_wtot[kWavesPerBlock];
-    const int tid = threadIdx.x, c = blockIdx.x * kBlock + tid;
-    uint32_t total = 0;
-    const uint32_t t = tid < nblk ? (uint32_t)blk_tot[tid] : 0u;
-    // the exclusive prefix at thread blockIdx.x is this block's carry; broadcast it through LDS
-    __shared__ uint32_t s_carry;
-    const uint32_t before = block_exclusive_scan(t, s_wtot, &total);
-    if (tid == (int)blockIdx.x) s_carry = before;
-    __syncthreads();
-    if (c < nlist) {
-        const uint32_t base = (uint32_t)seg_off[c] + s_carry;
-        const uint32_t n1 = (uint32_t)counts[c];
-        seg_off[c] = cursor[c] = (int32_t)base;
-        seg_off[nlist + 1 + c] = cursor[nlist + 1 + c] = (int32_t)(base + n1);
-    }
-    if (blockIdx.x == 0 && tid == 0) {
-        seg_off[nlist] = cursor[nlist] = (int32_t)total;
-        seg_off[2 * nlist + 1] = cursor[2 * nlist + 1] = (int32_t)total;
-    }
-}
-
 __global__ void scatter_pairs_kernel(const int32_t* __restrict__ probe_cids,
                                      const float* __restrict__ probe_dqcs, int ld, int B,
                                      int nprobe, int p_init, int nlist, int32_t* cursor,
@@ -461,6 +412,46 @@ __global__ void count_pairs_rank_kernel(const int32_t* __restrict__ probe_cids, 
         if ((unsigned)cid >= (unsigned)nlist) continue;  // invalid caller input: never index
         rank[idx] = atomicAdd(&counts[(p < p_init ? 0 : (nlist + 1)) + cid], 1);
     }
+}
+
+// The same ranks where 2 (nlist + 1) counters fit 64 KiB of LDS: a block of 1024 threads takes
+// kRankChunk entries, ranks each within the block by a returning LDS atomic and adds its non-empty
+// bins to the counts (one global atomic per block and cluster, whose returned value completes the
+// ranks).
+__global__ __launch_bounds__(1024) void count_pairs_rank_lds_kernel(
+    const int32_t* __restrict__ probe_cids, int ld, int B, int nprobe, int p_init, int nlist,
+    int32_t* counts, int32_t* __restrict__ rank) {
+    extern __shared__ int32_t s_hist[];
+    const int H = 2 * (nlist + 1), tid = (int)threadIdx.x;
+    for (int i = tid; i < H; i += 1024) s_hist[i] = 0;
+    __syncthreads();
+    const int total = B * nprobe, i0 = blockIdx.x * kRankChunk;
+    constexpr int kPer = kRankChunk / 1024;  // entries per thread, loads issued together
+    int bin[kPer], local[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int idx = i0 + k * 1024 + tid;
+        bin[k] = -1;
+        local[k] = 0;
+        if (idx < total) {
+            const int q = idx / nprobe, p = idx - q * nprobe;
+            const int cid = probe_cids[(size_t)q * ld + p];
+            // invalid caller input: never index
+            if ((unsigned)cid < (unsigned)nlist) bin[k] = (p < p_init ? 0 : (nlist + 1)) + cid;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+        if (bin[k] >= 0) local[k] = atomicAdd(&s_hist[bin[k]], 1);
+    __syncthreads();
+    for (int i = tid; i < H; i += 1024) {
+        const int v = s_hist[i];
+        if (v) s_hist[i] = atomicAdd(&counts[i], v);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+        if (bin[k] >= 0) rank[i0 + k * 1024 + tid] = s_hist[bin[k]] + local[k];
 }
 
 __global__ void scatter_pairs_rank_kernel(const int32_t* __restrict__ probe_cids,
@@ -688,10 +679,10 @@ __global__ __launch_bounds__(256) void scatter_pairs_lds_kernel(
 // centroids that can still be among the nprobe nearest, and the exact (d, cid) selection.
 //
 // For float32 vectors q, c (exact reals) with d = |q - c|^2, nq = |q|^2, nc = |c|^2:
-//   s' = the matrix-core float32 dot product of q and c in any summation order, each product
-//        and addition with relative error <= 2^-23 (round-to-nearest gives 2^-24; the factor
-//        two also covers truncation): |s' - q.c| <= kappa sum |q_d c_d| <= kappa (nq + nc) / 2,
-//        kappa = (Dq + 2) 2^-23 (first-order bound of recursive summation over Dq terms);
+//   s' = the matrix-core dot product of q and c over split operands (below) in any summation
+//        order, each product and addition with relative error <= 2^-23 (round-to-nearest gives
+//        2^-24; the factor two also covers truncation): |s' - q.c| <= kappa sum |q_d c_d| <=
+//        kappa (nq + nc) / 2;
 //   a  = fma(-2, s', fl(nq32 + nc32)) with nq32, nc32 the float64 norms rounded to float32:
 //        the three roundings add at most 2^-22 (nq + nc) (1 + 2^-20);
 //   d64, the canonical float64 chain, is within 2^-44 (nq + nc) of d.
@@ -713,25 +704,22 @@ __global__ __launch_bounds__(256) void scatter_pairs_lds_kernel(
 // bounds |s' - q.c| / sum |q_d c_d| to first order (the margins cover the second-order terms).
 // Subnormal bfloat16 operands or float32 products that the matrix cores flush to zero add at
 // most 3 Dp 2^-126 (1 + |q|_inf + |c|_inf) <= Dp 2^-100 (1 + nq + nc) in absolute terms.
+//
+// Three-part form (Dq > 128, coarse_gemm_split3_kernel): x = h + m + l + r, |m| <= 2^-8 (1 + 2^-8)
+// |x|, |l| <= 2^-16 (1 + 2^-7) |x|, |r| <= 2^-24 |x|.  The dropped terms m l + l m + l l and those
+// with an r are at most 4.2 * 2^-24 |q_d c_d| per dimension.  The h h products pass through at most
+// Dp + 6 additions, the h m and m h ones (<= 2^-7 (1 + 2^-6) |q_d c_d| a pair) through at most
+// 2 Dp + 6, the other three (<= 3 * 2^-16 (1 + 2^-6) |q_d c_d|) through at most 3 Dp + 6, so
+//   kappa = (Dp + 6) 2^-23 (1 + 2^-7) + (2 Dp + 6) 2^-30 (1 + 2^-5) + (10 Dp + 20) 2^-39 + 4.2 * 2^-24.
 
-// Matrix-core tile layout of zero-padded float32 rows (Dq = D rounded up to 16, S = Dq / 4):
-// for rows 16 t .. 16 t + 15, float4 number (t S/4 + j) 64 + lane holds, for row 16 t + lane % 16
-// and lane group g = lane / 16, dimensions g S + 4 j .. g S + 4 j + 3 -- the A (or B) operands
-// of four consecutive v_mfma_f32_16x16x4f32 steps, so one float4 load of a wave is 1 KiB
-// contiguous.
-__device__ __forceinline__ size_t mfma_tile_offset(int row, int d, int S) {
-    const int g = d / S, sd = d - g * S;
-    return ((((size_t)(row >> 4) * (S >> 2) + (sd >> 2)) * kWave + (row & 15) + 16 * g) << 2) +
-           (sd & 3);
-}
-
-// bfloat16 split tile layout (NS 32-dim steps): for rows 16 t .. 16 t + 15, step s and part p
-// (0: h, 1: l), the 16 bytes ((t NS + s) 2 + p) 64 + lane hold row 16 t + lane % 16, dimensions
-// 32 s + 8 g .. 32 s + 8 g + 7 (g = lane / 16) -- one v_mfma_f32_16x16x32_bf16 operand, read by
-// a wave as 1 KiB contiguous.  Returns the offset of (row, d, p) in bfloat16 units.
-__device__ __forceinline__ size_t bf16_tile_offset(int row, int d, int NS, int p) {
+// bfloat16 split tile layout (NS 32-dim steps, NP parts): for rows 16 t .. 16 t + 15, step s and
+// part p (0: h, 1: l; or 0: h, 1: m, 2: l), the 16 bytes ((t NS + s) NP + p) 64 + lane hold row
+// 16 t + lane % 16, dimensions 32 s + 8 g .. 32 s + 8 g + 7 (g = lane / 16) -- one
+// v_mfma_f32_16x16x32_bf16 operand, read by a wave as 1 KiB contiguous.  Returns the offset of
+// (row, d, p) in bfloat16 units.
+__device__ __forceinline__ size_t bf16_tile_offset(int row, int d, int NS, int NP, int p) {
     const int s = d >> 5, k = d & 31;
-    return ((((size_t)(row >> 4) * NS + s) * 2 + p) * kWave + (row & 15) + 16 * (k >> 3)) * 8 +
+    return ((((size_t)(row >> 4) * NS + s) * NP + p) * kWave + (row & 15) + 16 * (k >> 3)) * 8 +
            (k & 7);
 }
 
@@ -744,58 +732,192 @@ __device__ __forceinline__ uint16_t bf16_rne(float x) {
     return (uint16_t)(fin && (r & 0x7f80u) == 0x7f80u ? (u >> 16) : r);
 }
 
-// x = h + l + r: h = bf16(x), l = bf16(x - h) (x - h is exact in float32)
-__device__ __forceinline__ void split_bf16(float x, uint16_t& h, uint16_t& l) {
-    h = bf16_rne(x);
-    l = bf16_rne(x - __uint_as_float((uint32_t)h << 16));
+// x = h + l + r (NP = 2): h = bf16(x), l = bf16(x - h); or x = h + m + l + r (NP = 3): the same
+// with the rest split once more (every difference is exact in float32).
+__device__ __forceinline__ void split_bf16(float x, int NP, uint16_t (&v)[3]) {
+    v[0] = bf16_rne(x);
+    const float r1 = x - __uint_as_float((uint32_t)v[0] << 16);
+    v[1] = bf16_rne(r1);
+    v[2] = NP > 2 ? bf16_rne(r1 - __uint_as_float((uint32_t)v[1] << 16)) : (uint16_t)0;
 }
 
-// Queries in the tile layout (qt32) and their squared norms (float64 sum, float32 copy).
-__global__ __launch_bounds__(256) void pad_queries_kernel(const float* __restrict__ xq, int B,
-                                                          int D, int Dq,
-                                                          float* __restrict__ qt32,
-                                                          float* __restrict__ qn32, int NS,
-                                                          uint16_t* __restrict__ qtb) {
-    const int lane = threadIdx.x & 63;
-    const int q = blockIdx.x * kWavesPerBlock + (int)(threadIdx.x >> 6);
-    if (q >= B) return;
-    const int S = Dq >> 2;
-    double acc = 0.0;
-    for (int d = lane; d < Dq; d += kWave) {
-        const float v = d < D ? xq[(size_t)q * D + d] : 0.0f;
-        if (qt32) qt32[mfma_tile_offset(q, d, S)] = v;
-        acc = fma((double)v, (double)v, acc);
-    }
-    if (qtb) {  // the bfloat16 split layout (NS 32-dim steps, zero past D)
-        for (int d = lane; d < 32 * NS; d += kWave) {
-            uint16_t h, l;
-            split_bf16(d < D ? xq[(size_t)q * D + d] : 0.0f, h, l);
-            qtb[bf16_tile_offset(q, d, NS, 0)] = h;
-            qtb[bf16_tile_offset(q, d, NS, 1)] = l;
-        }
-    }
+// Everything a search needs before its coarse distances, in one launch; block ranges by role:
+//   rotation  (nb_rot blocks, 16 queries x 16 NC columns each): xrot64 = xq R + b in float64,
+//             xrot32 its rounding, qerr its error bound (as prep_queries_kernel's: the bound
+//             holds for any order of the D products, with its factor of two);
+//   queries   (nb_pad): one wave per query: the float64 copy xq64, and, for the matrix-core
+//             coarse pass, the bfloat16 split qtb and the squared norm qn32;
+//   centroids (nb_cent): rows cm32 [nlist, Dq] -> the split tile layout cmtb, rows up to the
+//             next multiple of 16 and dimensions past Dq zero;
+//   clears    (nb_clear): zero words (counters, telemetry) and the per-query state.
+// These were five launches (about 4.6 us each in a stream, whatever they do) before.
+//
+// The rotation runs on v_mfma_f64_16x16x4_f64: the four waves take every fourth 16-dim step of
+// the same tile and meet in LDS, so a chain is D / 16 products long instead of D, and lane group
+// g holds dims 4 g .. 4 g + 3 of a step (any assignment shared by both operands sums the same
+// products), one 16-byte load a query.  A chain per column in scalar float64 waited on its loads:
+// 128 us for 24 queries and 176 for 1000 at D = 960; this whole launch takes 26 and 93.
+template <int NC>
+__global__ __launch_bounds__(256) void front_prologue_kernel(PrologueArgs a) {
+    typedef double d4 __attribute__((ext_vector_type(4)));
+    __shared__ double s_acc[kWavesPerBlock][NC * 4][kWave];
+    __shared__ double s_nq[kWavesPerBlock][16], s_nc[kWavesPerBlock][NC * 16];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int blk = (int)blockIdx.x;
+    if (blk < a.nb_rot) {
+        const int m = lane & 15, g = lane >> 4;
+        const int ncg = (a.D_pad + 16 * NC - 1) / (16 * NC);
+        const int q0 = blk / ncg * 16, c0 = blk % ncg * (16 * NC);
+        const int D = a.D;
+        const bool vec4 = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(a.xq) & 15) == 0;
+        const float* qr = a.xq + (size_t)min(q0 + m, a.B - 1) * D;
+        const float* wc = a.W + a.nlist + c0 + m;
+        d4 acc[NC];
+        double nq = 0.0, nc[NC];
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) acc += __shfl_xor(acc, o, kWave);
-    if (lane == 0) qn32[q] = (float)acc;
+        for (int t = 0; t < NC; ++t) {
+            acc[t] = d4{0.0, 0.0, 0.0, 0.0};
+            nc[t] = 0.0;
+        }
+        const int nst = (D + 15) >> 4;
+#pragma unroll 2
+        for (int s = wid; s < nst; s += kWavesPerBlock) {
+            const int k = 16 * s + 4 * g;
+            float qf[4] = {0.0f, 0.0f, 0.0f, 0.0f}, wf[NC][4];
+            if (vec4) {
+                if (k < D) {
+                    const float4 v = *reinterpret_cast<const float4*>(qr + k);
+                    qf[0] = v.x;
+                    qf[1] = v.y;
+                    qf[2] = v.z;
+                    qf[3] = v.w;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (k + i < D) qf[i] = qr[k + i];
+            }
+#pragma unroll
+            for (int t = 0; t < NC; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    wf[t][i] = k + i < D && c0 + 16 * t + m < a.D_pad
+                                   ? wc[(size_t)(k + i) * a.ldw + 16 * t] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double qd = (double)qf[i];
+                nq = fma(qd, qd, nq);
+#pragma unroll
+                for (int t = 0; t < NC; ++t) {
+                    const double wd = (double)wf[t][i];
+                    nc[t] = fma(wd, wd, nc[t]);
+                    acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(qd, wd, acc[t], 0, 0, 0);
+                }
+            }
+        }
+        // squared norms: over the lane groups here, over the waves below
+        nq += shfl_f64(nq, lane ^ 16);
+        nq += shfl_f64(nq, lane ^ 32);
+        if (g == 0) s_nq[wid][m] = nq;
+#pragma unroll
+        for (int t = 0; t < NC; ++t) {
+            double n = nc[t];
+            n += shfl_f64(n, lane ^ 16);
+            n += shfl_f64(n, lane ^ 32);
+            if (g == 0) s_nc[wid][16 * t + m] = n;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s_acc[wid][4 * t + i][lane] = acc[t][i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < NC; ++e) {  // result (t, i): rows g + 4 i, column m of tile t
+            const int o = e * kWavesPerBlock + wid, t = o >> 2, i = o & 3;
+            const int r = g + 4 * i, q = q0 + r, j = c0 + 16 * t + m;
+            const double sum = (s_acc[0][o][lane] + s_acc[1][o][lane]) +
+                               (s_acc[2][o][lane] + s_acc[3][o][lane]);
+            const double nx = (s_nq[0][r] + s_nq[1][r]) + (s_nq[2][r] + s_nq[3][r]);
+            const double rn = (s_nc[0][16 * t + m] + s_nc[1][16 * t + m]) +
+                              (s_nc[2][16 * t + m] + s_nc[3][16 * t + m]);
+            if (q < a.B && j < a.D_pad) {
+                const double bj = (double)a.bvec[a.nlist + j], xr = sum + bj;
+                const size_t at = (size_t)q * a.D_pad + j;
+                a.xrot64[at] = xr;
+                a.xrot32[at] = (float)xr;
+                a.qerr[at] = (double)(D + 3) * 0x1p-52 * (sqrt(nx) * sqrt(rn) * (1.0 + 1e-12) + fabs(bj)) +
+                             0x1p-1000;
+            }
+        }
+        return;
+    }
+    blk -= a.nb_rot;
+    if (blk < a.nb_pad) {
+        const int q = blk * kWavesPerBlock + wid;
+        if (q >= a.B) return;
+        const float* x = a.xq + (size_t)q * a.D;
+        double acc = 0.0;
+        for (int d = lane; d < a.D; d += kWave) {
+            const double v = (double)x[d];
+            a.xq64[(size_t)q * a.D + d] = v;
+            acc = fma(v, v, acc);
+        }
+        if (a.NS == 0) return;
+        for (int d = lane; d < 32 * a.NS; d += kWave) {
+            uint16_t v[3];
+            split_bf16(d < a.D ? x[d] : 0.0f, a.NP, v);
+            for (int p = 0; p < a.NP; ++p) a.qtb[bf16_tile_offset(q, d, a.NS, a.NP, p)] = v[p];
+        }
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) acc += shfl_f64(acc, lane ^ o);
+        if (lane == 0) a.qn32[q] = (float)acc;
+        return;
+    }
+    blk -= a.nb_pad;
+    if (blk < a.nb_cent) {
+        const int npair = 16 * a.NS;  // dimension pairs per row
+        const int64_t n = (int64_t)((a.nlist + 15) & ~15) * npair;
+        for (int64_t i = (int64_t)blk * kBlock + tid; i < n; i += (int64_t)a.nb_cent * kBlock) {
+            const int row = (int)(i / npair), d = 2 * (int)(i - (int64_t)row * npair);
+            const float* src = a.cm32 + (size_t)row * a.Dq;
+            uint16_t v0[3], v1[3];
+            split_bf16(row < a.nlist && d < a.Dq ? src[d] : 0.0f, a.NP, v0);
+            split_bf16(row < a.nlist && d + 1 < a.Dq ? src[d + 1] : 0.0f, a.NP, v1);
+            // d even: (d, d + 1) share one 32-bit word of each part
+            for (int p = 0; p < a.NP; ++p)
+                a.cmtb[bf16_tile_offset(row, d, a.NS, a.NP, p) >> 1] = (uint32_t)v0[p] | ((uint32_t)v1[p] << 16);
+        }
+        return;
+    }
+    blk -= a.nb_cent;
+    const int64_t i0 = (int64_t)blk * kBlock + tid, step = (int64_t)a.nb_clear * kBlock;
+#pragma unroll
+    for (int f = 0; f < kClears; ++f)
+        for (int64_t i = i0; i < a.clear.n[f]; i += step) a.clear.p[f][i] = 0;
+    if (a.clear.tau)
+        for (int64_t q = i0; q < a.B; q += step) {
+            a.clear.tau[q] = INFINITY;
+            a.clear.ub_best[q] = 0x7f800000u;  // +inf
+            a.clear.cand_cnt[q] = a.clear.ub_cnt[q] = a.clear.seed_cnt[q] = 0;
+        }
 }
+
+template __global__ void front_prologue_kernel<1>(PrologueArgs);
+template __global__ void front_prologue_kernel<4>(PrologueArgs);
 
 // Centroids (c_d = -0.5f W[d, c], the same float32 values the float64 chains use) as
-// centroid-major zero-padded rows cm32 [nlist, Dq] and in the tile layout (cmt32), their
-// squared norms cn32 (float64 partial sums rounded to float32: only the error bound and the
+// centroid-major zero-padded rows cm32 [nlist, Dq], their squared norms cn32 (float64 partial sums rounded to float32: only the error bound and the
 // approximations use them) and the largest squared norm (float64 bit pattern, atomicMax into a
 // cell the caller zeroes).  grid ceil(nlist / 64), block 256: 64 centroids per block,
 // transposed through LDS in 64-dim tiles (W rows read and cm32 rows written coalesced).
 __global__ __launch_bounds__(256) void pad_centroids_kernel(const float* __restrict__ W, int ldw,
                                                             int nlist, int D, int Dq,
                                                             float* __restrict__ cm32,
-                                                            float* __restrict__ cmt32,
                                                             float* __restrict__ cn32,
                                                             unsigned long long* __restrict__ cmax2) {
     __shared__ float s_t[64][65];
     __shared__ double s_n[4][64];
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     const int c0 = blockIdx.x * 64;
-    const int S = Dq >> 2;
     double nrm = 0.0;  // centroid c0 + tx over dims ty, ty + 4, ...
     for (int d0 = 0; d0 < Dq; d0 += 64) {
 #pragma unroll
@@ -810,9 +932,7 @@ __global__ __launch_bounds__(256) void pad_centroids_kernel(const float* __restr
         for (int k = 0; k < 16; ++k) {  // centroid c0 + r, dim d0 + tx
             const int r = ty + 4 * k, c = c0 + r, d = d0 + tx;
             if (c < nlist && d < Dq) {
-                const float v = s_t[tx][r];
-                cm32[(size_t)c * Dq + d] = v;
-                cmt32[mfma_tile_offset(c, d, S)] = v;
+                cm32[(size_t)c * Dq + d] = s_t[tx][r];
             }
         }
         __syncthreads();
@@ -832,110 +952,104 @@ __global__ __launch_bounds__(256) void pad_centroids_kernel(const float* __restr
     }
 }
 
-// One-dimensional grid of 8 * ceil(B / 64) * ceil(ncg / 8) blocks (ncg = ceil(nlist / (16
-// kGemmTiles)) centroid groups), block 256.  Blocks are dealt to the XCDs round-robin, so block
-// b runs on XCD b % 8: XCD x takes centroid groups [x cpx, (x + 1) cpx) (cpx = ceil(ncg / 8)) for
-// every query block, and its share of the centroid tiles stays in its L2.  Used for Dq > 128
-// (coarse_gemm_bf16_kernel takes Dq <= 128).  Each wave 16 queries (one query tile), all four
-// waves the same kGemmTiles centroid tiles in the same order.  v_mfma_f32_16x16x4f32 with query
-// rows as A (16 x 4) and centroids as B (4 x 16), operands straight from the tile layouts: a
-// chunk of 32 k-steps is 8 + 8 coalesced float4 loads, issued whole before its 32 MFMAs; steps
-// past S are zero (clamped loads, no branch among the MFMAs).
-// a32[q, c] = fma(-2, dot, nq32 + nc32).
-__global__ __launch_bounds__(256) void coarse_gemm_kernel(const float* __restrict__ qt32,
-                                                          const float* __restrict__ qn32, int B,
-                                                          const float* __restrict__ cmt32,
-                                                          const float* __restrict__ cn32,
-                                                          int nlist, int Dq,
-                                                          float* __restrict__ a32) {
+// Dq > 128: the coarse pass over three-part bfloat16 operands (x = h + m + l + r, |r| <= 2^-24
+// |x|), six products a dimension -- h h; h m, m h; h l, l h, m m, one accumulator each -- so the
+// approximations are as close as float32 matrix products were, at 16 / 6 of their rate.  A wave
+// computes 16 queries x 16 TC centroids, operands straight from the tile layouts (1 KiB a load).
+//   SPLITK false: a block's four waves take 64 queries against the same centroids; grid of
+//     8 * ceil(B / 64) * ceil(ncg / 8) blocks (ncg = ceil(nlist / (16 TC))), XCD x = block % 8
+//     taking centroid groups [x cpx, (x + 1) cpx), whose tiles stay in its L2;
+//   SPLITK true (few queries: the chip is idle otherwise): the waves take every fourth 32-dim
+//     step of one tile and meet in LDS; grid ceil(B / 16) * ncg.
+// The float32 form took 64 us for 24 queries and 79 for 1000 (nlist 512, D = 960; one wave per
+// 64 centroids walking 960 dimensions), this one 7 and 17.
+// a32[q, c] = fma(-2, dot, nq32 + nc32), rows of band_lda(nlist) floats.
+template <int TC, bool SPLITK>
+__global__ __launch_bounds__(256) void coarse_gemm_split3_kernel(const uint32_t* __restrict__ qtb,
+                                                                 const float* __restrict__ qn32,
+                                                                 int B,
+                                                                 const uint32_t* __restrict__ cmtb,
+                                                                 const float* __restrict__ cn32,
+                                                                 int nlist, int NS,
+                                                                 float* __restrict__ a32) {
     typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    __shared__ f4 s_acc[SPLITK ? kWavesPerBlock : 1][SPLITK ? TC : 1][SPLITK ? kWave : 1];
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = lane & 15, g = lane >> 4;
-    const int ncg = (nlist + 16 * kGemmTiles - 1) / (16 * kGemmTiles), cpx = (ncg + 7) >> 3;
-    const int xcd = (int)(blockIdx.x & 7), local = (int)(blockIdx.x >> 3);
-    const int bx = local / cpx, by = xcd * cpx + (local - (local / cpx) * cpx);
-    if (by >= ncg || bx * 64 >= B) return;  // the whole block
-    const int qb0 = bx * 64 + wid * 16;
-    const bool wave_live = qb0 < B;
-    const int qtile = wave_live ? qb0 / 16 : 0;
-    const int qb = wave_live ? qb0 : 0;
-    const int F = Dq >> 4;  // float4 per lane and row tile (= S / 4)
-    const float4* qt = reinterpret_cast<const float4*>(qt32) + (size_t)qtile * F * kWave + lane;
-    const bool qv = wave_live && qb + m < B;
-    auto store = [&](int n0, const f4 (&acc4)[4]) {
-        // matrix-core results: wait states before the first VALU read, fenced
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_nop 7\n\ts_nop 7");
-        __builtin_amdgcn_sched_barrier(0);
-        const f4 acc = (acc4[0] + acc4[1]) + (acc4[2] + acc4[3]);
-        const int c = n0 + m;
-        if (c < nlist) {
-            const float ncv = cn32[c];
+    const int ntl = (nlist + 15) >> 4, ncg = (ntl + TC - 1) / TC;
+    int qt, cg;
+    if constexpr (SPLITK) {
+        qt = (int)blockIdx.x / ncg;
+        cg = (int)blockIdx.x - qt * ncg;
+    } else {
+        const int cpx = (ncg + 7) >> 3;
+        const int xcd = (int)(blockIdx.x & 7), local = (int)(blockIdx.x >> 3);
+        const int bx = local / cpx;
+        cg = xcd * cpx + (local - bx * cpx);
+        qt = bx * 4 + wid;
+    }
+    if (cg >= ncg || qt * 16 >= B) return;  // SPLITK: the whole block
+    const u4* qp = reinterpret_cast<const u4*>(qtb) + (size_t)qt * NS * 3 * kWave + lane;
+    const u4* cp[TC];
+    f4 hh[TC], mid[TC], low[TC];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int q = qb + 4 * g + i;
-                if (q < B) a32[(size_t)q * nlist + c] = fmaf(-2.0f, acc[i], qn32[q] + ncv);
-            }
+    for (int t = 0; t < TC; ++t) {  // tiles past the last redo it, never stored
+        cp[t] = reinterpret_cast<const u4*>(cmtb) + (size_t)min(cg * TC + t, ntl - 1) * NS * 3 * kWave + lane;
+        hh[t] = mid[t] = low[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll 2
+    for (int s = SPLITK ? wid : 0; s < NS; s += SPLITK ? kWavesPerBlock : 1) {
+        bf8 q[3], c[TC][3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            q[p] = __builtin_bit_cast(bf8, qp[(size_t)(3 * s + p) * kWave]);
+#pragma unroll
+            for (int t = 0; t < TC; ++t) c[t][p] = __builtin_bit_cast(bf8, cp[t][(size_t)(3 * s + p) * kWave]);
         }
+#pragma unroll
+        for (int t = 0; t < TC; ++t) {  // centroids are the A operand, queries the B operand
+            hh[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[t][0], q[0], hh[t], 0, 0, 0);
+            mid[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[t][0], q[1], mid[t], 0, 0, 0);
+            low[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[t][0], q[2], low[t], 0, 0, 0);
+            mid[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[t][1], q[0], mid[t], 0, 0, 0);
+            low[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[t][1], q[1], low[t], 0, 0, 0);
+            low[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[t][2], q[0], low[t], 0, 0, 0);
+        }
+    }
+    const int lda = band_lda(nlist), qi = qt * 16 + m;
+    auto store = [&](int t, const f4& acc) __attribute__((always_inline)) {
+        // lane (m, g) holds centroids 16 t' + 4 g .. + 3 of query 16 qt + m
+        const int tt = cg * TC + t, c0 = 16 * tt + 4 * g;
+        if (tt >= ntl || qi >= B || c0 >= nlist) return;
+        const float nq = qn32[qi];
+        float4 o;
+        o.x = fmaf(-2.0f, acc[0], nq + cn32[c0]);
+        o.y = fmaf(-2.0f, acc[1], nq + cn32[min(c0 + 1, nlist - 1)]);
+        o.z = fmaf(-2.0f, acc[2], nq + cn32[min(c0 + 2, nlist - 1)]);
+        o.w = fmaf(-2.0f, acc[3], nq + cn32[min(c0 + 3, nlist - 1)]);
+        *reinterpret_cast<float4*>(a32 + (size_t)qi * lda + c0) = o;  // padding never read
     };
-    if (!wave_live) return;
-#pragma unroll 1
-    for (int t = 0; t < kGemmTiles; ++t) {
-        const int n0 = by * 16 * kGemmTiles + t * 16;
-        if (n0 >= nlist) break;
-        const bool cv = n0 + m < nlist;
-        const float4* ct = reinterpret_cast<const float4*>(cmt32) + (size_t)(n0 >> 4) * F * kWave +
-                           lane;
-        // four independent accumulator chains (k-step 4 j + u -> chain u), summed at the end:
-        // the error bound holds for any summation order
-        f4 acc4[4];
+    if constexpr (SPLITK) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) acc4[u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-        for (int f0 = 0; f0 < F; f0 += 8) {
-            float4 av[8], bv[8];
+        for (int t = 0; t < TC; ++t) s_acc[wid][t][lane] = hh[t] + (mid[t] + low[t]);
+        __syncthreads();
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const bool in = f0 + j < F;
-                const size_t o = (size_t)(in ? f0 + j : 0) * kWave;
-                av[j] = qt[o];
-                bv[j] = ct[o];
-                if (!in || !qv) av[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (!cv) bv[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            }
+        for (int t = 0; t < TC; ++t)
+            if (wid == t % kWavesPerBlock)
+                store(t, (s_acc[0][t][lane] + s_acc[1][t][lane]) + (s_acc[2][t][lane] + s_acc[3][t][lane]));
+    } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                acc4[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j].x, bv[j].x, acc4[0], 0, 0, 0);
-                acc4[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j].y, bv[j].y, acc4[1], 0, 0, 0);
-                acc4[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j].z, bv[j].z, acc4[2], 0, 0, 0);
-                acc4[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j].w, bv[j].w, acc4[3], 0, 0, 0);
-            }
-        }
-        store(n0, acc4);
+        for (int t = 0; t < TC; ++t) store(t, hh[t] + (mid[t] + low[t]));
     }
 }
 
-
-// Centroid rows cm32 [nlist, Dq] -> the bfloat16 split tile layout (NS steps), rows up to the
-// next multiple of 16 and dimensions past Dq zero.  One thread per (row, dimension pair).
-__global__ __launch_bounds__(256) void centroid_bf16_kernel(const float* __restrict__ cm32,
-                                                            int nlist, int Dq, int NS,
-                                                            uint32_t* __restrict__ cmtb) {
-    const int npair = 16 * NS;  // dimension pairs per row
-    const int64_t n = (int64_t)((nlist + 15) & ~15) * npair;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int row = (int)(i / npair), d = 2 * (int)(i - (int64_t)row * npair);
-        const float* src = cm32 + (size_t)row * Dq;
-        uint16_t h0, l0, h1, l1;
-        split_bf16(row < nlist && d < Dq ? src[d] : 0.0f, h0, l0);
-        split_bf16(row < nlist && d + 1 < Dq ? src[d + 1] : 0.0f, h1, l1);
-        // d even: (d, d + 1) share one 32-bit word of each part
-        cmtb[bf16_tile_offset(row, d, NS, 0) >> 1] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-        cmtb[bf16_tile_offset(row, d, NS, 1) >> 1] = (uint32_t)l0 | ((uint32_t)l1 << 16);
-    }
-}
+template __global__ void coarse_gemm_split3_kernel<4, false>(const uint32_t*, const float*, int, const uint32_t*,
+                                                             const float*, int, int, float*);
+template __global__ void coarse_gemm_split3_kernel<1, true>(const uint32_t*, const float*, int, const uint32_t*,
+                                                            const float*, int, int, float*);
 
 // Dq <= 128: the coarse pass on the bfloat16 matrix cores, with a block's query tiles kept for a
 // run of centroid stages.  One-dimensional grid of 8 * ceil(B / 64) * nrun blocks: block b runs
@@ -1153,7 +1267,7 @@ __global__ __launch_bounds__(256) void select_band_kernel(
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) nq += __shfl_xor(nq, o, kWave);
     // kappa: the dot product's relative bound of the pass that wrote a32, kabs its absolute
-    // term per unit of 1 + nq + nc (float32 operands: (Dq + 2) 2^-23 and 0; bfloat16 split)
+    // term per unit of 1 + nq + nc
     const double cmax2 = cmax_dev ? __longlong_as_double((long long)*cmax_dev) : cmax_host;
     const double E = (kappa + 0x1p-21) * (nq + cmax2) * (1.0 + 0x1p-10) +
                      kabs * (1.0 + nq + cmax2) + 1e-30;

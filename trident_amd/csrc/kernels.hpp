@@ -83,15 +83,17 @@ struct MergeArgs {
     const double* xrot64;       // [B, D_pad]
     const double* qerr;         // [B, D_pad]
     double lb_scale, ub_scale;  // as ScanArgs
-    // Parallel bounded rescan (ovf_par = 1, with ovf_bounds): ovf_collect_kernel gives up to
-    // ovf_max overflowed queries a slot; ovf_scan_kernel rescans them one wave per (slot, probe),
-    // each keeping its cluster's K best in ovf_key / ovf_id [ovf_max, nprobe, KP] (upper bounds
-    // first, reduced by ovf_kth_kernel to the slot's threshold ovf_t, then refined distances);
-    // merge_kernel merges a slot's lists.  Overflowed queries past ovf_max take the serial rescan.
+    // Parallel bounded rescan (ovf_par = 1, with ovf_bounds): the refine gives up to ovf_max
+    // overflowed queries a slot; ovf_scan_kernel rescans them one wave per (slot, probe), each
+    // keeping its cluster's K best in ovf_key / ovf_id [ovf_max, nprobe, KP] -- upper bounds first,
+    // which the slot's last wave to finish (ovf_done) reduces to the slot's threshold ovf_t, then
+    // refined distances; merge_kernel merges a slot's lists.  Overflowed queries past ovf_max take
+    // the serial rescan.
     int ovf_par, ovf_max;
-    int32_t* ovf_n;       // [1] overflowed queries (may exceed ovf_max); zero before the collect
+    int32_t* ovf_n;       // [1] overflowed queries (may exceed ovf_max); zero before the refine
     int32_t* ovf_q;       // [ovf_max] the query of each slot
     int32_t* ovf_slot;    // [B] each query's slot, -1 for none
+    int32_t* ovf_done;    // [ovf_max] the slot's finished waves of the first pass
     double* ovf_t;        // [ovf_max]
     uint64_t* ovf_key;
     int32_t* ovf_id;
@@ -196,6 +198,10 @@ struct BatchArgs {
     const uint16_t* fine_codes; // [N, D_pad] or null
     const float* fine_qp;       // [N, 4] (offset, step, rho, 0)
     int fine_mode;              // 1: seeds bounded and survivors filtered with the fine level
+    // refine_survivors_kernel gives up to ovf_max overflowed lists a slot of the parallel rescan
+    // (MergeArgs); 0: none
+    int ovf_max;
+    int32_t *ovf_n, *ovf_q, *ovf_slot, *ovf_done;
     int cm_emit;                // cm_scan_kernel: 1 lists rows, 0 only lowers the thresholds
     unsigned long long* host_rows;  // [1] rows read from the host-mapped base, or null
 };
@@ -209,9 +215,43 @@ __global__ void stats_fold_kernel(const unsigned long long* slots, int64_t* out)
 
 __global__ void prep_queries_kernel(const float* __restrict__ xq, int B, int D, int D_pad,
                                     const float* __restrict__ W, int ldw, int nlist,
-                                    const float* __restrict__ bvec, double* __restrict__ xq64,
-                                    double* __restrict__ xrot64, float* __restrict__ xrot32,
-                                    double* __restrict__ qerr, int do_rot);
+                                    const float* __restrict__ bvec, double* __restrict__ xrot64,
+                                    float* __restrict__ xrot32, double* __restrict__ qerr);
+
+// What front_prologue_kernel clears: kClears runs of zero words (n = 0: none), and, with tau, the
+// batched routes' per-query state (tau = ub_best = +inf, empty lists).
+constexpr int kClears = 7;
+struct ClearArgs {
+    int32_t* p[kClears];
+    int64_t n[kClears];
+    double* tau;
+    uint32_t* ub_best;
+    int32_t* cand_cnt;
+    int32_t* ub_cnt;
+    int32_t* seed_cnt;
+};
+
+struct PrologueArgs {
+    const float* xq;      // [B, D]
+    int B, D, D_pad, Dq;
+    const float* W;       // rotation: columns nlist .. nlist + D_pad of [D, ldw]
+    int ldw, nlist;
+    const float* bvec;
+    double* xq64;
+    double* xrot64;
+    float* xrot32;
+    double* qerr;
+    int NS, NP;           // 32-dim steps and parts of the split layouts (NS = 0: none wanted)
+    uint16_t* qtb;
+    float* qn32;
+    const float* cm32;
+    uint32_t* cmtb;
+    ClearArgs clear;
+    int nb_rot, nb_pad, nb_cent, nb_clear;
+};
+
+template <int NC>
+__global__ void front_prologue_kernel(PrologueArgs a);
 
 __global__ void coarse_dist_kernel(const double* __restrict__ xq64, int B, int D,
                                    const float* __restrict__ W, int ldw, int nlist,
@@ -236,16 +276,6 @@ __global__ void count_pairs_kernel(const int32_t* __restrict__ probe_cids, int l
 __global__ void scan_pairs_kernel(const int32_t* counts, int nlist, int32_t* seg_off,
                                   int32_t* cursor);
 
-// The cluster-major layout of the batched route, each cluster's pass-1 pairs followed by its
-// pass-2 pairs: seg_off[c] = the cluster's first pair, seg_off[nlist + 1 + c] = its first pass-2
-// pair (both rows end with M); cursor receives the two rows for the scatter.  Two launches of
-// nblk = ceil(nlist / kBlock) <= kBlock blocks: in-block offsets and block totals, then carries.
-__global__ void scan_pairs_joint_local_kernel(const int32_t* counts, int nlist, int32_t* seg_off,
-                                              int32_t* blk_tot);
-__global__ void scan_pairs_joint_carry_kernel(const int32_t* counts, int nlist,
-                                              const int32_t* blk_tot, int nblk, int32_t* seg_off,
-                                              int32_t* cursor);
-
 __global__ void scatter_pairs_kernel(const int32_t* __restrict__ probe_cids,
                                      const float* __restrict__ probe_dqcs, int ld, int B,
                                      int nprobe, int p_init, int nlist, int32_t* cursor,
@@ -254,20 +284,17 @@ __global__ void scatter_pairs_kernel(const int32_t* __restrict__ probe_cids,
                                      int32_t* __restrict__ p2_qids, float* __restrict__ p2_dqcs);
 
 constexpr int kGroupChunk = 2048;  // (query, probe) entries per block of the LDS grouping
+constexpr int kRankChunk = 4096;   // ... of the ranked LDS count
 // band front end (frontend.hip)
-__global__ void pad_queries_kernel(const float* __restrict__ xq, int B, int D, int Dq,
-                                   float* __restrict__ qt32, float* __restrict__ qn32, int NS,
-                                   uint16_t* __restrict__ qtb);
-__global__ void centroid_bf16_kernel(const float* __restrict__ cm32, int nlist, int Dq, int NS,
-                                     uint32_t* __restrict__ cmtb);
 __global__ void pad_centroids_kernel(const float* __restrict__ W, int ldw, int nlist, int D,
-                                     int Dq, float* __restrict__ cm32, float* __restrict__ cmt32,
-                                     float* __restrict__ cn32,
+                                     int Dq, float* __restrict__ cm32, float* __restrict__ cn32,
                                      unsigned long long* __restrict__ cmax2);
-__global__ void coarse_gemm_kernel(const float* __restrict__ qt32, const float* __restrict__ qn32,
-                                   int B, const float* __restrict__ cmt32,
-                                   const float* __restrict__ cn32, int nlist, int Dq,
-                                   float* __restrict__ a32);
+template <int TC, bool SPLITK>
+__global__ void coarse_gemm_split3_kernel(const uint32_t* __restrict__ qtb,
+                                          const float* __restrict__ qn32, int B,
+                                          const uint32_t* __restrict__ cmtb,
+                                          const float* __restrict__ cn32, int nlist, int NS,
+                                          float* __restrict__ a32);
 template <int KP, int V, bool STREAM>
 __global__ void select_band_kernel(const float* __restrict__ a32, const double* __restrict__ xq64,
                                    const float* __restrict__ cm32,
@@ -279,7 +306,7 @@ __global__ void select_band_kernel(const float* __restrict__ a32, const double* 
                                    float* __restrict__ out_dqcs, int ld,
                                    int32_t* __restrict__ out2_cids,
                                    float* __restrict__ out2_dqcs, int ld2);
-constexpr int kGemmTiles = 4;  // coarse_gemm_kernel: 16-centroid tiles per wave
+constexpr int kGemmTiles = 4;  // coarse_gemm_split3_kernel: 16-centroid tiles per wave
 // coarse_gemm_bf16_kernel (Dq <= 128): 16-centroid tiles per stage; the run of stages per
 // block is the longest that still gives a grid of about kStreamBlocks blocks
 constexpr int kStageTiles = 2;
@@ -292,8 +319,14 @@ __global__ void coarse_gemm_bf16_kernel(const uint32_t* __restrict__ qtb,
                                         const float* __restrict__ cn32, int nlist, int run_stages,
                                         float* __restrict__ a32, float* __restrict__ tmin);
 // relative and absolute dot-product bounds of the two coarse passes (select_band_kernel's E)
-inline double band_kappa_f32(int Dq) { return (double)(Dq + 2) * 0x1p-23; }
+inline double band_kappa_split3(int Dq) {
+    const double Dp = 32.0 * ((Dq + 31) / 32);
+    return (Dp + 6) * 0x1p-23 * (1.0 + 0x1p-7) + (2 * Dp + 6) * 0x1p-30 * (1.0 + 0x1p-5) +
+           (10 * Dp + 20) * 0x1p-39 + 4.2 * 0x1p-24;
+}
 inline int band_steps_bf16(int Dq) { return (Dq + 31) / 32; }
+// parts of the bfloat16 split operands: two with the wide band they need, or three
+inline int band_parts(int Dq) { return Dq <= 128 ? 2 : 3; }
 // row length (floats) of the bfloat16 coarse pass's approximations: nlist rounded up to 4, so
 // that each tile's results are one aligned 16-byte store
 __host__ __device__ inline int band_lda(int nlist) { return (nlist + 3) & ~3; }
@@ -320,6 +353,9 @@ inline size_t group_lds_bytes(int nlist) { return (size_t)2 * (nlist + 1) * size
 __global__ void count_pairs_rank_kernel(const int32_t* __restrict__ probe_cids, int ld, int B,
                                         int nprobe, int p_init, int nlist, int32_t* counts,
                                         int32_t* __restrict__ rank);
+__global__ void count_pairs_rank_lds_kernel(const int32_t* __restrict__ probe_cids, int ld, int B,
+                                            int nprobe, int p_init, int nlist, int32_t* counts,
+                                            int32_t* __restrict__ rank);
 __global__ void scatter_pairs_rank_kernel(const int32_t* __restrict__ probe_cids,
                                           const float* __restrict__ probe_dqcs, int ld, int B,
                                           int nprobe, int p_init, int nlist,
@@ -425,19 +461,37 @@ inline int64_t max_groups_of(int64_t pairs, int64_t nlist) {
     return (pairs + kGroupQ - 1) / kGroupQ + nlist;
 }
 
-// seed_all: the seeding units cover every pair of a cluster (TRIDENT_UB_SEED 2), not only its
-// pass-1 pairs; seed_sl: the seeding units scan the first seed_sl slices of each cluster.
-// Two launches of ceil(2 nlist / kBlock) blocks; blk_tot holds 2 * kBlock block totals.
-// sv: the seeding units' slice length, svb: the lower-bound units'.
-__global__ void unit_scan_local_kernel(const int32_t* seg, const int32_t* vec_off, int nlist,
-                                       int uqB, int seed_all, int seed_sl, int sv, int svb,
-                                       int32_t* unit_off, int32_t* grp_off, int32_t* blk_tot);
-__global__ void unit_scan_carry_kernel(int nlist, const int32_t* blk_tot, int nblk,
-                                       int32_t* unit_off, int32_t* grp_off);
-
-__global__ void unit_fill_kernel(const int32_t* seg, const int32_t* vec_off, int nlist, int uqB,
-                                 int seed_all, int sv, int svb, const int32_t* unit_off, int4* units, int max_units,
-                                 const int32_t* grp_off, int2* groups, int max_groups);
+// The batched routes' cluster-major layout: each cluster's pass-1 pairs followed by its pass-2
+// pairs in one array, and its work units and weight groups.
+struct GroupArgs {
+    const int32_t* probe_cids;  // [B, nprobe]
+    const float* probe_dqcs;
+    int B, nprobe, p_init, nlist;
+    const int32_t* counts;      // [2, nlist + 1] pairs per pass and cluster
+    const int32_t* rank;        // [B, nprobe] each pair's arrival rank in its bin
+    const int32_t* vec_off;
+    int uqB;                    // queries per lower-bound unit
+    int seed_all;               // the seeding units cover every pair of a cluster (TRIDENT_UB_SEED 2)
+    int seed_sl;                // ... and scan the first seed_sl slices of it
+    int sv, svb;                // slice lengths of the seeding and of the lower-bound units
+    int32_t* seg;               // [2, nlist + 1]: cluster c's pairs at [seg[c], seg[c + 1]), its
+                                // pass-2 pairs from seg[nlist + 1 + c]; both rows end with B nprobe
+    int32_t* unit_off;          // [2 nlist + 1] seeding units per cluster, then lower-bound units
+    int32_t* grp_off;           // [nlist + 1]
+    int32_t* pair_cid;
+    int32_t* pair_qid;
+    float* pair_dqc;            // or null
+    int4* units;
+    int max_units;
+    int2* groups;
+    int max_groups;
+    const double* qerr;         // [B, D_pad], or null (no rotation)
+    int D_pad;
+    double* qep;                // [B] sum of qerr^2
+    int nb_scatter, nb_fill;    // blocks of each role; the rest of the grid takes qep
+};
+__global__ void group_scan_kernel(GroupArgs a);
+__global__ void group_fill_kernel(GroupArgs a);
 
 __global__ void fill_u64_kernel(unsigned long long* p, unsigned long long v, int64_t n);
 
@@ -461,12 +515,8 @@ template <int KP>
 __global__ void fine_tau_kernel(BatchArgs a, int B);
 
 // Parallel rescan of overflowed candidate lists (MergeArgs, ovf_par).
-__global__ void ovf_collect_kernel(MergeArgs a);
 template <int KP, bool UB>
 __global__ void ovf_scan_kernel(MergeArgs a);
-template <int KP>
-__global__ void ovf_kth_kernel(MergeArgs a);
-
 template <int KP>
 __global__ void cm_seed_kernel(BatchArgs a, int B);
 
@@ -511,10 +561,8 @@ __global__ void cm_scan_wide_kernel(BatchArgs a);
 template <int KS>
 __global__ void pair_prep_kernel(BatchArgs a);
 
-// Waves [0, ncl) fill the per-cluster bounds, waves [ncl, ncl + B) the per-query state; block
-// 0 clears unit_ctr when given.
-__global__ void aux_bounds_kernel(BatchArgs a, int ncl, int B, double* cbound, double* qep,
-                                  int32_t* unit_ctr);
+// The per-cluster bounds, one wave per cluster.
+__global__ void cluster_bounds_kernel(BatchArgs a, int ncl, double* cbound);
 
 __global__ void sq8_bounds_kernel(ScanArgs a, const int32_t* __restrict__ qids,
                                   const int32_t* __restrict__ cids,

@@ -544,22 +544,8 @@ __device__ __forceinline__ void ovf_bounded_pass(const MergeArgs& a, int q, Wave
 // entries of that probe's cluster: every member of the query's top-K over all probed rows is
 // among its own cluster's K best, so merging the per-probe lists gives the same result as one
 // list over every probed row (the serial rescan).
-__global__ void ovf_collect_kernel(MergeArgs a) {
-    const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (q >= a.B) return;
-    int slot = -1;
-    if (a.cand_cnt[q] > a.cap) {
-        const int s = atomicAdd(a.ovf_n, 1);
-        if (s < a.ovf_max) {
-            slot = s;
-            a.ovf_q[s] = q;
-        }
-    }
-    a.ovf_slot[q] = slot;
-}
-
 // One wave per (slot, probe) item, grid-strided (the grid is sized for the slots, items past the
-// taken slots end the loop at once): UB lists the cluster's K smallest upper bounds, else its K
+// taken slots end the loop at once).  UB lists the cluster's K smallest upper bounds, else its K
 // best refined rows among those whose lower bound is within the slot's threshold.
 template <int KP, bool UB>
 __global__ __launch_bounds__(256) void ovf_scan_kernel(MergeArgs a) {
@@ -574,30 +560,28 @@ __global__ __launch_bounds__(256) void ovf_scan_kernel(MergeArgs a) {
         L.init();
         ovf_cluster_pass<KP, UB>(a, q, p, L, UB ? 0.0 : a.ovf_t[slot], s_par);
         list_store(L, a.ovf_key + (size_t)it * KP, a.ovf_id + (size_t)it * KP);
+        if constexpr (UB) {
+            // the slot's last wave: the K-th smallest upper bound over the slot's per-probe lists
+            // (and the pass's threshold) bounds the query's K-th distance.  The fences order the
+            // lists' stores before the count and the count before their loads, across XCDs.
+            __threadfence();
+            int done = 0;
+            if ((threadIdx.x & 63) == 0) done = atomicAdd(&a.ovf_done[slot], 1);
+            if (__builtin_amdgcn_readfirstlane(done) != a.nprobe - 1) continue;
+            __threadfence();
+            const int lane = threadIdx.x & 63, total = a.nprobe * KP;
+            const uint64_t* k = a.ovf_key + (size_t)slot * total;
+            const int32_t* id = a.ovf_id + (size_t)slot * total;
+            L.init();
+            for (int e0 = 0; e0 < total; e0 += kWave) {  // total is a multiple of the wave
+                list_offer(L, a.K, k[e0 + lane], id[e0 + lane]);
+            }
+            uint64_t kk;
+            int32_t ki;
+            L.at(a.K - 1, kk, ki);
+            if (lane == 0) a.ovf_t[slot] = fmin(a.tau64[q], kk != kKeyInvalid ? dist_of(kk) : (double)INFINITY);
+        }
     }
-}
-
-// One wave per taken slot: the K-th smallest upper bound over the slot's per-probe lists (and
-// the pass's threshold) bounds the query's K-th distance.
-template <int KP>
-__global__ __launch_bounds__(256) void ovf_kth_kernel(MergeArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int slot = (int)blockIdx.x * kWavesPerBlock + (int)(threadIdx.x >> 6);
-    if (slot >= min(*a.ovf_n, a.ovf_max)) return;
-    const int q = a.ovf_q[slot];
-    const int total = a.nprobe * KP;
-    const uint64_t* k = a.ovf_key + (size_t)slot * total;
-    const int32_t* id = a.ovf_id + (size_t)slot * total;
-    WaveList<KP> L;
-    L.init();
-    for (int e0 = 0; e0 < total; e0 += kWave) {
-        const int e = e0 + lane;
-        list_offer(L, a.K, e < total ? k[e] : kKeyInvalid, e < total ? id[e] : kIdInvalid);
-    }
-    uint64_t kk;
-    int32_t ki;
-    L.at(a.K - 1, kk, ki);
-    if (lane == 0) a.ovf_t[slot] = fmin(a.tau64[q], kk != kKeyInvalid ? dist_of(kk) : (double)INFINITY);
 }
 
 template <int KP>
@@ -807,8 +791,6 @@ template __global__ void ovf_scan_kernel<64, true>(MergeArgs);
 template __global__ void ovf_scan_kernel<64, false>(MergeArgs);
 template __global__ void ovf_scan_kernel<128, true>(MergeArgs);
 template __global__ void ovf_scan_kernel<128, false>(MergeArgs);
-template __global__ void ovf_kth_kernel<64>(MergeArgs);
-template __global__ void ovf_kth_kernel<128>(MergeArgs);
 template __global__ void merge_kernel<64>(MergeArgs);
 template __global__ void merge_kernel<128>(MergeArgs);
 template __global__ void merge_kernel<256>(MergeArgs);

@@ -416,8 +416,15 @@ int dispatch_scan(const ScanArgs& a, int kind, hipStream_t st) {
 // Route of a mode-2 search.  The batched route needs the per-vector scalars, K <= 128 (a
 // seeding unit lists K <= 128 bounds per query and the merge keeps 128), D_pad <= 1024 (query weights
 // held in registers: 8 VGPRs per 64 dims) and N < 2^27 (a queued survivor packs its index within the cluster
-// into 28 bits); AUTO takes it when clusters are shared by >= 8 queries on average, where
-// the contraction is dense enough for the matrix cores.
+// into 28 bits).  AUTO takes it when clusters are shared by >= 8 queries on average, where the
+// contraction is dense enough for the matrix cores, and below that when a cluster is long: the
+// per-pair route gives a cluster to one workgroup and its two passes run one after the other, so a
+// few queries wait for the longest cluster of each (1e6 rows, nlist 1024, D = 128, K = 10: 1 query 164
+// us per-pair, 149 batched; 16: 337, 185; D = 960, 390 rows a cluster: 24 queries 1588, 618).  On
+// short clusters the batched route's four launches more cost about 10 us (50,000 rows, nlist 200: 92
+// against 104).  The line: rows x dims of an average cluster >= 80,000 (333 x 64 and 250 x 128 are
+// even or slower, 977 x 128 and 1333 x 64 faster), 200,000 past 256 dims (250 x 384 about even, 390
+// x 960 faster); one query's single neighbour stays per-pair (105 against 119 at 1333 x 64).
 int choose_route(const TridentIndexView* ix, const TridentSearchParams* sp, int B, int K,
                  int nprobe, int* route) {
     const bool ok = ix->vec_Ar && ix->sq8_cells && ix->orig_ids_sorted && K <= 128 &&
@@ -447,9 +454,13 @@ int choose_route(const TridentIndexView* ix, const TridentSearchParams* sp, int 
                             "the index view lacks sq8_packed (per-pair route) and this search "
                             "cannot take the batched route (K=%d, D_pad=%d, N=%d)",
                             K, ix->D_pad, ix->N);
-            *route = (ok && (!pair_ok || (double)B * nprobe >= 8.0 * ix->nlist))
-                         ? TRIDENT_ROUTE_BATCHED
-                         : TRIDENT_ROUTE_PAIR;
+            {
+                const double cells = (double)ix->N / ix->nlist * ix->D;
+                const bool longc = cells >= (ix->D_pad <= 256 ? 80000.0 : 200000.0) && (B > 1 || K > 1);
+                *route = ok && (!pair_ok || (double)B * nprobe >= 8.0 * ix->nlist || longc)
+                             ? TRIDENT_ROUTE_BATCHED
+                             : TRIDENT_ROUTE_PAIR;
+            }
             return TRIDENT_OK;
         default:
             return fail(TRIDENT_ERR_INVALID_ARGUMENT, "route=%d outside {0,1,2}", sp->route);
@@ -471,8 +482,12 @@ inline int seed_slice_count(int K, bool xb_host, bool fine) {
 // route reads a row once per unit (up to 64 queries of its cluster) instead of once per (query,
 // probe) pair.  It needs D_pad <= 1024 (the refine's query row in LDS) and K <= 128 (the
 // merge's lists).  AUTO takes it when clusters are shared by at least 4 queries on average
-// (16-row tiles with fewer rows leave most of each matrix instruction idle), and always for a
-// base in mapped host memory (every row read crosses PCIe, and this route reads fewer).
+// (16-row tiles with fewer rows leave most of each matrix instruction idle), always for a base in
+// mapped host memory (every row read crosses PCIe, and this route reads fewer), and, while K <= 16
+// (past that its lists take every row of the first probes, and may overflow), from 48,000 rows x dims
+// of an average cluster on: one float64 pass over a cluster takes longer than the idle lanes cost
+// (40 queries, 977 x 128: 1300 us per-pair, 400 here; 600 x 96: 311, 143; even at 250 x 128, slower at
+// 333 x 64).
 int choose_cm_route(const TridentIndexView* ix, const TridentSearchParams* sp, int B, int K,
                     int nprobe, bool xb_host, bool* cm) {
     const bool ok = ix->orig_ids_sorted && K <= 128 && ix->D_pad <= 1024 &&
@@ -491,7 +506,8 @@ int choose_cm_route(const TridentIndexView* ix, const TridentSearchParams* sp, i
             *cm = true;
             return TRIDENT_OK;
         case TRIDENT_ROUTE_AUTO:
-            *cm = ok && (xb_host || (double)B * nprobe >= 4.0 * ix->nlist);
+            *cm = ok && (xb_host || (double)B * nprobe >= 4.0 * ix->nlist ||
+                         (K <= 16 && (double)ix->N / ix->nlist * ix->D >= 48000.0));
             return TRIDENT_OK;
         default:
             return fail(TRIDENT_ERR_INVALID_ARGUMENT, "route=%d outside {0,1,2}", sp->route);
@@ -1169,6 +1185,9 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
     // caller sets it) for thresholds only, so that its other probes, scanned together, start
     // from a threshold instead of +inf
     if (cm) p_init = sp->p_init >= 0 ? std::min(sp->p_init, nprobe) : (nprobe > 1 ? 1 : 0);
+    // a single probe seeds too: without a threshold every row of it would be listed and refined
+    // (8 queries, 977 rows: 701 us)
+    if (cascade && batched && sp->p_init < 0 && p_init == 0) p_init = 1;
     const int64_t M1 = (int64_t)B * p_init, M2 = (int64_t)B * (nprobe - p_init);
     // per-pair route: the two passes' pairs in consecutive arrays; batched: one cluster-major array
     int32_t *p1c = w.pair_cids, *p1q = w.pair_qids, *p2c = w.pair_cids + M1, *p2q = w.pair_qids + M1;

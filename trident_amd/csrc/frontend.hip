@@ -781,7 +781,6 @@ __global__ __launch_bounds__(256) void front_prologue_kernel(PrologueArgs a) {
             nc[t] = 0.0;
         }
         const int nst = (D + 15) >> 4;
-#pragma unroll 2
         for (int s = wid; s < nst; s += kWavesPerBlock) {
             const int k = 16 * s + 4 * g;
             float qf[4] = {0.0f, 0.0f, 0.0f, 0.0f}, wf[NC][4];
@@ -1000,7 +999,6 @@ __global__ __launch_bounds__(256) void coarse_gemm_split3_kernel(const uint32_t*
         cp[t] = reinterpret_cast<const u4*>(cmtb) + (size_t)min(cg * TC + t, ntl - 1) * NS * 3 * kWave + lane;
         hh[t] = mid[t] = low[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-#pragma unroll 2
     for (int s = SPLITK ? wid : 0; s < NS; s += SPLITK ? kWavesPerBlock : 1) {
         bf8 q[3], c[TC][3];
 #pragma unroll

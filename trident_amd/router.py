@@ -30,7 +30,8 @@ import torch
 W0_REFERENCE_A100 = 946_811_200.0
 # Smallest stable crossover over the calibrated configs on MI355X (configs[0]: B = 32).
 W0_MI355X = 2.56e7
-# Pairs per cluster from which the cascade takes its batched route (capi.hip, choose_route).
+# Pairs per cluster from which the cascade takes its batched route whatever the clusters' length
+# (capi.hip, choose_route).
 BATCHED_PAIRS_PER_CLUSTER = 8.0
 
 MODE_CM_EXACT = 10

@@ -133,7 +133,7 @@ typedef struct TridentIndexView {
 } TridentIndexView;
 
 /* How modes 2 and 10 are executed.  Both routes are exact; they differ in speed only.  Mode 10
- * batched is the float32 matrix-core cluster-major scan: it needs K <= 128 and D_pad <= 1024
+ * batched is the matrix-core cluster-major scan: it needs K <= 128 and D_pad <= 1024
  * (AUTO takes it from 4 queries per probed cluster on average, for K <= 16 on long clusters, and
  * always for a base in mapped host memory, where it reads each probed row once per unit instead of
  * once per pair). */
@@ -142,7 +142,7 @@ enum TridentRoute {
     TRIDENT_ROUTE_PAIR = 1,     /* one workgroup per (cluster, query): Stage X / Y / Z per pair
                                    (mode 10: the float64 scan of every row) */
     TRIDENT_ROUTE_BATCHED = 2   /* one workgroup per (cluster, query block): int8 matrix-core bound
-                                   (mode 10: float32 matrix-core distances with an error band) */
+                                   (mode 10: matrix-core distances with an error band) */
 };
 
 typedef struct TridentSearchParams {

@@ -530,7 +530,7 @@ unsigned cm_grid() {
         if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             cu < 1)
             cu = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, cm_kernel_ptr<D4>(), kBlock, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, cm_kernel_ptr<D4>(), kCmThreads, 0) !=
                 hipSuccess ||
             per_cu < 1)
             per_cu = 2;
@@ -567,7 +567,7 @@ int launch_cm(const BatchArgs& b, hipStream_t st) {
         return check_launch("cm_scan_wide_kernel");
     } else {
         if (b.D_pad != 4 * D4) return launch_cm<D4 + 8>(b, st);
-        cm_scan_kernel<D4><<<cm_grid<D4>(), kBlock, 0, st>>>(b);
+        cm_scan_kernel<D4><<<cm_grid<D4>(), kCmThreads, 0, st>>>(b);
         return check_launch("cm_scan_kernel");
     }
 }
@@ -1196,7 +1196,7 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
     const int seed_all = cascade && sp->ub_seed == 2 ? 1 : 0;
     const bool fine = ix->fine_codes && ix->fine_qp && xb_host;
     if (cm) {
-        rc = group_units(ix, w, B, nprobe, p_init, kUnitQWide, 0, seed_slice_count(K, false, false), kSplitVec,
+        rc = group_units(ix, w, B, nprobe, p_init, cm_unit_q(ix->D_pad), 0, seed_slice_count(K, false, false), kSplitVec,
                          kSplitVec, false, false, st);
     } else if (batched) {
         const int split_vec = ix->D_pad <= 256 ? kSplitVecNarrow : kSplitVec;
@@ -1271,7 +1271,6 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         b.seg = w.seg_off;
         b.M = (int)(M1 + M2);
         b.nlist = ix->nlist;
-        b.unit_q = kUnitQWide;
         b.ub_cnt = w.ub_cnt;
         b.ub_best = w.ub_best;
         b.seed_cnt = w.seed_cnt;

@@ -548,7 +548,13 @@ __global__ void lb_scan_wide_kernel(BatchArgs a);  // 4 < KS <= 16
 template <bool HOST, int DQ>
 __global__ void refine_survivors_kernel(BatchArgs a, int B);
 
-// Mode 10 on the float32 matrix cores (D_pad = 4 D4 <= 256, K <= 128): the lower-bound units of
+// Mode 10's matrix-core scan up to 256 dims: eight waves a workgroup, 16 queries of the unit each
+// (the wide kernel: four waves, 64 queries).
+constexpr int kCmThreads = 512;
+constexpr int kCmUnitQ = 128;
+inline int cm_unit_q(int D_pad) { return D_pad <= 256 ? kCmUnitQ : kUnitQWide; }
+
+// Mode 10 on the matrix cores (D_pad = 4 D4 <= 256, K <= 128): the lower-bound units of
 // one launch (unit_beg / unit_end), each listing (lb, ub) keys of the rows that can still enter
 // the top-K; a.ctr[0] is the work counter (zero at launch), a.ub_best the per-query thresholds
 // (+inf at launch).

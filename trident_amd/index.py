@@ -804,7 +804,7 @@ class TridentV4Index:
 
     def route_for(self, B: int, nprobe: int, k: Optional[int] = None, route: int = 0, mode: int = 2) -> int:
         """The route (_lib.ROUTE_PAIR / ROUTE_BATCHED) a search of B queries takes (mode 2, or
-        mode 10 whose batched route is the float32 matrix-core scan)."""
+        mode 10 whose batched route is the matrix-core scan)."""
         view = self.view()
         r = _lib.lib().trident_route_for_mode(ctypes.byref(view), int(mode), int(B), int(k or self.k),
                                               int(nprobe), int(route))

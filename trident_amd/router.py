@@ -10,14 +10,14 @@ measured work, which ignores an isolated win at a tiny batch.
 
 W0 is hardware-specific.  The reference's A100 value is 946,811,200 (README rounds it to
 9.0e8).  On MI355X (calibrate_w0, bench.py --calibrate-w0; mode 10 timed on its faster route,
-the float32 matrix cores at every calibrated batch) the stable crossovers are W = 2.56e7 at
+the matrix cores at every calibrated batch) the stable crossovers are W = 2.56e7 at
 configs[0] (B = 32), 6.4e7 at configs[1] (B = 8), 7.68e9 at configs[2] (D = 960, B = 128) and
 7.68e9 at configs[3] (B = 512).  W0_MI355X is the smallest, as the reference takes the smaller
 of its datasets' crossovers.
 
 No single W0 fits all four: the crossing follows the pairs per probed cluster, not W.  From
 B * nprobe = 8 nlist on, the cascade runs its batched int8 matrix-core route and wins by 4-10x;
-below that it runs per (query, cluster) pair and mode 10's single float32 matrix-core pass is
+below that it runs per (query, cluster) pair and mode 10's single matrix-core pass is
 faster or within 10 % (except single queries).  ``choose_mode_pairs`` routes by that (the
 library's own AUTO threshold for the cascade's batched route), and ``CostRouter`` uses it unless
 it is given a W0.
@@ -77,7 +77,7 @@ def calibrate_w0(index, xq_pool: torch.Tensor, nprobe: int,
             break
         q = xq_pool[:b].contiguous()
         w = work_measure(b, nprobe, N, nlist, D)
-        # mode 10 on each of its routes (1: float64 per pair, 2: float32 matrix cores), the
+        # mode 10 on each of its routes (1: float64 per pair, 2: matrix cores), the
         # faster of them standing for mode 10
         ms_routes = {}
         for rt in (1, 2):

@@ -643,10 +643,45 @@ __global__ __launch_bounds__(256) void cluster_bounds_kernel(BatchArgs a, int nc
     }
 }
 
-// One weight group per wave (its <= 32 pairs share a cluster), 2 lanes per pair: lane l =
-// lane % 2 of pair slot lane / 2 owns dims 64 k + 32 l + [0, 32) of every 64-dim step k
-// (16-byte loads, two 16-byte stores per plane and step), so the group's scale is a wave
-// reduction (no LDS, no barrier) and the per-pair sums take one shuffle.  The queries' int8
+// Sum over the 16 lanes of a row, in every lane.
+__device__ __forceinline__ float row_sum(float v) {
+    constexpr int kRowRor = 0x120;  // DPP: rotate within the 16-lane row
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kRowRor + 8, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kRowRor + 4, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kRowRor + 2, 0xf, 0xf, false));
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kRowRor + 1, 0xf, 0xf, false));
+}
+__device__ __forceinline__ int row_sum(int v) {
+    constexpr int kRowRor = 0x120;
+    v += __builtin_amdgcn_update_dpp(0, v, kRowRor + 8, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowRor + 4, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowRor + 2, 0xf, 0xf, false);
+    return v + __builtin_amdgcn_update_dpp(0, v, kRowRor + 1, 0xf, 0xf, false);
+}
+
+// The threshold-independent terms of pair (q, c) in float64 from its record (a record is 32 bytes, the
+// terms 80, and each pass that takes them holds a pair per lane).
+__device__ __forceinline__ PairTerms pair_terms(const BatchArgs& a, const PairRec& r, int q, int c) {
+    const double D_pad = (double)a.D_pad, s = (double)r.s, up = 1.0 + a.sum_rel, l1 = (double)r.wl1 * up;
+    PairTerms t;
+    t.Qp = (double)r.Qp;  // sum_rel margins where it is used
+    t.err_q = 255.0 * (0.5 * D_pad * s + 0x1p-22 * l1);
+    // the query is the float32 rotation q32: |q32 - q_exact| <= e_q(float64) + 2^-23 |q32|
+    t.e_q = sqrt(a.qep[q]) * (1.0 + 1e-12) + 0x1p-23 * sqrt((double)r.qq) * up + 1e-30;
+    t.cW = 128.0 * (double)r.wsum;
+    t.c1 = 2.0 * s;
+    t.a_max = a.cbound[kCbStride * c];
+    t.r_max = a.cbound[kCbStride * c + 1];
+    t.acc_max = 128.0 * (l1 * (1.0 / s) + 0.5 * D_pad);  // 1 / s is exact
+    t.lo_max = 128.0 * (double)r.lsum;                   // <= 128 * 128 * D_pad <= 2^24
+    t.lo_l2 = sqrt((double)r.lsq) * (1.0 + 0x1p-50);     // lsq is exact; sqrt within half an ulp
+    return t;
+}
+
+// One weight group (its <= 32 pairs share a cluster) per wave up to 256 dims, per workgroup past
+// them, whose waves take every fourth 64-dim step.  Sixteen lanes hold a pair's step, so every load
+// and store is a run of 256 (weights 64) contiguous bytes, the grid's values are loaded once for
+// all of the group's pairs, and four pairs are in work at a time.  The queries' int8
 // weight planes against the cluster's SQ8 grid and each pair's threshold-independent scalars,
 // all in float32 on the float32 rotated query q32 (the bounds take q32 as the query point: e_q
 // grows by |q32 - q64| <= 2^-24 |q32| per dimension):
@@ -654,83 +689,114 @@ __global__ __launch_bounds__(256) void cluster_bounds_kernel(BatchArgs a, int nc
 //   scale for the group: s = 2^(ilogb(m) - 14), doubled if m / s > 32639, for m = the largest
 //   |w_d| of the group's pairs, so |w_int| <= 32639;  w_int = rint(w / s) = 256 hi + lo
 //   (hi, lo in [-128, 127]);  Q = sum (q32_d - vmin_d)^2 (relative error < 2^-15).
+// w / s + 1.5 2^23 rounds to an integer (w / s is exact, a power of two), and its low 16 bits are
+// w_int's: one fma a dimension; the planes and the sums over them then work on packed bytes.
 // The quantisation error is charged by its bound, |w - s w_int| <= s / 2 per dimension:
 //   err_q = 255 (D_pad s / 2 + 2^-22 sum |w|),  and |w_int| <= |w| / s + 1 / 2 gives
 //   acc_max = 128 (sum |w| / s + D_pad / 2) >= |sum (c - 128) w_int|
 // (per-dimension sums of the exact residuals would tighten err_q by ~2x, a 2^-16-relative
 // change of the bounds, for four more instructions per dimension).
+// Measured (us): 1.28e6 pairs of 128 dims 224 -> 141 (580 MB moved, 80 of instruction issue), 320,000
+// pairs 110 -> 73, 48,000 of 960 dims 122 -> 50, 768 of 960 dims (24 queries) 53 -> 10.  The earlier
+// layout gave a pair two lanes, so a load touched 64 separate lines and rows were fetched again as L1
+// turned over.  Two waves of 16 pairs a group were slower (209, 106): the group's fixed part doubles.
 // (A common scale lets the lower-bound scan compare a wave's 32 queries against one integer
 // threshold per vector.)  Plane bytes past D_pad (up to DP) are zero, so the scan may read
 // whole 64-dim steps.
 template <int KS>
 __global__ __launch_bounds__(256) void pair_prep_kernel(BatchArgs a) {
-    const int lane = threadIdx.x & 63, l = lane & 1, slot = lane >> 1;
-    const int gi = blockIdx.x * kWavesPerBlock + (int)(threadIdx.x >> 6);
-    if (gi >= min(a.grp_off[a.nlist], a.max_groups)) return;
+    constexpr int WPG = pair_prep_waves(KS);                // waves of a group
+    constexpr int V = KS == 2 || KS == 4 ? 2 : 1;           // 64-dim steps taken together
+    constexpr int NS = (KS / V + WPG - 1) / WPG;            // the wave's steps
+    constexpr int E = 4 * V;                                // dims of a lane's step
+    constexpr int NP = kGroupQ / 4;                         // passes of four pairs
+    static_assert(kGroupQ == 32, "eight passes of four pairs, lanes j < 8 keep their sums");
+    constexpr int CH = 4;                                   // passes whose loads are in flight together
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    const int lane = threadIdx.x & 63, j = lane & 15, r = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg = WPG > 1 ? wid : 0;  // this wave's place in its group
+    const int gi = WPG > 1 ? (int)blockIdx.x : (int)blockIdx.x * kWavesPerBlock + wid;
+    if (gi >= min(a.grp_off[a.nlist], a.max_groups)) return;  // whole groups (WPG > 1: whole blocks)
     const int2 grp = a.groups[gi];
-    const bool valid = slot < grp.y;
-    const int pp = grp.x + (valid ? slot : 0);  // idle slots redo the first pair, store nothing
-    const int c = a.pair_cid[pp], q = a.pair_qid[pp];
+    const int cnt = grp.y;
+    const int my_q = a.pair_qid[grp.x + min(lane & 31, cnt - 1)];
+    const int c = a.pair_cid[grp.x];
     const int D_pad = a.D_pad, DP = a.DP;
     const size_t off = a.per_cluster ? (size_t)c * D_pad : 0;
-    const float* xr = a.xrot32 + (size_t)q * D_pad;
-    // Up to 128 dims the weights stay in registers between the group scale and the
-    // quantisation; wider, the second loop recomputes them (the same operations, so the same
-    // values).
-    constexpr bool KEEP = KS <= 2;
-    float w[KEEP ? KS : 1][32];
-    float mx = 0.0f, Qp = 0.0f, qq = 0.0f, wl1 = 0.0f;
-    auto weights = [&](int k, float (&wk)[32], auto sums_c) {
-        constexpr bool SUMS = decltype(sums_c)::value;
+    auto dim0 = [&](int s) { return (s * WPG + wg) * 64 * V + E * j; };
+    float w[NP][NS * E];
+    float mx = 0.0f, l1g = 0.0f, Qp = 0.0f, qq = 0.0f, wl1 = 0.0f;  // sums: of the pair of slot 4 j + r
+    float vm[NS * E], dl[NS * E];
 #pragma unroll
-        for (int h2 = 0; h2 < 2; ++h2) {
-            const int d0 = 64 * k + 32 * l + 16 * h2;  // D_pad is a multiple of 32: all 16 or none
+    for (int s = 0; s < NS; ++s)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) wk[16 * h2 + e] = 0.0f;
-            if (d0 < D_pad) {
-#pragma unroll
-                for (int h = 0; h < 4; ++h) {
-                    const float4 x4 = *reinterpret_cast<const float4*>(xr + d0 + 4 * h);
-                    const float4 v4 = *reinterpret_cast<const float4*>(a.vmin + off + d0 + 4 * h);
-                    const float4 g4 = *reinterpret_cast<const float4*>(a.delta + off + d0 + 4 * h);
-                    const float xv[4] = {x4.x, x4.y, x4.z, x4.w}, vv[4] = {v4.x, v4.y, v4.z, v4.w},
-                                gv[4] = {g4.x, g4.y, g4.z, g4.w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float qp = xv[e] - vv[e];
-                        wk[16 * h2 + 4 * h + e] = gv[e] * qp;
-                        if constexpr (SUMS) {
-                            mx = fmaxf(mx, fabsf(wk[16 * h2 + 4 * h + e]));
-                            wl1 += fabsf(wk[16 * h2 + 4 * h + e]);
-                            Qp = fmaf(qp, qp, Qp);
-                            qq = fmaf(xv[e], xv[e], qq);
-                        }
-                    }
-                }
-            }
+        for (int v = 0; v < V; ++v) {
+            const int d = dim0(s) + 4 * v;  // D_pad is a multiple of 32: all four or none
+            const bool in = d < D_pad;
+            const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const float4 v4 = in ? *reinterpret_cast<const float4*>(a.vmin + off + d) : z;
+            const float4 g4 = in ? *reinterpret_cast<const float4*>(a.delta + off + d) : z;
+            vm[s * E + 4 * v] = v4.x, vm[s * E + 4 * v + 1] = v4.y, vm[s * E + 4 * v + 2] = v4.z, vm[s * E + 4 * v + 3] = v4.w;
+            dl[s * E + 4 * v] = g4.x, dl[s * E + 4 * v + 1] = g4.y, dl[s * E + 4 * v + 2] = g4.z, dl[s * E + 4 * v + 3] = g4.w;
         }
-    };
-    if constexpr (KEEP) {
 #pragma unroll
-        for (int k = 0; k < KS; ++k) weights(k, w[k], std::true_type{});
-    } else {
-        // rolled loops: unrolled, the compiler would keep every step's weights live into the
-        // second loop instead of recomputing them
-#pragma unroll 1
-        for (int k = 0; k < KS; ++k) {
-            float wk[32];
-            weights(k, wk, std::true_type{});
+    for (int p0 = 0; p0 < NP; p0 += CH) {
+        if (4 * p0 >= cnt) break;
+#pragma unroll
+        for (int p = p0; p < p0 + CH; ++p) {  // idle slots redo the last pair, store nothing
+            const float* xr = a.xrot32 + (size_t)__shfl(my_q, min(4 * p + r, cnt - 1), kWave) * D_pad;
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    const int d = dim0(s) + 4 * v;
+                    const float4 x4 = d < D_pad ? *reinterpret_cast<const float4*>(xr + d)
+                                                : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    float* o = &w[p][s * E + 4 * v];
+                    o[0] = x4.x, o[1] = x4.y, o[2] = x4.z, o[3] = x4.w;
+                }
+        }
+#pragma unroll
+        for (int p = p0; p < p0 + CH; ++p) {
+            float sQ = 0.0f, sq = 0.0f, sl = 0.0f;
+#pragma unroll
+            for (int e = 0; e < NS * E; ++e) {
+                const float x = w[p][e], qp = x - vm[e];
+                const float we = dl[e] * qp;
+                w[p][e] = we;
+                mx = fmaxf(mx, fabsf(we));
+                sl += fabsf(we);
+                sQ = fmaf(qp, qp, sQ);
+                sq = fmaf(x, x, sq);
+            }
+            sQ = row_sum(sQ), sq = row_sum(sq), sl = row_sum(sl);
+            if (j == p) Qp = sQ, qq = sq, wl1 = sl;
         }
     }
+    // lanes j < 8 hold the slots (4 j + r); the others zeros
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));  // the group
-    // the pair's two lanes
-    Qp += __shfl_xor(Qp, 1, kWave);
-    qq += __shfl_xor(qq, 1, kWave);
-    wl1 += __shfl_xor(wl1, 1, kWave);
-    float l1g = wl1;  // the group's largest sum |w|
+    for (int o = 1; o < kWave; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
+    __shared__ float s_part[WPG > 1 ? WPG : 1][4][kWave];
+    __shared__ int s_sum[WPG > 1 ? WPG : 1][3][kWave];
+    if constexpr (WPG > 1) {
+        s_part[wid][0][lane] = mx;
+        s_part[wid][1][lane] = Qp;
+        s_part[wid][2][lane] = qq;
+        s_part[wid][3][lane] = wl1;
+        __syncthreads();
+        Qp = qq = wl1 = 0.0f;
 #pragma unroll
-    for (int o = 2; o < kWave; o <<= 1) l1g = fmaxf(l1g, __shfl_xor(l1g, o, kWave));
+        for (int u = 0; u < WPG; ++u) {
+            mx = fmaxf(mx, s_part[u][0][lane]);
+            Qp += s_part[u][1][lane];
+            qq += s_part[u][2][lane];
+            wl1 += s_part[u][3][lane];
+        }
+    }
+    l1g = wl1;  // the group's largest sum |w|
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) l1g = fmaxf(l1g, __shfl_xor(l1g, o, kWave));
     // s and 1/s are powers of two in [2^-114, 2^114], so w * (1/s) is exactly w / s and
     // s * wi is exact.  Two limits: |w_int| <= 32639 (the hi / lo split), and, for every pair,
     // sum |w_int| <= sum |w| / s + D_pad / 2 <= 2^23 - 1, so that |acc| <= 128 sum |w_int| <
@@ -746,64 +812,66 @@ __global__ __launch_bounds__(256) void pair_prep_kernel(BatchArgs a) {
     }
     const float s = ldexpf(1.0f, es), inv_s = ldexpf(1.0f, -es);
     int wsum = 0, lsum = 0, lsq = 0;  // sum w_int, sum |lo|, sum lo^2 (<= 2^14 DP)
-    int8_t* hi_p = a.pw + (size_t)pp * 2 * DP;
-#pragma unroll KEEP ? KS : 1
-    for (int k = 0; k < KS; ++k) {
-        float wre[32];
-        if constexpr (!KEEP) weights(k, wre, std::false_type{});
-        const float(&wk)[32] = KEEP ? w[KEEP ? k : 0] : wre;
+    int8_t* planes = a.pw + (size_t)grp.x * 2 * DP;
 #pragma unroll
-        for (int h2 = 0; h2 < 2; ++h2) {
-            uint32_t hw[4], lw[4];
+    for (int p = 0; p < NP; ++p) {
+        if (4 * p >= cnt) break;
+        const int slot = 4 * p + r;
+        int hsum = 0, lo1 = 0, sl = 0, sl2 = 0;
 #pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                int wi[4];
+        for (int st = 0; st < NS; ++st) {
+            uint32_t hw[V], lw[V];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    wi[e] = (int)rintf(wk[16 * h2 + 4 * h + e] * inv_s);  // 0 for dims >= D_pad
-                    wsum += wi[e];
-                    const int lo = (int)(int8_t)(wi[e] & 0xff);
-                    lsum += abs(lo);
-                    lsq += lo * lo;
-                }
-                // lo = the low byte of wi as int8, hi = (wi - lo) / 256 = the second byte of
-                // wi + 128
-                lw[h] = ((uint32_t)wi[0] & 0xffu) | (((uint32_t)wi[1] & 0xffu) << 8) |
-                        (((uint32_t)wi[2] & 0xffu) << 16) | ((uint32_t)wi[3] << 24);
-                hw[h] = (((uint32_t)(wi[0] + 128) >> 8) & 0xffu) |
-                        ((uint32_t)(wi[1] + 128) & 0xff00u) |
-                        ((((uint32_t)(wi[2] + 128) >> 8) & 0xffu) << 16) |
-                        ((uint32_t)(wi[3] + 128) >> 8 << 24);
+            for (int v = 0; v < V; ++v) {
+                uint32_t b[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    b[e] = __float_as_uint(fmaf(w[p][st * E + 4 * v + e], inv_s, 12582912.0f));
+                const uint32_t w01 = __builtin_amdgcn_perm(b[1], b[0], 0x05040100u);
+                const uint32_t w23 = __builtin_amdgcn_perm(b[3], b[2], 0x05040100u);
+                // lo = the low byte of wi as int8, hi = (wi - lo) / 256 = the second byte of wi + 128
+                const u16x2 half = {128, 128};
+                const uint32_t h01 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, w01) + half);
+                const uint32_t h23 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, w23) + half);
+                lw[v] = __builtin_amdgcn_perm(w23, w01, 0x06040200u);
+                hw[v] = __builtin_amdgcn_perm(h23, h01, 0x07050301u);
+                hsum = __builtin_amdgcn_sdot4((int)hw[v], 0x01010101, hsum, false);
+                lo1 = __builtin_amdgcn_sdot4((int)lw[v], 0x01010101, lo1, false);
+                sl = (int)__builtin_amdgcn_sad_u8(lw[v] ^ 0x80808080u, 0x80808080u, (uint32_t)sl);
+                sl2 = __builtin_amdgcn_sdot4((int)lw[v], (int)lw[v], sl2, false);
             }
-            if (valid) {
-                const int b = 64 * k + 32 * l + 16 * h2;
-                *reinterpret_cast<uint4*>(hi_p + b) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-                *reinterpret_cast<uint4*>(hi_p + DP + b) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+            const int d = dim0(st);
+            if (slot < cnt && d < DP) {
+                int8_t* hp = planes + (size_t)slot * 2 * DP + d;
+                if constexpr (V == 2) {
+                    *reinterpret_cast<uint2*>(hp) = make_uint2(hw[0], hw[V - 1]);
+                    *reinterpret_cast<uint2*>(hp + DP) = make_uint2(lw[0], lw[V - 1]);
+                } else {
+                    *reinterpret_cast<uint32_t*>(hp) = hw[0];
+                    *reinterpret_cast<uint32_t*>(hp + DP) = lw[0];
+                }
             }
         }
+        const int ws = row_sum(256 * hsum + lo1);
+        sl = row_sum(sl), sl2 = row_sum(sl2);
+        if (j == p) wsum = ws, lsum = sl, lsq = sl2;
     }
-    wsum += __shfl_xor(wsum, 1, kWave);
-    lsum += __shfl_xor(lsum, 1, kWave);
-    lsq += __shfl_xor(lsq, 1, kWave);
-    if (valid && l == 0) {
-        PairRec r;
-        r.Qp = (double)Qp;
-        // float32 sums of D_pad non-negative terms: relative error < sum_rel (the
-        // (1 + sum_rel) factors here and the sum_rel margins on Qp where it is used)
-        const double l1 = (double)wl1 * (1.0 + a.sum_rel);
-        r.err_q = 255.0 * (0.5 * (double)D_pad * (double)s + 0x1p-22 * l1);
-        // the query is the float32 rotation q32: |q32 - q_exact| <= e_q(float64) + 2^-23 |q32|
-        r.e_q = sqrt(a.qep[q]) * (1.0 + 1e-12) + 0x1p-23 * sqrt((double)qq) * (1.0 + a.sum_rel) +
-                1e-30;
-        r.cW = 128.0 * (double)wsum;
-        r.c1 = 2.0 * (double)s;
-        r.a_max = a.cbound[kCbStride * c];
-        r.r_max = a.cbound[kCbStride * c + 1];
-        r.acc_max = 128.0 * (l1 * (double)inv_s + 0.5 * (double)D_pad);
-        r.lo_max = 128.0 * (double)lsum;  // <= 128 * 128 * D_pad <= 2^24
-        r.lo_l2 = sqrt((double)lsq) * (1.0 + 0x1p-50);  // lsq is exact; sqrt within half an ulp
-        a.prec[pp] = r;
+    if constexpr (WPG > 1) {
+        s_sum[wid][0][lane] = wsum;
+        s_sum[wid][1][lane] = lsum;
+        s_sum[wid][2][lane] = lsq;
+        __syncthreads();
+        if (wid > 0) return;
+#pragma unroll
+        for (int u = 1; u < WPG; ++u) {
+            wsum += s_sum[u][0][lane];
+            lsum += s_sum[u][1][lane];
+            lsq += s_sum[u][2][lane];
+        }
     }
+    const int slot = 4 * j + r;
+    if (j < NP && slot < cnt)
+        a.prec[grp.x + slot] = PairRec{Qp, wl1, qq, s, wsum, lsum, lsq, 0};
 }
 
 template __global__ void pair_prep_kernel<1>(BatchArgs);
@@ -1086,7 +1154,7 @@ __global__ __launch_bounds__(256) void ub_scan_kernel(BatchArgs a) {
                 }
             }
             if (hasq) {
-                const PairRec pr = a.prec[pj];
+                const PairTerms pr = pair_terms(a, a.prec[pj], q, cid);
                 const double AQ = (pr.Qp * (1.0 + a.sum_rel) + 1e-30 + 2.0 * pr.err_q) * (1.0 + 1e-13);
                 const double C = AQ - pr.c1 * pr.cW;
                 const double slack =
@@ -1628,7 +1696,7 @@ __global__ __launch_bounds__(256) void lb_prep_kernel(BatchArgs a) {
     const bool valid = slot < grp.y;
     const int p = grp.x + (valid ? slot : 0);
     const int q = a.pair_qid[p], c = a.pair_cid[p];
-    const PairRec pr = a.prec[p];
+    const PairTerms pr = pair_terms(a, a.prec[p], q, c);
     const double Qp = pr.Qp, err_q = pr.err_q, cW = pr.cW, c1 = pr.c1;
     const double tq = sqrt(a.tau[q] * a.rot_sq_max) * (1.0 + 1e-12) + pr.e_q;
     const bool thr = tq < 1e30;

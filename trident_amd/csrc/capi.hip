@@ -643,11 +643,11 @@ bool with_ks(int ks, F&& f) {
 
 int launch_pair_prep(const BatchArgs& b, hipStream_t st) {
     if (b.M <= 0) return TRIDENT_OK;
-    static_assert(kGroupQ * 2 == kWave, "one weight group per wave, 2 lanes a pair");
-    // one group per wave; waves past the group count return
-    const unsigned grid = (unsigned)((b.max_groups + kWavesPerBlock - 1) / kWavesPerBlock);
+    // groups past the device's count return
     const bool ok = with_ks(b.DP / 64, [&](auto ks_c) {
-        pair_prep_kernel<decltype(ks_c)::value><<<grid, kBlock, 0, st>>>(b);
+        constexpr int KS = decltype(ks_c)::value, per_block = kWavesPerBlock / pair_prep_waves(KS);
+        const unsigned grid = (unsigned)((b.max_groups + per_block - 1) / per_block);
+        pair_prep_kernel<KS><<<grid, kBlock, 0, st>>>(b);
     });
     if (!ok) return fail(TRIDENT_ERR_UNSUPPORTED, "batched route needs D_pad <= 1024");
     return check_launch("pair_prep_kernel");

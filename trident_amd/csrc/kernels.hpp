@@ -101,6 +101,18 @@ struct MergeArgs {
 
 // Per-(query, cluster) pair scalars of the batched bound (threshold-independent part).
 struct PairRec {
+    float Qp;      // |q32 - vmin|^2: float32 sums of D_pad non-negative terms, relative error < sum_rel
+    float wl1;     // sum |w_d|, likewise
+    float qq;      // |q32|^2, likewise
+    float s;       // the group's scale, a power of two
+    int32_t wsum;  // sum w_int
+    int32_t lsum;  // sum |lo_d| <= 128 D_pad
+    int32_t lsq;   // sum lo_d^2 <= 2^14 DP
+    int32_t pad;
+};
+
+// What the passes take from it and from the pair's query and cluster (pair_terms).
+struct PairTerms {
     double Qp;       // |q_rot - vmin|^2
     double err_q;    // 255 * sum |w - s w_int|  (bound on the weight quantisation error)
     double e_q;      // >= |q_rot(float64) - q_rot(exact)|
@@ -563,6 +575,9 @@ __global__ void cm_scan_kernel(BatchArgs a);
 
 // The same for 256 < D_pad <= 1024: dims in chunks of 128, query chunks reloaded per block.
 __global__ void cm_scan_wide_kernel(BatchArgs a);
+
+// Waves that share one weight group: past 256 dims one wave's registers would not hold its weights.
+constexpr int pair_prep_waves(int KS) { return KS <= 4 ? 1 : kWavesPerBlock; }
 
 template <int KS>
 __global__ void pair_prep_kernel(BatchArgs a);

@@ -1304,6 +1304,20 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         if (K <= 64) fine_tau_kernel<64><<<qg, kBlock, 0, st>>>(b, B);
         else fine_tau_kernel<128><<<qg, kBlock, 0, st>>>(b, B);
         if ((rc = check_launch("fine_tau_kernel"))) return rc;
+        // Past K = 16 a query whose first probe holds fewer than K rows has no threshold and lists
+        // every row: such lists, when they overflow, are rescanned in parallel before the merge.  Up
+        // to 16 the scan's own thresholds keep lists short, and the launch (5 us) is saved.
+        const bool rescan = K > 16;
+        if (rescan) {
+            b.ovf_max = m.ovf_max = (int)w.ovf_max;
+            b.ovf_n = m.ovf_n = w.ovf_n;
+            b.ovf_q = m.ovf_q = w.ovf_q;
+            b.ovf_slot = m.ovf_slot = w.ovf_slot;
+            b.ovf_done = w.ovf_done;
+            m.ovf_key = w.ovf_key;
+            m.ovf_id = w.ovf_id;
+            m.ovf_par = 1;
+        }
         const dim3 rgrid(qg, (unsigned)std::min<int64_t>((cap + kWave - 1) / kWave, 16));
         if (ix->D <= 256) {
             if (xb_host) refine_survivors_kernel<true, 256><<<rgrid, kBlock, 0, st>>>(b, B);
@@ -1326,6 +1340,13 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         m.tile_off = ix->cluster_tile_off;
         m.T = ix->tile_size;
         m.D = ix->D;
+        if (rescan) {
+            constexpr int NW = kOvfExactThreads / kWave;
+            const unsigned og = (unsigned)std::min<int64_t>((w.ovf_max * nprobe + NW - 1) / NW, 4096);
+            if (KP == 64) ovf_exact_kernel<64><<<og, kOvfExactThreads, 0, st>>>(m);
+            else ovf_exact_kernel<128><<<og, kOvfExactThreads, 0, st>>>(m);
+            if ((rc = check_launch("ovf_exact_kernel"))) return rc;
+        }
         if ((rc = launch_merge(m, KP, st))) return rc;
         if ((rc = mark(TRIDENT_EV_END))) return rc;
         if (out->stats) {

@@ -83,7 +83,7 @@ struct MergeArgs {
     const double* xrot64;       // [B, D_pad]
     const double* qerr;         // [B, D_pad]
     double lb_scale, ub_scale;  // as ScanArgs
-    // Parallel bounded rescan (ovf_par = 1, with ovf_bounds): the refine gives up to ovf_max
+    // Parallel rescan (ovf_par = 1; without ovf_bounds ovf_exact_kernel reads every probed row): the refine gives up to ovf_max
     // overflowed queries a slot; ovf_scan_kernel rescans them one wave per (slot, probe), each
     // keeping its cluster's K best in ovf_key / ovf_id [ovf_max, nprobe, KP] -- upper bounds first,
     // which the slot's last wave to finish (ovf_done) reduces to the slot's threshold ovf_t, then
@@ -529,6 +529,9 @@ __global__ void fine_tau_kernel(BatchArgs a, int B);
 // Parallel rescan of overflowed candidate lists (MergeArgs, ovf_par).
 template <int KP, bool UB>
 __global__ void ovf_scan_kernel(MergeArgs a);
+constexpr int kOvfExactThreads = 128;
+template <int KP>
+__global__ void ovf_exact_kernel(MergeArgs a);
 template <int KP>
 __global__ void cm_seed_kernel(BatchArgs a, int B);
 

@@ -584,6 +584,44 @@ __global__ __launch_bounds__(256) void ovf_scan_kernel(MergeArgs a) {
     }
 }
 
+// The same without bounds (mode 10's matrix-core scan, D <= 1024): one wave per (slot, probe) reads
+// the cluster's rows whole, 64 at a time (refine_rows), and keeps its K best; the largest cluster's
+// wave bounds it.  Rescanned by the merge, one wave took 93 ms for one query's 40 probes while every
+// other query waited.  K = 100: 200 queries at D = 960 95.0 -> 7.2 ms, 1000 at D = 128 18.3 -> 1.8;
+// K = 20, D = 960 101 -> 7.1; where no list overflows the launch costs 5 us (297 -> 304).  Two waves a
+// block: 33 KB of LDS.
+template <int KP>
+__global__ __launch_bounds__(kOvfExactThreads) void ovf_exact_kernel(MergeArgs a) {
+    constexpr int NW = kOvfExactThreads / kWave;
+    __shared__ double s_q64[NW][1024];
+    __shared__ float s_stage[NW][kStageCh][kWave + 1];
+    __shared__ int32_t s_pos[NW][kWave];
+    const int lane = threadIdx.x & 63, wid = (int)(threadIdx.x >> 6);
+    const int total = __builtin_amdgcn_readfirstlane(min(*a.ovf_n, a.ovf_max)) * a.nprobe;
+    for (int it = (int)blockIdx.x * NW + wid; it < total; it += (int)gridDim.x * NW) {
+        const int slot = it / a.nprobe, p = it - slot * a.nprobe;
+        const int q = __builtin_amdgcn_readfirstlane(a.ovf_q[slot]);
+        const int c = __builtin_amdgcn_readfirstlane(a.probe_cids[(size_t)q * a.nprobe + p]);
+        const int v0 = a.vec_off[c], n = a.vec_off[c + 1] - v0;
+        const int32_t* oids = a.tile_oids + (size_t)a.tile_off[c] * a.T;
+        wave_sync();  // the previous item's query is no longer read
+        for (int d = lane; d < a.D; d += kWave) s_q64[wid][d] = a.xq64[(size_t)q * a.D + d];
+        if (a.host_rows && lane == 0) atomicAdd(a.host_rows, (unsigned long long)max(n, 0));
+        WaveList<KP> L;
+        L.init();
+        for (int b0 = 0; b0 < n; b0 += kWave) {
+            const int m = min(kWave, n - b0);
+            wave_sync();
+            s_pos[wid][lane] = v0 + b0 + min(lane, m - 1);
+            wave_sync();
+            const double d64 = refine_rows(a.xb, nullptr, a.D, s_pos[wid], m, s_stage[wid], s_q64[wid]);
+            const bool in = lane < m;
+            list_offer(L, a.K, in ? key_of(d64) : kKeyInvalid, in ? oids[b0 + lane] : kIdInvalid);
+        }
+        list_store(L, a.ovf_key + (size_t)it * KP, a.ovf_id + (size_t)it * KP);
+    }
+}
+
 template <int KP>
 __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
     extern __shared__ float s_ovf[];  // ovf_bounds: 3 D_pad floats per wave
@@ -791,6 +829,8 @@ template __global__ void ovf_scan_kernel<64, true>(MergeArgs);
 template __global__ void ovf_scan_kernel<64, false>(MergeArgs);
 template __global__ void ovf_scan_kernel<128, true>(MergeArgs);
 template __global__ void ovf_scan_kernel<128, false>(MergeArgs);
+template __global__ void ovf_exact_kernel<64>(MergeArgs);
+template __global__ void ovf_exact_kernel<128>(MergeArgs);
 template __global__ void merge_kernel<64>(MergeArgs);
 template __global__ void merge_kernel<128>(MergeArgs);
 template __global__ void merge_kernel<256>(MergeArgs);

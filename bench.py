@@ -65,6 +65,7 @@ METRIC = "QPS at 100% exact top-10, 1×MI355X; achieved HBM GB/s vs peak"  # BAS
 HBM_PEAK_GBPS = 8000.0
 INT8_PEAK_TOPS = 5000.0  # MI355X dense int8 matrix throughput
 FP32_PEAK_TFLOPS = 157.3  # MI355X dense float32 matrix throughput
+BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bfloat16 matrix throughput
 PROFILES = os.path.join(ROOT, "profiles")
 T_START = time.perf_counter()
 
@@ -293,12 +294,16 @@ def roofline(w, stage, probes, mode, route_used):
     rows_all = int(sizes[probes].sum())
     t_scan = stage["pass2_scan_ms"] * 1e-3
     if route_used == _lib.ROUTE_BATCHED and mode == 10:
-        flops = 2.0 * rows_all * ix.D_pad  # float32 matrix cores: 2 D_pad flops per (query, row)
+        # 2 D_pad flops per (query, row); up to 256 dims six bfloat16 products each
+        flops = 2.0 * rows_all * ix.D_pad
         achieved = flops / t_scan / 1e12
-        kname = "cm_scan_kernel<D4>" if ix.D_pad <= 256 else "cm_scan_wide_kernel"
-        roof = {"bound": "mfma", "kernel": f"{kname} (mode 10, float32 matrix cores)",
-                "achieved": round(achieved, 2), "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                "frac": round(achieved / FP32_PEAK_TFLOPS, 4), "flops_alg_per_launch": flops}
+        if ix.D_pad <= 256:
+            kname, peak = "cm_scan_kernel (mode 10, six bfloat16 products)", BF16_PEAK_TFLOPS / 6
+        else:
+            kname, peak = "cm_scan_wide_kernel (mode 10, float32 matrix cores)", FP32_PEAK_TFLOPS
+        roof = {"bound": "mfma", "kernel": kname,
+                "achieved": round(achieved, 2), "peak": round(peak, 1), "unit": "TFLOP/s",
+                "frac": round(achieved / peak, 4), "flops_alg_per_launch": flops}
     elif route_used == _lib.ROUTE_BATCHED:
         ops_alg = 4 * rows_all * ix.D_pad
         achieved = ops_alg / t_scan / 1e12
@@ -568,7 +573,7 @@ def measure_sweeps(args, dev, cfg_ids):
                 v["cpu_baseline"] = cpu_baseline(w, npb, K, probes, gd, gi, cfg["cpu"])
             res[f"configs[{cid - 1}]_nprobe{npb}_K{K}"] = v
         # mode 10 (exact cluster-major scan; the reference's router sends configs[0] there) at the
-        # config's stated nprobe and K, on the library's AUTO route (float32 matrix cores here)
+        # config's stated nprobe and K, on the library's AUTO route (matrix cores here)
         npb, K = cfg["nprobe"], cfg["K"]
         v, _ = measure_variant(w, npb, K, 10, 0, 0, args.extra_steps, 5, 2, label=f"cfg{cid} mode 10")
         v["workload"] = (f"BASELINE {cfg['desc']}, N={cfg['N']}, D={cfg['D']}, nlist={cfg['nlist']}, "

@@ -479,7 +479,7 @@ inline int seed_slice_count(int K, bool xb_host, bool fine) {
 
 // Mode 10: the matrix-core cluster-major scan (cm_scan_kernel, cm_scan_wide_kernel past 256
 // dims) or the per-pair float64 scan.  Both read every probed row from the base; the matrix-core
-// route reads a row once per unit (up to 64 queries of its cluster) instead of once per (query,
+// route reads a row once per unit (up to 128 queries of its cluster) instead of once per (query,
 // probe) pair.  It needs D_pad <= 1024 (the refine's query row in LDS) and K <= 128 (the
 // merge's lists).  AUTO takes it when clusters are shared by at least 4 queries on average
 // (16-row tiles with fewer rows leave most of each matrix instruction idle), always for a base in

@@ -295,7 +295,7 @@ __device__ inline void fine_row_bounds(const BatchArgs& a, const double* q64, do
 //     d64 <= it).
 // Every row with d64 <= the old tau is listed, so every row of the exact top-K keeps
 // lb <= the new tau, and the refine reads only rows with lb <= tau.  An overflowed list
-// (count > cap) is left alone: the merge rescans that query's probes.
+// (count > cap) is left alone: that query's probes are rescanned (mode 10: it is listed here).
 __device__ __forceinline__ float fine_lb_of(uint64_t k) { return __uint_as_float((uint32_t)(k >> 32)); }
 __device__ __forceinline__ float fine_ub_of(uint64_t k) { return __uint_as_float((uint32_t)k); }
 
@@ -400,6 +400,7 @@ __global__ __launch_bounds__(256) void fine_tau_kernel(BatchArgs a, int B) {
     const int q = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + (int)(threadIdx.x >> 6));
     if (q >= B) return;
     const int cnt = a.cand_cnt[q];
+    if (cnt > a.cap && a.probe_cids && lane == 0) a.ovf_q[atomicAdd(a.ovf_n, 1)] = q;
     if (cnt <= 0 || cnt > a.cap) return;
     const float t = listed_kth_ub<KP>(a, a.cand_key + (size_t)q * a.cap, cnt);
     if (lane == 0 && t < INFINITY) a.tau[q] = fmin(a.tau[q], (double)t);
@@ -445,6 +446,111 @@ __global__ void fine_bounds_kernel(BatchArgs a, const int32_t* __restrict__ qids
     fine_row_bounds(a, a.xrot64 + (size_t)q * a.D_pad, sqrt(ep) * (1.0 + 1e-12), pos, lb[i], ub[i]);
 }
 
+// The canonical float64 distance of a row (device memory) to the query row qr staged in LDS, in
+// dimension order; vec4: both may be read 16 bytes at a time (64 dims arrive together, all 16
+// loads issued before their first use).
+__device__ __forceinline__ double row_d64(const float* __restrict__ xr, const float* qr, int D, bool vec4) {
+    double acc = 0.0;
+    if (vec4) {
+        int d = 0;
+        auto chunk = [&](auto n4c) {
+            constexpr int N4 = decltype(n4c)::value;
+            float4 xv[N4];
+#pragma unroll
+            for (int k = 0; k < N4; ++k) xv[k] = *reinterpret_cast<const float4*>(xr + d + 4 * k);
+#pragma unroll
+            for (int k = 0; k < N4; ++k) {
+                const float4 y = *reinterpret_cast<const float4*>(qr + d + 4 * k);
+                double t = (double)xv[k].x - (double)y.x;
+                acc = fma(t, t, acc);
+                t = (double)xv[k].y - (double)y.y;
+                acc = fma(t, t, acc);
+                t = (double)xv[k].z - (double)y.z;
+                acc = fma(t, t, acc);
+                t = (double)xv[k].w - (double)y.w;
+                acc = fma(t, t, acc);
+            }
+            d += 4 * N4;
+        };
+        while (d + 64 <= D) chunk(std::integral_constant<int, 16>{});
+        while (d + 4 <= D) chunk(std::integral_constant<int, 1>{});
+    } else {
+        for (int d = 0; d < D; ++d) {
+            const double t = (double)xr[d] - (double)qr[d];
+            acc = fma(t, t, acc);
+        }
+    }
+    return acc;
+}
+
+// Mode 10's overflowed lists (ovf_n queries in ovf_q), in the refine's launch, its first blocks
+// (the queries' follow): one block per (query, probe) reads the cluster's rows whole, each wave every
+// fourth run of 64, and puts the cluster's K best by (float64 distance, original id) in place of
+// the query's list, at p * rescan_stride(K).  Every member of the query's top-K is among its own
+// cluster's K best, so the merge of these entries is the exact result.  Without an overflow the
+// blocks end on reading ovf_n: a launch of their own cost each search 5 us, and one wave of the
+// merge, where a query's lists fell to it, took 55 ms for 63 clusters of 4000 rows (D = 128).
+template <bool HOST, int KP>
+__device__ __forceinline__ void rescan_lists(const BatchArgs& a, int B, float* s_q, int32_t* s_pos, double* s_q64,
+                                             float (*s_stage)[kWave + 1]) {
+    __shared__ uint64_t s_ck[kWavesPerBlock - 1][KP];
+    __shared__ int32_t s_ci[kWavesPerBlock - 1][KP];
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rb = (int)(blockIdx.x * gridDim.y + blockIdx.y);
+    const int nrb = ((int)gridDim.x - (B + kWavesPerBlock - 1) / kWavesPerBlock) * (int)gridDim.y;
+    const int D = a.D, K = a.K, S = rescan_stride(K);
+    const bool vec4 = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(a.xb) & 15) == 0;
+    const int total = __builtin_amdgcn_readfirstlane(*a.ovf_n) * a.nprobe;
+    for (int it = rb; it < total; it += nrb) {  // the same items for all four waves
+        const int o = it / a.nprobe, p = it - o * a.nprobe;
+        const int q = __builtin_amdgcn_readfirstlane(a.ovf_q[o]);
+        const int c = __builtin_amdgcn_readfirstlane(a.probe_cids[(size_t)q * a.nprobe + p]);
+        const int v0 = a.vec_off[c], n = a.vec_off[c + 1] - v0;
+        for (int d = lane; d < D; d += kWave) {
+            const float x = a.xq[(size_t)q * D + d];
+            if constexpr (HOST) s_q64[d] = (double)x;
+            else s_q[d] = x;
+        }
+        if (HOST && a.host_rows && wid == 0 && lane == 0) atomicAdd(a.host_rows, (unsigned long long)n);
+        wave_sync();
+        WaveList<KP> L;
+        L.init();
+        for (int b0 = wid * kWave; b0 < n; b0 += kBlock) {
+            const int m = min(kWave, n - b0), pos = v0 + b0 + min(lane, m - 1);
+            double d64;
+            if constexpr (HOST) {
+                s_pos[lane] = pos;
+                wave_sync();
+                d64 = refine_rows(a.xb, a.xb8, D, s_pos, m, s_stage, s_q64);
+                wave_sync();
+            } else {
+                d64 = row_d64(a.xb + (size_t)pos * D, s_q, D, vec4);
+            }
+            const bool in = lane < m;
+            list_offer(L, K, in ? key_of(d64) : kKeyInvalid, in ? a.orig_ids[pos] : kIdInvalid);
+        }
+        if (wid > 0) list_store(L, s_ck[wid - 1], s_ci[wid - 1]);
+        __syncthreads();
+        if (wid == 0) {
+#pragma unroll
+            for (int w = 0; w < kWavesPerBlock - 1; ++w) list_absorb(L, K, s_ck[w], s_ci[w]);
+            uint64_t* ck = a.cand_key + (size_t)q * a.cap + (size_t)p * S;
+            int32_t* ci = a.cand_id + (size_t)q * a.cap + (size_t)p * S;
+            for_chunks<KP>([&](auto cc) __attribute__((always_inline)) {
+                constexpr int h = decltype(cc)::value;
+                uint64_t k;
+                int32_t i;
+                list_chunk<h>(L, k, i);
+                if (h * kWave + lane < S) {
+                    ck[h * kWave + lane] = k;
+                    ci[h * kWave + lane] = i;
+                }
+            });
+        }
+        __syncthreads();  // the lists in LDS are read
+    }
+}
+
 // Exact test of the listed survivors, in place: slot s >= seed_cnt[q] of query q holds a sorted
 // position on entry and (key, original id) on exit, or (kKeyInvalid, kIdInvalid) when the
 // canonical float64 distance exceeds tau[q] or the row is one of the query's seeds (slots
@@ -452,17 +558,32 @@ __global__ void fine_bounds_kernel(BatchArgs a, const int32_t* __restrict__ qids
 // (query, 64-slot chunk of its list), one survivor per lane (a query with many survivors
 // spreads over many waves); each lane walks its own row in dimension order with 16-byte loads,
 // against the query row staged in LDS (DQ >= D floats per wave: 256, or 1024 for the wide
-// batched route).  An overflowed list (count > cap) is left alone: the merge rescans that
-// query's probes through the SQ8 bounds (merge_kernel), in a slot of the parallel rescan taken
-// here while there are any.
-template <bool HOST, int DQ>
-__global__ __launch_bounds__(256) void refine_survivors_kernel(BatchArgs a, int B) {
-    __shared__ __align__(16) float s_q[kWavesPerBlock][HOST ? 1 : DQ];  // host: float64 copy below
+// batched route).  An overflowed list (count > cap) is left alone: with KP = 0 the merge rescans
+// that query's probes through the SQ8 bounds (merge_kernel), in a slot of the parallel rescan taken
+// here while there are any; with KP > 0 (mode 10) the launch's first blocks rescan it
+// (rescan_lists).
+// (Registers for as many waves as the LDS leaves room for: the rescan would take more.)
+template <bool HOST, int DQ, int KP>
+__global__ __launch_bounds__(256, !HOST ? 4 : DQ > 256 ? 2 : 3) void refine_survivors_kernel(BatchArgs a, int B) {
+    constexpr int W = kWavesPerBlock, WH = HOST ? W : 1;
+    __shared__ __align__(16) float s_q[W][HOST ? 1 : DQ];  // device base: the query rows
+    __shared__ int32_t s_pos[WH][kWave];                   // host base: refine_rows' areas
+    __shared__ double s_q64[WH][HOST ? DQ : 1];
+    __shared__ float s_stage[WH][kStageCh][kWave + 1];
     const int lane = threadIdx.x & 63, wid = (int)(threadIdx.x >> 6);
-    const int q = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + wid);
+    int bx = (int)blockIdx.x;
+    if constexpr (KP > 0) {
+        bx -= (int)gridDim.x - (B + W - 1) / W;  // the rescan's blocks come first: idle ones end unseen
+        if (bx < 0) {
+            rescan_lists<HOST, KP>(a, B, s_q[wid], s_pos[HOST ? wid : 0], s_q64[HOST ? wid : 0],
+                                   s_stage[HOST ? wid : 0]);
+            return;
+        }
+    }
+    const int q = __builtin_amdgcn_readfirstlane(bx * W + wid);
     if (q >= B) return;
     const int cnt = a.cand_cnt[q], ns = a.seed_cnt[q];
-    if (a.ovf_max > 0 && blockIdx.y == 0 && lane == 0) {
+    if (KP == 0 && a.ovf_max > 0 && blockIdx.y == 0 && lane == 0) {
         int slot = -1;
         if (cnt > a.cap) {
             const int s = atomicAdd(a.ovf_n, 1);
@@ -498,9 +619,6 @@ __global__ __launch_bounds__(256) void refine_survivors_kernel(BatchArgs a, int 
         // base in mapped host memory: rows cross PCIe, so the wave's rows are read whole (512
         // contiguous bytes at a time, a group's loads all in flight: refine_rows) and staged
         // through LDS; seed rows are left out of the group
-        __shared__ int32_t s_pos[kWavesPerBlock][kWave];
-        __shared__ double s_q64[kWavesPerBlock][DQ];
-        __shared__ float s_stage[kWavesPerBlock][kStageCh][kWave + 1];
         for (int d = lane; d < D; d += kWave) s_q64[wid][d] = (double)a.xq[(size_t)q * D + d];
         for (int s0 = ns + (int)blockIdx.y * kWave; s0 < cnt; s0 += kWave * (int)gridDim.y) {
             const int s = s0 + lane;
@@ -539,37 +657,7 @@ __global__ __launch_bounds__(256) void refine_survivors_kernel(BatchArgs a, int 
             continue;
         }
         const float* xr = a.xb + (size_t)pos * D;
-        double acc = 0.0;
-        if (vec4) {
-            // the row arrives 64 dims at a time, all 16 loads issued before their first use
-            int d = 0;
-            auto chunk = [&](auto n4c) {
-                constexpr int N4 = decltype(n4c)::value;
-                float4 xv[N4];
-#pragma unroll
-                for (int k = 0; k < N4; ++k) xv[k] = *reinterpret_cast<const float4*>(xr + d + 4 * k);
-#pragma unroll
-                for (int k = 0; k < N4; ++k) {
-                    const float4 y = *reinterpret_cast<const float4*>(qr + d + 4 * k);
-                    double t = (double)xv[k].x - (double)y.x;
-                    acc = fma(t, t, acc);
-                    t = (double)xv[k].y - (double)y.y;
-                    acc = fma(t, t, acc);
-                    t = (double)xv[k].z - (double)y.z;
-                    acc = fma(t, t, acc);
-                    t = (double)xv[k].w - (double)y.w;
-                    acc = fma(t, t, acc);
-                }
-                d += 4 * N4;
-            };
-            while (d + 64 <= D) chunk(std::integral_constant<int, 16>{});
-            while (d + 4 <= D) chunk(std::integral_constant<int, 1>{});
-        } else {
-            for (int d = 0; d < D; ++d) {
-                const double t = (double)xr[d] - (double)qr[d];
-                acc = fma(t, t, acc);
-            }
-        }
+        const double acc = row_d64(xr, qr, D, vec4);
         const bool ok = acc <= tau;
         ck[s] = ok ? key_of(acc) : kKeyInvalid;
         ci[s] = ok ? oid : kIdInvalid;
@@ -582,10 +670,18 @@ __global__ __launch_bounds__(256) void refine_survivors_kernel(BatchArgs a, int 
     }
 }
 
-template __global__ void refine_survivors_kernel<false, 256>(BatchArgs, int);
-template __global__ void refine_survivors_kernel<true, 256>(BatchArgs, int);
-template __global__ void refine_survivors_kernel<false, 1024>(BatchArgs, int);
-template __global__ void refine_survivors_kernel<true, 1024>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<false, 256, 0>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<false, 256, 64>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<false, 256, 128>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<true, 256, 0>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<true, 256, 64>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<true, 256, 128>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<false, 1024, 0>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<false, 1024, 64>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<false, 1024, 128>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<true, 1024, 0>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<true, 1024, 64>(BatchArgs, int);
+template __global__ void refine_survivors_kernel<true, 1024, 128>(BatchArgs, int);
 
 __device__ __forceinline__ double wave_sum_f64(double v) {
 #pragma unroll

@@ -149,7 +149,7 @@ struct Workspace {
     int64_t ovf_max;
     int32_t* ovf_n;                  // [1]
     int32_t* ovf_q;                  // [ovf_max]
-    int32_t* ovf_slot;               // [B]
+    int32_t* ovf_slot;               // [B]; mode 10: its overflowed queries
     int32_t* ovf_done;               // [ovf_max]
     double* ovf_t;                   // [ovf_max]
     uint64_t* ovf_key;               // [ovf_max, nprobe, KP <= 128]
@@ -157,7 +157,8 @@ struct Workspace {
     size_t bytes;
 };
 
-// Overflowed queries rescanned in parallel per search (the rest take the merge's serial rescan):
+// Overflowed queries of a cascade rescanned in parallel per search (the rest take the merge's
+// serial rescan; mode 10 rescans every one in parallel, in its refine):
 // 188 at B = 10,000, 18.5 MB of per-probe lists at K <= 64.  A configs[4] search whose seeding
 // threshold was made loose on purpose (p_init 1) overflows fewer than that: 243 -> 17 ms per
 // step against the serial rescan; larger budgets (B / 16, B / 4) changed nothing.
@@ -660,6 +661,18 @@ int launch_batch(const BatchArgs& b, hipStream_t st) {
         rc = launch_batch_ks<UB, decltype(ks_c)::value>(b, st);
     });
     return ok ? rc : fail(TRIDENT_ERR_UNSUPPORTED, "batched route needs D_pad <= 1024");
+}
+
+// refine_survivors_kernel<host base, query row length, KP>
+template <int KP>
+void launch_refine(const BatchArgs& b, dim3 grid, hipStream_t st) {
+    if (b.D <= 256) {
+        if (b.xb_host) refine_survivors_kernel<true, 256, KP><<<grid, kBlock, 0, st>>>(b, b.B);
+        else refine_survivors_kernel<false, 256, KP><<<grid, kBlock, 0, st>>>(b, b.B);
+    } else {
+        if (b.xb_host) refine_survivors_kernel<true, 1024, KP><<<grid, kBlock, 0, st>>>(b, b.B);
+        else refine_survivors_kernel<false, 1024, KP><<<grid, kBlock, 0, st>>>(b, b.B);
+    }
 }
 
 int launch_merge(const MergeArgs& m, int KP, hipStream_t st) {
@@ -1276,6 +1289,10 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         b.seed_cnt = w.seed_cnt;
         b.qep = w.qep;
         b.fine_mode = 1;  // the candidate keys hold (lb, ub): the refine skips lb > tau
+        b.ovf_n = w.ovf_n;
+        b.ovf_q = w.ovf_slot;  // [B]
+        b.probe_cids = w.probe_cids;
+        b.nprobe = nprobe;
         const unsigned qg = (unsigned)((B + kWavesPerBlock - 1) / kWavesPerBlock);
         if (M1 > 0) {
             // warm-up over the first probes: for K <= 16 the scan's own thresholds (the K-th
@@ -1304,49 +1321,17 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         if (K <= 64) fine_tau_kernel<64><<<qg, kBlock, 0, st>>>(b, B);
         else fine_tau_kernel<128><<<qg, kBlock, 0, st>>>(b, B);
         if ((rc = check_launch("fine_tau_kernel"))) return rc;
-        // Past K = 16 a query whose first probe holds fewer than K rows has no threshold and lists
-        // every row: such lists, when they overflow, are rescanned in parallel before the merge.  Up
-        // to 16 the scan's own thresholds keep lists short, and the launch (5 us) is saved.
-        const bool rescan = K > 16;
-        if (rescan) {
-            b.ovf_max = m.ovf_max = (int)w.ovf_max;
-            b.ovf_n = m.ovf_n = w.ovf_n;
-            b.ovf_q = m.ovf_q = w.ovf_q;
-            b.ovf_slot = m.ovf_slot = w.ovf_slot;
-            b.ovf_done = w.ovf_done;
-            m.ovf_key = w.ovf_key;
-            m.ovf_id = w.ovf_id;
-            m.ovf_par = 1;
-        }
-        const dim3 rgrid(qg, (unsigned)std::min<int64_t>((cap + kWave - 1) / kWave, 16));
-        if (ix->D <= 256) {
-            if (xb_host) refine_survivors_kernel<true, 256><<<rgrid, kBlock, 0, st>>>(b, B);
-            else refine_survivors_kernel<false, 256><<<rgrid, kBlock, 0, st>>>(b, B);
-        } else {
-            if (xb_host) refine_survivors_kernel<true, 1024><<<rgrid, kBlock, 0, st>>>(b, B);
-            else refine_survivors_kernel<false, 1024><<<rgrid, kBlock, 0, st>>>(b, B);
-        }
+        // the refine, and before its queries' blocks those that rescan overflowed lists
+        const unsigned gy = (unsigned)std::min<int64_t>((cap + kWave - 1) / kWave, 16);
+        const dim3 rgrid(qg + (unsigned)((std::min<int64_t>((int64_t)B * nprobe, kRescanBlocks) + gy - 1) / gy), gy);
+        if (K <= 64) launch_refine<64>(b, rgrid, st);
+        else launch_refine<128>(b, rgrid, st);
         if ((rc = check_launch("refine_survivors_kernel"))) return rc;
         m.use_prev = 0;
         m.tau_sq_out = out->tau_sq;
         m.out_d = out->topk_d;
         m.out_i = out->topk_i;
-        m.probe_cids = w.probe_cids;
-        m.nprobe = nprobe;
-        m.vec_off = ix->cluster_vec_off;
-        m.xb = ix->xb_sorted;
-        m.xq64 = w.xq64;
-        m.tile_oids = ix->tile_orig_ids;
-        m.tile_off = ix->cluster_tile_off;
-        m.T = ix->tile_size;
-        m.D = ix->D;
-        if (rescan) {
-            constexpr int NW = kOvfExactThreads / kWave;
-            const unsigned og = (unsigned)std::min<int64_t>((w.ovf_max * nprobe + NW - 1) / NW, 4096);
-            if (KP == 64) ovf_exact_kernel<64><<<og, kOvfExactThreads, 0, st>>>(m);
-            else ovf_exact_kernel<128><<<og, kOvfExactThreads, 0, st>>>(m);
-            if ((rc = check_launch("ovf_exact_kernel"))) return rc;
-        }
+        m.ovf_cnt = nprobe * rescan_stride(K);
         if ((rc = launch_merge(m, KP, st))) return rc;
         if ((rc = mark(TRIDENT_EV_END))) return rc;
         if (out->stats) {
@@ -1484,17 +1469,7 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         // the chunk dimension stops at 16: waves loop over further chunks
         const dim3 rgrid((unsigned)((B + kWavesPerBlock - 1) / kWavesPerBlock),
                          (unsigned)std::min<int64_t>((cap + kWave - 1) / kWave, 16));
-        if (ix->D <= 256) {
-            if (b.xb_host)
-                refine_survivors_kernel<true, 256><<<rgrid, kBlock, 0, st>>>(b, B);
-            else
-                refine_survivors_kernel<false, 256><<<rgrid, kBlock, 0, st>>>(b, B);
-        } else {
-            if (b.xb_host)
-                refine_survivors_kernel<true, 1024><<<rgrid, kBlock, 0, st>>>(b, B);
-            else
-                refine_survivors_kernel<false, 1024><<<rgrid, kBlock, 0, st>>>(b, B);
-        }
+        launch_refine<0>(b, rgrid, st);
         if ((rc = check_launch("refine_survivors_kernel"))) return rc;
         m.use_prev = 0;
         m.out_d = out->topk_d;

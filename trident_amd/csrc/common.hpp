@@ -295,6 +295,50 @@ __device__ __forceinline__ bool list_offer(WaveList<KP>& L, int K, uint64_t ck, 
     return true;
 }
 
+template <int KP>
+__device__ __forceinline__ void list_store(const WaveList<KP>& L, uint64_t* k, int32_t* i) {
+    const int lane = lane_id();
+    k[lane] = L.k0;
+    i[lane] = L.i0;
+    if constexpr (KP >= 128) {
+        k[kWave + lane] = L.k1;
+        i[kWave + lane] = L.i1;
+    }
+    if constexpr (KP == 256) {
+        k[2 * kWave + lane] = L.k2;
+        i[2 * kWave + lane] = L.i2;
+        k[3 * kWave + lane] = L.k3;
+        i[3 * kWave + lane] = L.i3;
+    }
+}
+
+template <int KP>
+__device__ __forceinline__ void list_load(WaveList<KP>& L, const uint64_t* k, const int32_t* i) {
+    const int lane = lane_id();
+    L.k0 = k[lane];
+    L.i0 = i[lane];
+    if constexpr (KP >= 128) {
+        L.k1 = k[kWave + lane];
+        L.i1 = i[kWave + lane];
+    }
+    if constexpr (KP == 256) {
+        L.k2 = k[2 * kWave + lane];
+        L.i2 = i[2 * kWave + lane];
+        L.k3 = k[3 * kWave + lane];
+        L.i3 = i[3 * kWave + lane];
+    }
+}
+
+template <int KP>
+__device__ __forceinline__ void list_absorb(WaveList<KP>& L, int K, const uint64_t* k,
+                                            const int32_t* i) {
+    const int lane = lane_id();
+    for_chunks<KP>([&](auto cc) __attribute__((always_inline)) {
+        constexpr int c = decltype(cc)::value;
+        if (c * kWave < K) list_offer(L, K, k[c * kWave + lane], i[c * kWave + lane]);
+    });
+}
+
 // Stage Z staging area per wave: kStageCh x (kWave + 1) floats, used by refine_rows as
 // kStageRows rows of kStageDims + 1 floats
 constexpr int kStageCh = 32;

@@ -58,10 +58,11 @@ struct MergeArgs {
     float* out_d;         // [B, K] or null (final pass only)
     int64_t* out_i;
     float* tau_sq_out;    // [B] or null
-    // Rescan of a query whose candidate list overflowed `cap` (only the batched routes append
-    // without a per-pair cap): through the SQ8 bounds (ovf_bounds below), else every probed row
-    // refined exactly (mode 10's matrix route, whose index carries no SQ8 codes).
-    const int32_t* probe_cids;  // [B, nprobe] or null (no fallback needed)
+    // A query whose candidate list overflowed `cap` (only the batched routes append without a
+    // per-pair cap).  Mode 10's refine has replaced its list by ovf_cnt entries (the best of each
+    // probe); the cascade rescans it here through the SQ8 bounds (ovf_bounds below).
+    int ovf_cnt;
+    const int32_t* probe_cids;  // [B, nprobe], ovf_bounds only, as the rest
     int nprobe;
     const int32_t* vec_off;
     const float* xb;
@@ -83,7 +84,7 @@ struct MergeArgs {
     const double* xrot64;       // [B, D_pad]
     const double* qerr;         // [B, D_pad]
     double lb_scale, ub_scale;  // as ScanArgs
-    // Parallel rescan (ovf_par = 1; without ovf_bounds ovf_exact_kernel reads every probed row): the refine gives up to ovf_max
+    // Parallel rescan (ovf_par = 1): the refine gives up to ovf_max
     // overflowed queries a slot; ovf_scan_kernel rescans them one wave per (slot, probe), each
     // keeping its cluster's K best in ovf_key / ovf_id [ovf_max, nprobe, KP] -- upper bounds first,
     // which the slot's last wave to finish (ovf_done) reduces to the slot's threshold ovf_t, then
@@ -214,6 +215,10 @@ struct BatchArgs {
     // (MergeArgs); 0: none
     int ovf_max;
     int32_t *ovf_n, *ovf_q, *ovf_slot, *ovf_done;
+    // mode 10 (probe_cids not null): fine_tau_kernel lists the queries whose list overflowed in
+    // ovf_q [B], and the refine's launch rescans their probes
+    const int32_t* probe_cids;  // [B, nprobe]
+    int nprobe;
     int cm_emit;                // cm_scan_kernel: 1 lists rows, 0 only lowers the thresholds
     unsigned long long* host_rows;  // [1] rows read from the host-mapped base, or null
 };
@@ -529,9 +534,6 @@ __global__ void fine_tau_kernel(BatchArgs a, int B);
 // Parallel rescan of overflowed candidate lists (MergeArgs, ovf_par).
 template <int KP, bool UB>
 __global__ void ovf_scan_kernel(MergeArgs a);
-constexpr int kOvfExactThreads = 128;
-template <int KP>
-__global__ void ovf_exact_kernel(MergeArgs a);
 template <int KP>
 __global__ void cm_seed_kernel(BatchArgs a, int B);
 
@@ -560,8 +562,12 @@ __global__ void lb_scan_kernel(BatchArgs a);       // KS <= 4 (D_pad <= 256)
 template <int KS>
 __global__ void lb_scan_wide_kernel(BatchArgs a);  // 4 < KS <= 16
 
-template <bool HOST, int DQ>
+template <bool HOST, int DQ, int KP>
 __global__ void refine_survivors_kernel(BatchArgs a, int B);
+// Blocks of mode 10's refine that wait for overflowed lists (two a CU).
+constexpr int kRescanBlocks = 512;
+// Entries per probe that a rescanned list of mode 10 holds (cand_cap_min gives a list the room).
+__host__ __device__ constexpr int rescan_stride(int K) { return K < 64 ? 64 : K; }
 
 // Mode 10's matrix-core scan up to 256 dims: eight waves a workgroup, 16 queries of the unit each
 // (the wide kernel: four waves, 64 queries).

@@ -101,51 +101,6 @@ __device__ __forceinline__ float sq8_accumulate(const uint32_t* cp, int T, int d
     return acc;
 }
 
-template <int KP>
-__device__ __forceinline__ void list_store(const WaveList<KP>& L, uint64_t* k, int32_t* i) {
-    const int lane = lane_id();
-    k[lane] = L.k0;
-    i[lane] = L.i0;
-    if constexpr (KP >= 128) {
-        k[kWave + lane] = L.k1;
-        i[kWave + lane] = L.i1;
-    }
-    if constexpr (KP == 256) {
-        k[2 * kWave + lane] = L.k2;
-        i[2 * kWave + lane] = L.i2;
-        k[3 * kWave + lane] = L.k3;
-        i[3 * kWave + lane] = L.i3;
-    }
-}
-
-template <int KP>
-__device__ __forceinline__ void list_load(WaveList<KP>& L, const uint64_t* k, const int32_t* i) {
-    const int lane = lane_id();
-    L.k0 = k[lane];
-    L.i0 = i[lane];
-    if constexpr (KP >= 128) {
-        L.k1 = k[kWave + lane];
-        L.i1 = i[kWave + lane];
-    }
-    if constexpr (KP == 256) {
-        L.k2 = k[2 * kWave + lane];
-        L.i2 = i[2 * kWave + lane];
-        L.k3 = k[3 * kWave + lane];
-        L.i3 = i[3 * kWave + lane];
-    }
-}
-
-
-template <int KP>
-__device__ __forceinline__ void list_absorb(WaveList<KP>& L, int K, const uint64_t* k,
-                                            const int32_t* i) {
-    const int lane = lane_id();
-    for_chunks<KP>([&](auto cc) __attribute__((always_inline)) {
-        constexpr int c = decltype(cc)::value;
-        if (c * kWave < K) list_offer(L, K, k[c * kWave + lane], i[c * kWave + lane]);
-    });
-}
-
 __device__ __forceinline__ float hat_step(uint32_t code, float dl, float bs, float acc) {
     const float a = fmaf((float)code, dl, bs);
     return fmaf(a, a, acc);
@@ -584,44 +539,6 @@ __global__ __launch_bounds__(256) void ovf_scan_kernel(MergeArgs a) {
     }
 }
 
-// The same without bounds (mode 10's matrix-core scan, D <= 1024): one wave per (slot, probe) reads
-// the cluster's rows whole, 64 at a time (refine_rows), and keeps its K best; the largest cluster's
-// wave bounds it.  Rescanned by the merge, one wave took 93 ms for one query's 40 probes while every
-// other query waited.  K = 100: 200 queries at D = 960 95.0 -> 7.2 ms, 1000 at D = 128 18.3 -> 1.8;
-// K = 20, D = 960 101 -> 7.1; where no list overflows the launch costs 5 us (297 -> 304).  Two waves a
-// block: 33 KB of LDS.
-template <int KP>
-__global__ __launch_bounds__(kOvfExactThreads) void ovf_exact_kernel(MergeArgs a) {
-    constexpr int NW = kOvfExactThreads / kWave;
-    __shared__ double s_q64[NW][1024];
-    __shared__ float s_stage[NW][kStageCh][kWave + 1];
-    __shared__ int32_t s_pos[NW][kWave];
-    const int lane = threadIdx.x & 63, wid = (int)(threadIdx.x >> 6);
-    const int total = __builtin_amdgcn_readfirstlane(min(*a.ovf_n, a.ovf_max)) * a.nprobe;
-    for (int it = (int)blockIdx.x * NW + wid; it < total; it += (int)gridDim.x * NW) {
-        const int slot = it / a.nprobe, p = it - slot * a.nprobe;
-        const int q = __builtin_amdgcn_readfirstlane(a.ovf_q[slot]);
-        const int c = __builtin_amdgcn_readfirstlane(a.probe_cids[(size_t)q * a.nprobe + p]);
-        const int v0 = a.vec_off[c], n = a.vec_off[c + 1] - v0;
-        const int32_t* oids = a.tile_oids + (size_t)a.tile_off[c] * a.T;
-        wave_sync();  // the previous item's query is no longer read
-        for (int d = lane; d < a.D; d += kWave) s_q64[wid][d] = a.xq64[(size_t)q * a.D + d];
-        if (a.host_rows && lane == 0) atomicAdd(a.host_rows, (unsigned long long)max(n, 0));
-        WaveList<KP> L;
-        L.init();
-        for (int b0 = 0; b0 < n; b0 += kWave) {
-            const int m = min(kWave, n - b0);
-            wave_sync();
-            s_pos[wid][lane] = v0 + b0 + min(lane, m - 1);
-            wave_sync();
-            const double d64 = refine_rows(a.xb, nullptr, a.D, s_pos[wid], m, s_stage[wid], s_q64[wid]);
-            const bool in = lane < m;
-            list_offer(L, a.K, in ? key_of(d64) : kKeyInvalid, in ? oids[b0 + lane] : kIdInvalid);
-        }
-        list_store(L, a.ovf_key + (size_t)it * KP, a.ovf_id + (size_t)it * KP);
-    }
-}
-
 template <int KP>
 __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
     extern __shared__ float s_ovf[];  // ovf_bounds: 3 D_pad floats per wave
@@ -645,7 +562,7 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
             const int e = e0 + lane;
             list_offer(L, a.K, e < total ? k[e] : kKeyInvalid, e < total ? id[e] : kIdInvalid);
         }
-    } else if (raw > a.cap && a.probe_cids && a.ovf_bounds) {
+    } else if (raw > a.cap && a.ovf_bounds) {
         // Overflowed list, SQ8 codes at hand: the K-th smallest upper bound over the probed rows
         // (and the pass's threshold) bounds the K-th distance; only rows whose lower bound
         // passes it are read and refined.
@@ -658,33 +575,8 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
         const double t = fmin(a.tau64[q], kk != kKeyInvalid ? dist_of(kk) : (double)INFINITY);
         L.init();
         ovf_bounded_pass<KP, false>(a, q, L, t, s_par);
-    } else if (raw > a.cap && a.probe_cids) {
-        // Overflowed list: rescan every probed vector exactly (canonical float64 distance).
-        L.init();
-        const double* qv = a.xq64 + (size_t)q * a.D;
-        for (int p = 0; p < a.nprobe; ++p) {
-            const int c = a.probe_cids[(size_t)q * a.nprobe + p];
-            const int v0 = a.vec_off[c], n = a.vec_off[c + 1] - v0, t0 = a.tile_off[c];
-            if (a.host_rows && lane == 0) atomicAdd(a.host_rows, (unsigned long long)max(n, 0));
-            for (int b0 = 0; b0 < n; b0 += kWave) {
-                const int li = b0 + lane;
-                uint64_t k = kKeyInvalid;
-                int32_t id = kIdInvalid;
-                if (li < n) {
-                    const float* xr = a.xb + (size_t)(v0 + li) * a.D;
-                    double acc = 0.0;
-                    for (int d = 0; d < a.D; ++d) {
-                        const double t = (double)xr[d] - qv[d];
-                        acc = fma(t, t, acc);
-                    }
-                    k = key_of(acc);
-                    id = a.tile_oids[(size_t)t0 * a.T + li];
-                }
-                list_offer(L, a.K, k, id);
-            }
-        }
     } else {
-        const int cnt = min(raw, a.cap);
+        const int cnt = raw > a.cap ? a.ovf_cnt : raw;
         const uint64_t* ck = a.cand_key + (size_t)q * a.cap;
         const int32_t* ci = a.cand_id + (size_t)q * a.cap;
         for (int b0 = 0; b0 < cnt; b0 += kWave) {
@@ -829,8 +721,6 @@ template __global__ void ovf_scan_kernel<64, true>(MergeArgs);
 template __global__ void ovf_scan_kernel<64, false>(MergeArgs);
 template __global__ void ovf_scan_kernel<128, true>(MergeArgs);
 template __global__ void ovf_scan_kernel<128, false>(MergeArgs);
-template __global__ void ovf_exact_kernel<64>(MergeArgs);
-template __global__ void ovf_exact_kernel<128>(MergeArgs);
 template __global__ void merge_kernel<64>(MergeArgs);
 template __global__ void merge_kernel<128>(MergeArgs);
 template __global__ void merge_kernel<256>(MergeArgs);

@@ -418,14 +418,36 @@ int dispatch_scan(const ScanArgs& a, int kind, hipStream_t st) {
 // seeding unit lists K <= 128 bounds per query and the merge keeps 128), D_pad <= 1024 (query weights
 // held in registers: 8 VGPRs per 64 dims) and N < 2^27 (a queued survivor packs its index within the cluster
 // into 28 bits).  AUTO takes it when clusters are shared by >= 8 queries on average, where the
-// contraction is dense enough for the matrix cores, and below that when a cluster is long: the
-// per-pair route gives a cluster to one workgroup and its two passes run one after the other, so a
-// few queries wait for the longest cluster of each (1e6 rows, nlist 1024, D = 128, K = 10: 1 query 164
-// us per-pair, 149 batched; 16: 337, 185; D = 960, 390 rows a cluster: 24 queries 1588, 618).  On
-// short clusters the batched route's four launches more cost about 10 us (50,000 rows, nlist 200: 92
-// against 104).  The line: rows x dims of an average cluster >= 80,000 (333 x 64 and 250 x 128 are
-// even or slower, 977 x 128 and 1333 x 64 faster), 200,000 past 256 dims (250 x 384 about even, 390
-// x 960 faster); one query's single neighbour stays per-pair (105 against 119 at 1333 x 64).
+// contraction is dense enough for the matrix cores, and below that when a cluster is long
+// (long_clusters).
+//
+// Below 8 queries a cluster.  The per-pair route gives a cluster to one workgroup and its two passes
+// run one after the other, so a few queries wait for the longest cluster of each; the batched route
+// cuts clusters into slices, and its launches cost about 10 us more (25 of 110 for a single probe, whose
+// search has one per-pair pass).  c = rows x dims of an average cluster; us per-pair / batched:
+//   up to 256 dims from c = 80,000 (1e6 rows, nlist 1024, D = 128, nprobe 64, K = 10: 1 query 133 / 114,
+//     16: 327 / 138; K = 100: 256 / 149; 650 x 128, 32 probes: 4 queries 237 / 130; 390 x 128 about even, 250 x
+//     128: 95 / 108).  One query's single neighbour, whose threshold is tight from the start, from 100,000
+//     (500 x 200: 188 / 129, 977 x 128: 114 / 112; 977 x 96: 96 / 117);
+//   past 256 dims from 200,000 (250 x 384, 24 queries 302 / 256, but 4 of one neighbour 154 / 241; 667 x 384:
+//     4 queries 292 / 227), for one query from 350,000 (390 x 960: 268 / 252; 667 x 500: 178 / 197, 833 x 320: 150
+//     / 197, 234 x 960 and 400 x 768 even), its single neighbour never (390 x 960: 230 / 258);
+//   one probe: from 120,000 and 350,000 on for more than one query (977 x 128, 4 queries 177 / 115; 390 x
+//     960: 553 / 290), or when the queries together make up for it, B c >= 400,000 (977 x 96: 4 queries 119 /
+//     129, 64: 165 / 143; 500 x 200, 4 queries 184 / 131), past 256 dims 1,200,000 (400 x 768, 4 queries 396 / 270;
+//     667 x 384, 4 queries 130 / 179);
+//   past K = 16, where the per-pair lists cost more, from the first two lines on in any form.
+bool long_clusters(const TridentIndexView* ix, int B, int K, int nprobe) {
+    const double c = (double)ix->N / ix->nlist * ix->D;
+    const bool wide = ix->D_pad > 256;
+    const double far = wide ? 350000.0 : 120000.0;
+    if (c < (wide ? 200000.0 : 80000.0)) return false;
+    if (K > 16) return true;
+    if (B == 1 && K == 1) return !wide && nprobe > 1 && c >= 100000.0;
+    if (nprobe == 1) return (B > 1 && c >= far) || B * c >= (wide ? 1.2e6 : 4e5);
+    return B > 1 || !wide || c >= far;
+}
+
 int choose_route(const TridentIndexView* ix, const TridentSearchParams* sp, int B, int K,
                  int nprobe, int* route) {
     const bool ok = ix->vec_Ar && ix->sq8_cells && ix->orig_ids_sorted && K <= 128 &&
@@ -455,13 +477,10 @@ int choose_route(const TridentIndexView* ix, const TridentSearchParams* sp, int 
                             "the index view lacks sq8_packed (per-pair route) and this search "
                             "cannot take the batched route (K=%d, D_pad=%d, N=%d)",
                             K, ix->D_pad, ix->N);
-            {
-                const double cells = (double)ix->N / ix->nlist * ix->D;
-                const bool longc = cells >= (ix->D_pad <= 256 ? 80000.0 : 200000.0) && (B > 1 || K > 1);
-                *route = ok && (!pair_ok || (double)B * nprobe >= 8.0 * ix->nlist || longc)
-                             ? TRIDENT_ROUTE_BATCHED
-                             : TRIDENT_ROUTE_PAIR;
-            }
+            *route = ok && (!pair_ok || (double)B * nprobe >= 8.0 * ix->nlist ||
+                            long_clusters(ix, B, K, nprobe))
+                         ? TRIDENT_ROUTE_BATCHED
+                         : TRIDENT_ROUTE_PAIR;
             return TRIDENT_OK;
         default:
             return fail(TRIDENT_ERR_INVALID_ARGUMENT, "route=%d outside {0,1,2}", sp->route);
@@ -485,10 +504,28 @@ inline int seed_slice_count(int K, bool xb_host, bool fine) {
 // merge's lists).  AUTO takes it when clusters are shared by at least 4 queries on average
 // (16-row tiles with fewer rows leave most of each matrix instruction idle), always for a base in
 // mapped host memory (every row read crosses PCIe, and this route reads fewer), and, while K <= 16
-// (past that its lists take every row of the first probes, and may overflow), from 48,000 rows x dims
-// of an average cluster on: one float64 pass over a cluster takes longer than the idle lanes cost
-// (40 queries, 977 x 128: 1300 us per-pair, 400 here; 600 x 96: 311, 143; even at 250 x 128, slower at
-// 333 x 64).
+// (past that its lists take every row of the first probes, and may overflow), below that where the
+// per-pair scan's one float64 pass over a cluster takes longer than the idle lanes cost
+// (cm_long_clusters).
+//
+// c = rows x dims of an average cluster, P c with P pairs the work of the search; us per-pair / here:
+//   up to 256 dims from c = 60,000 (977 x 128, nprobe 64: 1 query 230 / 152, 40: 888 / 269; 1000 x 64, 16
+//     probes, 4 queries 155 / 128; 469 x 128 even), from 48,000 for clusters of at least 550 rows (600 x 96, 37
+//     probes, 4 queries 202 / 147; 390 x 128, 16 probes, 8 queries 116 / 139), or while P c >= 2.5e7 keeps
+//     the chip busy (390 x 128, 16 probes: 32 queries 151 / 149, 64: 261 / 161);
+//   past 256 dims, in float32 products, from 320,000 (390 x 960, 32 probes: 4 queries 1061 / 979, 24: 2475 /
+//     1136; 667 x 500, 16 probes, 1 query 553 / 426; 400 x 768: 572 / 733, 833 x 320: 356 / 384, 250 x 384: 234 /
+//     438; 667 x 384 even), from 200,000 while P c >= 8e7 (667 x 384, 16 probes, 24 queries 569 / 515; 234 x 960
+//     1126 / 1009), from 96,000 while P c >= 1.5e8 (250 x 384, 32 probes: 24 queries, 7.4e7, 434 / 503; 100,
+//     3.1e8, 1110 / 649); one probe, which has no warm-up pass here, as the cascade (400 x 768, 4 queries
+//     577 / 450; 667 x 384, 4 queries 133 / 206, 24: 363 / 285).
+bool cm_long_clusters(const TridentIndexView* ix, int B, int nprobe) {
+    const double rows = (double)ix->N / ix->nlist, c = rows * ix->D, work = (double)B * nprobe * c;
+    if (ix->D_pad <= 256) return c >= 60000.0 || (c >= 48000.0 && (rows >= 550.0 || work >= 2.5e7));
+    if (nprobe == 1) return c >= 200000.0 && work >= 1.2e6;
+    return c >= 320000.0 || (c >= 200000.0 && work >= 8e7) || (c >= 96000.0 && work >= 1.5e8);
+}
+
 int choose_cm_route(const TridentIndexView* ix, const TridentSearchParams* sp, int B, int K,
                     int nprobe, bool xb_host, bool* cm) {
     const bool ok = ix->orig_ids_sorted && K <= 128 && ix->D_pad <= 1024 &&
@@ -508,7 +545,7 @@ int choose_cm_route(const TridentIndexView* ix, const TridentSearchParams* sp, i
             return TRIDENT_OK;
         case TRIDENT_ROUTE_AUTO:
             *cm = ok && (xb_host || (double)B * nprobe >= 4.0 * ix->nlist ||
-                         (K <= 16 && (double)ix->N / ix->nlist * ix->D >= 48000.0));
+                         (K <= 16 && cm_long_clusters(ix, B, nprobe)));
             return TRIDENT_OK;
         default:
             return fail(TRIDENT_ERR_INVALID_ARGUMENT, "route=%d outside {0,1,2}", sp->route);

@@ -190,15 +190,14 @@ __device__ __forceinline__ void cm_tile_epilogue(const BatchArgs& a, const v4f s
 
 }  // namespace
 
-// How many of the other fifteen values of this lane's group of sixteen are smaller (lt), and how
-// many are not larger (le).
-__device__ __forceinline__ void rank16(uint32_t v, int& lt, int& le) {
-    lt = le = 0;
+// How many of the other fifteen values of this lane's group of sixteen are smaller (EQ: equal).
+template <bool EQ>
+__device__ __forceinline__ int rank16(uint32_t v) {
+    int rank = 0;
     auto one = [&](auto o_c) __attribute__((always_inline)) {
         constexpr int kRowRor = 0x120;  // DPP: rotate within the 16-lane row
         const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kRowRor + decltype(o_c)::value, 0xf, 0xf, false);
-        lt += o < v ? 1 : 0;
-        le += o <= v ? 1 : 0;
+        rank += (EQ ? o == v : o < v) ? 1 : 0;
     };
     one(std::integral_constant<int, 1>{});
     one(std::integral_constant<int, 2>{});
@@ -215,6 +214,7 @@ __device__ __forceinline__ void rank16(uint32_t v, int& lt, int& le) {
     one(std::integral_constant<int, 13>{});
     one(std::integral_constant<int, 14>{});
     one(std::integral_constant<int, 15>{});
+    return rank;
 }
 
 // x = h + m + l + r, each part rounded to nearest even (|r| <= 2^-24 |x|; the differences are exact),
@@ -530,7 +530,7 @@ __global__ __launch_bounds__(kCmThreads, D4 <= 32 ? 4 : 2) void cm_scan_kernel(B
                 // ---- thresholds: where at least K of a query row's 16 column minima are below its
                 // t, the K-th smallest becomes t (the warm-up, which lists nothing, selects after its
                 // last block only).  Each lane ranks its minimum among the row's sixteen by fifteen
-                // lane rotations; lanes that tie at the K-th store the same value. ----
+                // lane rotations. ----
                 if (K <= kCmQW && __ballot(lower) != 0ull && (a.cm_emit || blk0 + kCmBV >= ve)) {
                     lower = false;
                     const int g = opaque(lane) >> 4;
@@ -540,10 +540,15 @@ __global__ __launch_bounds__(kCmThreads, D4 <= 32 ? 4 : 2) void cm_scan_kernel(B
                         const uint32_t my = __float_as_uint(cmin[r]);
                         const bool below = my < 0x7f800000u && __uint_as_float(my) < s_t[wid][slot];
                         const uint64_t bm = __ballot(below);
-                        if (__ballot(__popc((uint32_t)(bm >> (16 * g)) & 0xffffu) >= K) == 0ull) continue;
-                        int lt, le;
-                        rank16(my, lt, le);
-                        if (below && lt < K && le >= K - 1) {
+                        const bool enough = __popc((uint32_t)(bm >> (16 * g)) & 0xffffu) >= K;
+                        if (__ballot(enough) == 0ull) continue;
+                        const int lt = rank16<false>(my);
+                        bool kth = below && lt == K - 1;
+                        const uint64_t km = __ballot(kth);
+                        // a tie at the K-th leaves no lane with that rank: the lanes that tie store it
+                        if (__ballot(enough && ((uint32_t)(km >> (16 * g)) & 0xffffu) == 0u) != 0ull)
+                            kth = below && lt < K && lt + rank16<true>(my) >= K - 1;
+                        if (kth) {
                             s_t[wid][slot] = __uint_as_float(my);
                             atomicMin(&a.ub_best[s_qid[wid][slot]], my);
                         }

@@ -9,26 +9,29 @@ smallest work at which the cascade is at least as fast (the reference's rule);
 measured work, which ignores an isolated win at a tiny batch.
 
 W0 is hardware-specific.  The reference's A100 value is 946,811,200 (README rounds it to
-9.0e8).  On MI355X (calibrate_w0, bench.py --calibrate-w0; mode 10 timed on its faster route,
-the matrix cores at every calibrated batch) the stable crossovers are W = 2.56e7 at
-configs[0] (B = 32), 6.4e7 at configs[1] (B = 8), 7.68e9 at configs[2] (D = 960, B = 128) and
-7.68e9 at configs[3] (B = 512).  W0_MI355X is the smallest, as the reference takes the smaller
-of its datasets' crossovers.
+9.0e8); W0_MI355X = 2.56e7.
 
-No single W0 fits all four: the crossing follows the pairs per probed cluster, not W.  From
-B * nprobe = 8 nlist on, the cascade runs its batched int8 matrix-core route and wins by 4-10x;
-below that it runs per (query, cluster) pair and mode 10's single matrix-core pass is
-faster or within 10 % (except single queries).  ``choose_mode_pairs`` routes by that (the
-library's own AUTO threshold for the cascade's batched route), and ``CostRouter`` uses it unless
-it is given a W0.
+No W0 alone fits, because the cascade has two routes here.  Where the library takes its batched
+int8 matrix-core route (clusters shared by 8 queries on average, or long ones: trident_route_for)
+it wins at any work: 1e6 rows, D = 128, nlist 1024, 64 probes, K = 10, 1 / 16 / 40 / 200 queries take
+114 / 138 / 148 / 176 us against mode 10's 152 / 260 / 269 / 365; at D = 960, nlist 512, 260 - 373 against
+717 - 1589.  So it does for a base in host memory, of which mode 10 reads every probed row (147 -
+285 us against 335 - 4316).  On its per-pair route, short clusters, the crossing follows the work
+as in the reference: 311 searches on twelve indexes (33 to 960 dims, 1 to 256 queries, K 1 to 50)
+cross between 1.5e7 (up to 256 dims) and 4e7 (past them).  ``choose_mode_route`` is that rule, and
+``CostRouter`` uses it unless it is given a W0: on those searches 1.03 times the faster mode in the
+geometric mean, at worst 2.3 (one query at D = 768).  ``choose_mode_pairs``, the rule by pairs per
+probed cluster alone, stands at 1.27 there, at worst 15.
 """
 import time
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from . import _lib
+
 W0_REFERENCE_A100 = 946_811_200.0
-# Smallest stable crossover over the calibrated configs on MI355X (configs[0]: B = 32).
+# Work from which the cascade's per-pair route is at least as fast as mode 10 on MI355X.
 W0_MI355X = 2.56e7
 # Pairs per cluster from which the cascade takes its batched route whatever the clusters' length
 # (capi.hip, choose_route).
@@ -52,6 +55,19 @@ def choose_mode_pairs(B: int, nprobe: int, nlist: int) -> int:
     """MI355X rule: mode 2 (cascade) once B * nprobe >= 8 nlist (its batched route), else
     mode 10."""
     return MODE_CASCADE if float(B) * nprobe >= BATCHED_PAIRS_PER_CLUSTER * nlist else MODE_CM_EXACT
+
+
+def choose_mode_route(index, B: int, nprobe: int, k: Optional[int] = None, route: int = 0) -> int:
+    """MI355X rule: mode 2 (cascade) where it takes its batched route, where the base lives in host
+    memory, and from W0_MI355X on; else mode 10.  Where the index cannot run this cascade, as
+    choose_mode_pairs (mode 10 below 8 pairs per cluster)."""
+    try:
+        batched = index.route_for(B, nprobe, k, route=route, mode=MODE_CASCADE) == _lib.ROUTE_BATCHED
+    except _lib.TridentError:
+        return choose_mode_pairs(B, nprobe, index.nlist)
+    if batched or getattr(index.storage, "placement", "device") == "host":
+        return MODE_CASCADE
+    return choose_mode(work_measure(B, nprobe, index.N, index.nlist, index.D), W0_MI355X)
 
 
 def _time_ms(fn, warmup: int, iters: int) -> float:
@@ -110,22 +126,27 @@ def stable_crossover(rows: List[Dict]) -> float:
 
 class CostRouter:
     """Routes each batch of an index to mode 10 or mode 2: ``rule="work"`` by the reference's
-    work measure against W0 (W0_MI355X unless given), ``rule="pairs"`` by choose_mode_pairs;
-    ``rule="auto"`` (the default) is "work" when a W0 is given, else "pairs"."""
+    work measure against W0 (W0_MI355X unless given), ``rule="pairs"`` by choose_mode_pairs,
+    ``rule="route"`` by choose_mode_route; ``rule="auto"`` (the default) is "work" when a W0 is
+    given, else "route" ("pairs" for an index without ``route_for``)."""
 
     def __init__(self, index, W0: Optional[float] = None, rule: str = "auto"):
-        if rule not in ("auto", "work", "pairs"):
-            raise ValueError(f"rule must be 'auto', 'work' or 'pairs', not {rule!r}")
+        if rule not in ("auto", "work", "pairs", "route"):
+            raise ValueError(f"rule must be 'auto', 'work', 'pairs' or 'route', not {rule!r}")
+        if rule == "auto":
+            rule = "work" if W0 is not None else "route" if hasattr(index, "route_for") else "pairs"
         self.index = index
-        self.rule = ("work" if W0 is not None else "pairs") if rule == "auto" else rule
+        self.rule = rule
         self.W0 = W0_MI355X if W0 is None else float(W0)
 
-    def mode_for(self, B: int, nprobe: int) -> int:
+    def mode_for(self, B: int, nprobe: int, k: Optional[int] = None, route: int = 0) -> int:
         ix = self.index
+        if self.rule == "route":
+            return choose_mode_route(ix, B, nprobe, k, route)
         if self.rule == "pairs":
             return choose_mode_pairs(B, nprobe, ix.nlist)
         return choose_mode(work_measure(B, nprobe, ix.N, ix.nlist, ix.D), self.W0)
 
     def search(self, xq: torch.Tensor, nprobe: int, **kw):
-        mode = self.mode_for(int(xq.shape[0]), nprobe)
+        mode = self.mode_for(int(xq.shape[0]), nprobe, kw.get("k"), kw.get("route", 0))
         return self.index.search(xq, nprobe, mode=mode, **kw) + (mode,)

@@ -87,13 +87,12 @@ typedef struct TridentIndexView {
                                         (c - 128 as int8), each V-slot block contiguous; NULL
                                         disables the batched route */
     /* Centroids for the matrix-core coarse pass, Dq = D rounded up to 16, c_d = -W_combined[d, c]
-     * / 2.  Optional (all or none): when cent_rows is NULL every search derives them from
+     * / 2.  Optional (all but cent_tiles, or none): when cent_rows is NULL every search derives them from
      * W_combined into its workspace.  No counterpart in the reference (its coarse GEMM reads
      * W_coarse_only directly). */
     const float* cent_rows;          /* [nlist, Dq] zero-padded rows */
-    const float* cent_tiles;         /* [ceil(nlist / 16) * 16 * Dq] matrix-core tile layout: float4
-                                        (t Dq/16 + j) 64 + l holds dims (l / 16) Dq/4 + 4 j .. + 3
-                                        of centroid 16 t + l % 16 */
+    const float* cent_tiles;         /* ignored, may be NULL (a tile layout of the rows that no kernel
+                                        reads; the place keeps the other fields') */
     const float* cent_norms;         /* [nlist] float32(sum_d c_d^2) */
     double cent_norm_max;            /* max_c sum_d c_d^2 (float64) */
     const float* r_vec_sorted;       /* [N] |x - c(x)| in sorted order, float32 of the float64 norm

@@ -1,5 +1,5 @@
 """The bfloat16 split form of the coarse pass (csrc/frontend.hip, coarse_gemm_bf16_kernel and the
-band derivation above mfma_tile_offset), restated in numpy and checked against its error bound:
+band derivation above bf16_tile_offset), restated in numpy and checked against its error bound:
 
     x = h + l + r,  h = bf16(x), l = bf16(x - h)  (round to nearest even),
     s' = (H0 + H1) + (L0 + L1)  over Dp = 32 ceil(Dq / 32) zero-padded dimensions, where H0 / H1

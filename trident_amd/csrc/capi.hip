@@ -289,16 +289,16 @@ int validate_index(const TridentIndexView* ix) {
     if (!(ix->rot_sq_min > 0.0) || !(ix->rot_sq_max >= ix->rot_sq_min))
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "bad rotation bounds [%g, %g]", ix->rot_sq_min,
                     ix->rot_sq_max);
-    if (ix->cent_rows && (!ix->cent_tiles || !ix->cent_norms || !(ix->cent_norm_max >= 0.0) ||
-                          !(ix->cent_norm_max < INFINITY)))
+    if (ix->cent_rows && (!ix->cent_norms || !(ix->cent_norm_max >= 0.0) || !(ix->cent_norm_max < INFINITY)))
         return fail(TRIDENT_ERR_INVALID_ARGUMENT,
-                    "cent_rows needs cent_tiles, cent_norms and a finite cent_norm_max >= 0");
+                    "cent_rows needs cent_norms and a finite cent_norm_max >= 0");
     return TRIDENT_OK;
 }
 
-// The batched routes scan per-cluster counters in blocks of kBlock clusters and carry the block
-// totals in one block (unit_scan_carry_kernel: 2 nlist counters, at most kBlock blocks).
-constexpr int kMaxBatchedNlist = kBlock * kBlock / 2;
+// The batched routes' offsets come from one block that scans the clusters 4096 at a time
+// (group_scan_kernel: 13 us at nlist 4096, growing with it; its units hold the cluster in 20 bits), so
+// they stop at 32,768 clusters.
+constexpr int kMaxBatchedNlist = 32768;
 
 // The SQ8 parameters every SQ8 route reads; the reference packing (sq8_packed) only where
 // `packed` (the per-pair scans, modes 0 / 1, the bound entry points).  A mode-2 index may carry
@@ -1434,7 +1434,6 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         b.pair_cid = w.pair_cids;
         b.seg = w.seg_off;
         b.M = (int)(M1 + M2);
-        b.unit_q = lb_unit_q(ix->D_pad);
         b.DP = (int)plane_bytes(ix->D_pad);
         b.pw = w.pw;
         b.prec = w.prec;

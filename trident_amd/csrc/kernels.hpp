@@ -174,7 +174,6 @@ struct BatchArgs {
     const int32_t* seg;         // [2, nlist + 1] cluster starts, seeding ends
     int M;                      // pairs (both passes)
     int nlist;
-    int unit_q;                 // queries per lower-bound unit (kUnitQ or kUnitQWide)
     const int2* groups;        // weight groups {first pair, pair count}
     const int32_t* grp_off;     // [nlist + 1]; grp_off[nlist] = number of groups
     int max_groups;

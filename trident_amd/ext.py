@@ -192,8 +192,8 @@ def make_index_view(*, N, D, D_pad, nlist, tile_size, per_cluster_sq8, W_combine
     v.seed_rows = int(seed_rows)
     v.xb_sorted_u8 = device_pointer(xb_sorted_u8) if xb_sorted_u8 is not None else None
     if cent_band is not None:
-        rows, tiles, norms, nmax = cent_band
-        v.cent_rows, v.cent_tiles, v.cent_norms = _ptr(rows), _ptr(tiles), _ptr(norms)
+        rows, _, norms, nmax = cent_band
+        v.cent_rows, v.cent_norms = _ptr(rows), _ptr(norms)
         v.cent_norm_max = float(nmax)
     return v
 
@@ -213,23 +213,26 @@ def band_dq(D: int) -> int:
     return (int(D) + 15) & ~15
 
 
-def centroid_band_layouts(W_combined: torch.Tensor, nlist: int):
+def centroid_band_layouts(W_combined: torch.Tensor, nlist: int, tiles: bool = True):
     """(rows [nlist, Dq], tiles, norms [nlist], max norm) of the centroids c_d = -W[d, c] / 2,
-    the optional TridentIndexView fields cent_*: built once per index instead of per search."""
+    the optional TridentIndexView fields cent_*: built once per index instead of per search.  No
+    kernel reads the tile layout; ``tiles=False`` (what the index keeps) puts None in its place."""
     D = int(W_combined.shape[0])
     Dq = band_dq(D)
     dev = W_combined.device
     cen = (-0.5 * W_combined[:, :nlist]).t().contiguous()          # exact: power-of-two scale
     rows = torch.zeros((nlist, Dq), device=dev, dtype=torch.float32)
     rows[:, :D] = cen
-    nl16 = (nlist + 15) // 16 * 16
-    pad = torch.zeros((nl16, Dq), device=dev, dtype=torch.float32)
-    pad[:nlist] = rows
-    S = Dq // 4
-    # [t, m, g, j, e] -> [t, j, g, m, e]: float4 (t S/4 + j) 64 + (m + 16 g) = dims g S + 4 j + e
-    tiles = pad.view(nl16 // 16, 16, 4, S // 4, 4).permute(0, 3, 2, 1, 4).contiguous().view(-1)
     n64 = (rows.double() ** 2).sum(1)
-    return rows, tiles, n64.to(torch.float32), float(n64.max()) if nlist else 0.0
+    t = None
+    if tiles:
+        nl16 = (nlist + 15) // 16 * 16
+        pad = torch.zeros((nl16, Dq), device=dev, dtype=torch.float32)
+        pad[:nlist] = rows
+        S = Dq // 4
+        # [t, m, g, j, e] -> [t, j, g, m, e]: float4 (t S/4 + j) 64 + (m + 16 g) = dims g S + 4 j + e
+        t = pad.view(nl16 // 16, 16, 4, S // 4, 4).permute(0, 3, 2, 1, 4).contiguous().view(-1)
+    return rows, t, n64.to(torch.float32), float(n64.max()) if nlist else 0.0
 
 
 def _identity(*ts):
@@ -255,7 +258,7 @@ def derived_layouts(W_combined, b_combined, sq8_packed, cluster_vec_off, cluster
                                       W_combined, b_combined, vmin, delta, per_cluster_sq8, nlist,
                                       tile_size)
         cells = _index.cells_from_packed(sq8_packed, D_pad, int(tile_size))
-        band = centroid_band_layouts(W_combined, nlist)
+        band = centroid_band_layouts(W_combined, nlist, tiles=False)
         vec_cn = _index.derive_vec_cn(cells, cluster_vec_off, cluster_tile_off, D_pad, int(tile_size))
         if len(_derived_cache) >= 2:
             _derived_cache.pop(next(iter(_derived_cache)))
@@ -454,6 +457,8 @@ def launch_trident_v4_search(
         for name, t, numel in (("cent_band rows", rows_t, nlist * Dq),
                                ("cent_band tiles", tiles_t, (nlist + 15) // 16 * 16 * Dq),
                                ("cent_band norms", norms_t, nlist)):
+            if t is None and name == "cent_band tiles":
+                continue
             _check_tensor(name, t, torch.float32, dev)
             _need(t.numel() == numel, f"{name} must hold {numel} floats")
     if stats_buf is not None:

@@ -429,8 +429,8 @@ class TridentV4Index:
       cluster_tile_off int32 [nlist + 1]; vmin / delta / eps_pad f32 [nlist or 1, D_pad]
       blk_bounds4  int32 [nb + 1] (32-dim blocks, or the variable scheme of :233-247)
       W_combined [D, nlist + D_pad] = [-2 C^T | R | 0], b_combined = [|c|^2 | b | 0]
-      cent_band    the centroids for the matrix-core coarse pass (rows, tile layout, norms,
-                   max norm; ext.centroid_band_layouts)
+      cent_band    the centroids for the matrix-core coarse pass (rows, None, norms, max norm;
+                   ext.centroid_band_layouts)
     """
 
     def __init__(self, storage: SharedClusterStorage, centroids, mean64, R64, tile_size: int = 256,
@@ -486,7 +486,7 @@ class TridentV4Index:
         self.W_combined[:, nlist:nlist + D] = R32.to(dev)
         self.b_combined[0, :nlist] = c_norm_sq
         self.b_combined[0, nlist:nlist + D] = b32.to(dev)
-        self.cent_band = _ext.centroid_band_layouts(self.W_combined, nlist)
+        self.cent_band = _ext.centroid_band_layouts(self.W_combined, nlist, tiles=False)
 
         # ---- rotate, quantise, bound (chunked over sorted rows) ----
         vec_off = storage.cluster_vec_off.to(torch.int64)

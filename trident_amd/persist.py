@@ -251,7 +251,7 @@ def load_index(path: str, device="cuda:0", xb_placement: str = "device", xb_raw=
     ix.W_combined, ix.b_combined = f32(meta["W_combined"]), f32(meta["b_combined"])
     ix.W_coarse_only = ix.W_combined[:, :nlist].contiguous()
     ix.b_coarse_only = ix.b_combined[:, :nlist].contiguous()
-    ix.cent_band = _ext.centroid_band_layouts(ix.W_combined, nlist)
+    ix.cent_band = _ext.centroid_band_layouts(ix.W_combined, nlist, tiles=False)
     ix.vmin_pad, ix.delta_pad, ix.eps_pad = f32(meta["vmin"]), f32(meta["delta"]), f32(meta["eps"])
     ix.blk_bounds4 = i32(meta["blk_bounds4"])
     ix.tile_r_minmax = f32(meta["tile_r_minmax"])

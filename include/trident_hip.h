@@ -192,8 +192,12 @@ int trident_event_create(void** event);
 int trident_event_destroy(void* event);
 int trident_event_elapsed_ms(void* start, void* stop, float* ms);
 
-/* Bytes of scratch trident_search needs for batches up to max_B x max_nprobe x max_K.  For mode 0
- * with rerank_m > 0, max_K must cover M = min(max(rerank_m, K), 200) as well. */
+/* Bytes of scratch for trident_search at full speed, for batches up to max_B x max_nprobe x max_K.
+ * For mode 0 with rerank_m > 0, max_K must cover M = min(max(rerank_m, K), 200) as well.  Less is
+ * accepted, with the same results: candidate lists of max(K, 64) slots a probe instead of up to
+ * 4096 a query (more of them overflow and are rescanned), then float64 coarse distances instead of
+ * the matrix-core ones.  A workspace too small even for that is refused, and the message of
+ * trident_last_error names the least that this search takes. */
 size_t trident_workspace_bytes(const TridentIndexView* ix, int32_t max_B, int32_t max_nprobe,
                                int32_t max_K);
 
@@ -209,8 +213,8 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
  * is a fixed device array of TRIDENT_NOALLOC_SCRATCH_BYTES compiled into the library (one copy
  * per GPU, kept until the process ends).  No counterpart in the reference: it is for callers
  * that cannot allocate device memory (code under graph capture, tight serving loops, hosts that
- * forbid hipMalloc).  Batches whose trident_workspace_bytes exceeds the array fail with
- * TRIDENT_ERR_WORKSPACE_TOO_SMALL.  The stream's device must be the current device.  Every call
+ * forbid hipMalloc).  Batches whose least scratch (see trident_workspace_bytes) exceeds the array
+ * fail with TRIDENT_ERR_WORKSPACE_TOO_SMALL.  The stream's device must be the current device.  Every call
  * on one GPU shares that GPU's array (each call initialises what it reads), so calls that
  * overlap on one GPU -- on different streams or host threads -- race and must be serialised by
  * the caller; calls in one stream are ordered and safe. */

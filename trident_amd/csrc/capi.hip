@@ -112,6 +112,7 @@ struct Workspace {
     float* pair_dqcs;
     int32_t* pair_rank;              // arrival ranks of the pairs in their (pass, cluster) bins
     int64_t cap;                     // candidate-list slots per query
+    bool band;                       // the coarse pass is the matrix-core one
     uint64_t* cand_key;
     int32_t* cand_id;
     int32_t* cand_cnt;
@@ -192,8 +193,10 @@ inline int64_t cand_cap(const TridentIndexView* ix, int64_t nprobe, int64_t K, b
     return deep ? std::max<int64_t>(least, std::min<int64_t>(2 * rows, 4096)) : least;
 }
 
+// `band` false leaves out the matrix-core coarse pass: the search takes float64 distances to every
+// centroid instead, whose scratch is 8 B nlist bytes (see best_carve).
 Workspace carve(const TridentIndexView* ix, void* base, int64_t B, int64_t nprobe, int64_t K,
-                bool deep = true) {
+                bool deep = true, bool band = true) {
     Carver c{static_cast<char*>(base)};
     Workspace w;
     const int64_t KP = K <= 64 ? 64 : K <= 128 ? 128 : 256;
@@ -238,14 +241,18 @@ Workspace carve(const TridentIndexView* ix, void* base, int64_t B, int64_t nprob
     // float64 coarse distances [B, nlist], or, on the band path (nprobe <= 128), float32
     // approximations in rows of band_lda(nlist) floats
     const int64_t lda = band_lda(ix->nlist);
-    w.cd64 = c.take<double>(nprobe <= 128 ? (B * lda + 1) / 2 : B * std::max<int64_t>(ix->nlist, (lda + 1) / 2));
-    w.qtb = c.take<uint32_t>((B + 15) / 16 * 16 * row_words);
-    w.cmtb = c.take<uint32_t>(((int64_t)ix->nlist + 15) / 16 * 16 * row_words);
-    w.tmin = c.take<float>(ix->nlist >= kTileMinNlist && Dq <= 128 ? B * (((int64_t)ix->nlist + 15) / 16) : 0);
-    w.qn32 = c.take<float>(B);
-    w.cm32 = c.take<float>((int64_t)ix->nlist * Dq);
-    w.cn32 = c.take<float>(ix->nlist);
-    w.cmax2 = c.take<unsigned long long>(1);
+    band = w.band = band && nprobe <= 128;
+    w.cd64 = c.take<double>(band ? (B * lda + 1) / 2 : B * ix->nlist);
+    if (band) {
+        const int64_t derived = ix->cent_rows ? 0 : ix->nlist;  // centroid rows and norms made per search
+        w.qtb = c.take<uint32_t>((B + 15) / 16 * 16 * row_words);
+        w.cmtb = c.take<uint32_t>(((int64_t)ix->nlist + 15) / 16 * 16 * row_words);
+        w.tmin = c.take<float>(ix->nlist >= kTileMinNlist && Dq <= 128 ? B * (((int64_t)ix->nlist + 15) / 16) : 0);
+        w.qn32 = c.take<float>(B);
+        w.cm32 = c.take<float>(derived * Dq);
+        w.cn32 = c.take<float>(derived);
+        w.cmax2 = c.take<unsigned long long>(1);
+    }
     const size_t front_end = c.off;
     c.off = shared;
     w.cand_key = c.take<uint64_t>(B * cap);
@@ -262,6 +269,21 @@ Workspace carve(const TridentIndexView* ix, void* base, int64_t B, int64_t nprob
     w.ovf_id = c.take<int32_t>(w.ovf_max * nprobe * std::min<int64_t>(KP, 128));
     c.off = std::max(c.off, front_end);
     w.bytes = c.off;
+    return w;
+}
+
+// The carve that a workspace of `bytes` has room for: whole, with the smaller candidate lists, or
+// with those and the float64 coarse pass.  The last serves many centroids of many dimensions in little
+// scratch, where the split operands (6 bytes a dimension of each, and 4 for the rows when the index
+// does not hold them) would not fit: nlist 7026, D = 1024, 2 queries 70 MB against 30.
+Workspace best_carve(const TridentIndexView* ix, void* base, size_t bytes, int64_t B, int64_t nprobe, int64_t K,
+                     bool deep = true) {
+    Workspace w = carve(ix, base, B, nprobe, K, deep);
+    if (bytes < w.bytes && deep) w = carve(ix, base, B, nprobe, K, false);
+    if (bytes < w.bytes) {
+        const Workspace e = carve(ix, base, B, nprobe, K, false, false);
+        if (e.bytes < w.bytes) w = e;
+    }
     return w;
 }
 
@@ -790,7 +812,7 @@ int run_front_end(const TridentIndexView* ix, const float* xq, int B, int nprobe
                   int ld, hipStream_t st) {
     const int ldw = ix->nlist + ix->D_pad;
     int rc = TRIDENT_OK;
-    const bool band = nprobe <= 128;
+    const bool band = w.band;  // nprobe <= 128, unless the workspace is short
     const int Dq = band_dq(ix->D);
     const float *cm = ix->cent_rows, *cn = ix->cent_norms;
     const unsigned long long* cmax_dev = nullptr;
@@ -1078,7 +1100,7 @@ int trident_coarse_probe(const TridentIndexView* ix, const float* xq, int32_t B,
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "bad probe arguments B=%d nprobe=%d ld=%d", B,
                     nprobe, probe_ld);
     if (B == 0) return TRIDENT_OK;
-    Workspace w = carve(ix, workspace, B, nprobe, 1, false);
+    const Workspace w = best_carve(ix, workspace, workspace_bytes, B, nprobe, 1, false);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);
@@ -1160,8 +1182,7 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
     if (B == 0) return TRIDENT_OK;
     if (!xq) return fail(TRIDENT_ERR_INVALID_ARGUMENT, "xq is NULL");
 
-    Workspace w = carve(ix, workspace, B, nprobe, K_list);
-    if (workspace_bytes < w.bytes) w = carve(ix, workspace, B, nprobe, K_list, false);
+    const Workspace w = best_carve(ix, workspace, workspace_bytes, B, nprobe, K_list);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);
@@ -1648,7 +1669,9 @@ int trident_search_noalloc(const TridentIndexView* ix, const TridentSearchParams
     // the size check comes before any HIP call, so an oversized request fails without touching
     // the device
     const size_t need =
-        carve(ix, nullptr, sp->B, sp->nprobe, merged_list_len(sp->mode, sp->K, sp->rerank_m), false).bytes;
+        best_carve(ix, nullptr, (size_t)TRIDENT_NOALLOC_SCRATCH_BYTES, sp->B, sp->nprobe,
+                   merged_list_len(sp->mode, sp->K, sp->rerank_m))
+            .bytes;
     if (need > (size_t)TRIDENT_NOALLOC_SCRATCH_BYTES)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL,
                     "trident_search_noalloc: B=%d nprobe=%d K=%d needs %zu bytes of scratch, more "
@@ -1679,7 +1702,7 @@ int trident_sq8_bounds(const TridentIndexView* ix, const float* xq, int32_t B,
     if ((rc = validate_cascade_index(ix))) return rc;
     if (B < 1 || n < 0 || !xq || !qids || !cids || !spos || !lb || !ub)
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "bad sq8_bounds arguments");
-    Workspace w = carve(ix, workspace, B, 1, 1, false);
+    const Workspace w = carve(ix, workspace, B, 1, 1, false, false);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);
@@ -1717,7 +1740,7 @@ int trident_fine_bounds(const TridentIndexView* ix, const float* xq, int32_t B,
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "fine_bounds needs fine_codes and fine_qp");
     if (B < 1 || n < 0 || !xq || !qids || !spos || !lb || !ub)
         return fail(TRIDENT_ERR_INVALID_ARGUMENT, "bad fine_bounds arguments");
-    Workspace w = carve(ix, workspace, B, 1, 1, false);
+    const Workspace w = carve(ix, workspace, B, 1, 1, false, false);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(TRIDENT_ERR_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes", workspace_bytes,
                     w.bytes);

@@ -275,7 +275,7 @@ Workspace carve(const TridentIndexView* ix, void* base, int64_t B, int64_t nprob
 // The carve that a workspace of `bytes` has room for: whole, with the smaller candidate lists, or
 // with those and the float64 coarse pass.  The last serves many centroids of many dimensions in little
 // scratch, where the split operands (6 bytes a dimension of each, and 4 for the rows when the index
-// does not hold them) would not fit: nlist 7026, D = 1024, 2 queries 70 MB against 30.
+// does not hold them) would not fit: nlist 7000, D = 1024, 2 queries 72 MB against 2.6.
 Workspace best_carve(const TridentIndexView* ix, void* base, size_t bytes, int64_t B, int64_t nprobe, int64_t K,
                      bool deep = true) {
     Workspace w = carve(ix, base, B, nprobe, K, deep);

@@ -483,21 +483,25 @@ __device__ __forceinline__ double row_d64(const float* __restrict__ xr, const fl
     return acc;
 }
 
-// Mode 10's overflowed lists (ovf_n queries in ovf_q), in the refine's launch, its first blocks
-// (the queries' follow): one block per (query, probe) reads the cluster's rows whole, each wave every
-// fourth run of 64, and puts the cluster's K best by (float64 distance, original id) in place of
-// the query's list, at p * rescan_stride(K).  Every member of the query's top-K is among its own
-// cluster's K best, so the merge of these entries is the exact result.  Without an overflow the
-// blocks end on reading ovf_n: a launch of their own cost each search 5 us, and one wave of the
+// Overflowed lists (ovf_n queries in ovf_q) rescanned exactly, by blocks rb of nrb: one block per
+// (query, probe) reads the cluster's rows whole, each wave every fourth run of 64, and puts the
+// cluster's K best by (float64 distance, original id) in place of the query's list, at
+// p * rescan_stride(K).  Every member of the query's top-K is among its own cluster's K best, so
+// the merge of these entries is the exact result, for any number of queries.
+//   Mode 10: in the refine's launch, its first blocks (the queries' follow), which without an
+// overflow end on reading ovf_n (a launch of their own cost each search 5 us).  One wave of the
 // merge, where a query's lists fell to it, took 55 ms for 63 clusters of 4000 rows (D = 128).
+//   Cascade over a device base: rescan_kernel, after the refine, which lists the queries.  (Over a
+// host base ovf_scan_kernel goes through the SQ8 bounds, so that few rows cross PCIe.  Here that
+// was slower, a wave to a probe and two launches, for 32 + B / 64 queries, the others by one wave of
+// the merge: 58 clusters of 4000 rows, K = 10, no query with a threshold, 1 / 16 / 200 queries 772 / 1417 /
+// 25,032 us, this way 302 / 1091 / 6705; the per-pair cascade 224 / 285 / 1691.)
 template <bool HOST, int KP>
-__device__ __forceinline__ void rescan_lists(const BatchArgs& a, int B, float* s_q, int32_t* s_pos, double* s_q64,
-                                             float (*s_stage)[kWave + 1]) {
+__device__ __forceinline__ void rescan_lists(const BatchArgs& a, int rb, int nrb, float* s_q, int32_t* s_pos,
+                                             double* s_q64, float (*s_stage)[kWave + 1]) {
     __shared__ uint64_t s_ck[kWavesPerBlock - 1][KP];
     __shared__ int32_t s_ci[kWavesPerBlock - 1][KP];
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int rb = (int)(blockIdx.x * gridDim.y + blockIdx.y);
-    const int nrb = ((int)gridDim.x - (B + kWavesPerBlock - 1) / kWavesPerBlock) * (int)gridDim.y;
     const int D = a.D, K = a.K, S = rescan_stride(K);
     const bool vec4 = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(a.xb) & 15) == 0;
     const int total = __builtin_amdgcn_readfirstlane(*a.ovf_n) * a.nprobe;
@@ -558,10 +562,11 @@ __device__ __forceinline__ void rescan_lists(const BatchArgs& a, int B, float* s
 // (query, 64-slot chunk of its list), one survivor per lane (a query with many survivors
 // spreads over many waves); each lane walks its own row in dimension order with 16-byte loads,
 // against the query row staged in LDS (DQ >= D floats per wave: 256, or 1024 for the wide
-// batched route).  An overflowed list (count > cap) is left alone: with KP = 0 the merge rescans
-// that query's probes through the SQ8 bounds (merge_kernel), in a slot of the parallel rescan taken
-// here while there are any; with KP > 0 (mode 10) the launch's first blocks rescan it
-// (rescan_lists).
+// batched route).  An overflowed list (count > cap) is left alone and its query's probes are
+// rescanned: with KP > 0 (mode 10) by the launch's first blocks (rescan_lists); with KP = 0 (the
+// cascade) over a device base by rescan_kernel, for which it is listed here, over a host base
+// through the SQ8 bounds, in a slot of the parallel rescan taken here while there are any, else by
+// merge_kernel.
 // (Registers for as many waves as the LDS leaves room for: the rescan would take more.)
 template <bool HOST, int DQ, int KP>
 __global__ __launch_bounds__(256, !HOST ? 4 : DQ > 256 ? 2 : 3) void refine_survivors_kernel(BatchArgs a, int B) {
@@ -573,17 +578,19 @@ __global__ __launch_bounds__(256, !HOST ? 4 : DQ > 256 ? 2 : 3) void refine_surv
     const int lane = threadIdx.x & 63, wid = (int)(threadIdx.x >> 6);
     int bx = (int)blockIdx.x;
     if constexpr (KP > 0) {
-        bx -= (int)gridDim.x - (B + W - 1) / W;  // the rescan's blocks come first: idle ones end unseen
+        const int nx = (int)gridDim.x - (B + W - 1) / W;
+        bx -= nx;  // the rescan's blocks come first: idle ones end unseen
         if (bx < 0) {
-            rescan_lists<HOST, KP>(a, B, s_q[wid], s_pos[HOST ? wid : 0], s_q64[HOST ? wid : 0],
-                                   s_stage[HOST ? wid : 0]);
+            rescan_lists<HOST, KP>(a, (int)(blockIdx.x * gridDim.y + blockIdx.y), nx * (int)gridDim.y, s_q[wid],
+                                   s_pos[HOST ? wid : 0], s_q64[HOST ? wid : 0], s_stage[HOST ? wid : 0]);
             return;
         }
     }
     const int q = __builtin_amdgcn_readfirstlane(bx * W + wid);
     if (q >= B) return;
     const int cnt = a.cand_cnt[q], ns = a.seed_cnt[q];
-    if (KP == 0 && a.ovf_max > 0 && blockIdx.y == 0 && lane == 0) {
+    if (KP == 0 && !HOST && cnt > a.cap && blockIdx.y == 0 && lane == 0) a.ovf_q[atomicAdd(a.ovf_n, 1)] = q;
+    if (KP == 0 && HOST && blockIdx.y == 0 && lane == 0) {
         int slot = -1;
         if (cnt > a.cap) {
             const int s = atomicAdd(a.ovf_n, 1);
@@ -670,6 +677,16 @@ __global__ __launch_bounds__(256, !HOST ? 4 : DQ > 256 ? 2 : 3) void refine_surv
     }
 }
 
+template <int KP, int DQ>
+__global__ __launch_bounds__(256) void rescan_kernel(BatchArgs a) {
+    __shared__ __align__(16) float s_q[kWavesPerBlock][DQ];
+    rescan_lists<false, KP>(a, (int)blockIdx.x, (int)gridDim.x, s_q[threadIdx.x >> 6], nullptr, nullptr, nullptr);
+}
+
+template __global__ void rescan_kernel<64, 256>(BatchArgs);
+template __global__ void rescan_kernel<64, 1024>(BatchArgs);
+template __global__ void rescan_kernel<128, 256>(BatchArgs);
+template __global__ void rescan_kernel<128, 1024>(BatchArgs);
 template __global__ void refine_survivors_kernel<false, 256, 0>(BatchArgs, int);
 template __global__ void refine_survivors_kernel<false, 256, 64>(BatchArgs, int);
 template __global__ void refine_survivors_kernel<false, 256, 128>(BatchArgs, int);

@@ -150,7 +150,7 @@ struct Workspace {
     int64_t ovf_max;
     int32_t* ovf_n;                  // [1]
     int32_t* ovf_q;                  // [ovf_max]
-    int32_t* ovf_slot;               // [B]; mode 10: its overflowed queries
+    int32_t* ovf_slot;               // [B]; without slots (device base, mode 10) the overflowed queries
     int32_t* ovf_done;               // [ovf_max]
     double* ovf_t;                   // [ovf_max]
     uint64_t* ovf_key;               // [ovf_max, nprobe, KP <= 128]
@@ -158,8 +158,8 @@ struct Workspace {
     size_t bytes;
 };
 
-// Overflowed queries of a cascade rescanned in parallel per search (the rest take the merge's
-// serial rescan; mode 10 rescans every one in parallel, in its refine):
+// Overflowed queries of a cascade over a host base rescanned in parallel per search (the rest take
+// the merge's serial rescan; everything else rescans every one in parallel, rescan_lists):
 // 188 at B = 10,000, 18.5 MB of per-probe lists at K <= 64.  A configs[4] search whose seeding
 // threshold was made loose on purpose (p_init 1) overflows fewer than that: 243 -> 17 ms per
 // step against the serial rescan; larger budgets (B / 16, B / 4) changed nothing.
@@ -170,11 +170,10 @@ inline int64_t plane_bytes(int D_pad) { return 64 * (int64_t)((D_pad + 63) / 64)
 
 // Candidate-list slots per query.  The batched route stores every lower-bound survivor there
 // (before its exact test), so lists are at least 64 * nprobe deep (12 bytes a slot; only used
-// slots are touched): a longer list makes that query's probes be rescanned (the SQ8 bounds of
-// every probed row, one wave per (query, probe) for up to ovf_slots_of(B) queries, one wave per
-// query past that, and the rows near the top-K refined), so the lists are sized to make that
-// rare.  Past 64 neighbours in
-// more than 256 dims the K-th distance sits in the bulk of the distance distribution (cfg 3,
+// slots are touched): a longer list makes that query's probes be rescanned (rescan_lists; over a
+// host base the SQ8 bounds of every probed row, one wave per (query, probe) for up to ovf_slots_of(B)
+// queries, one wave per query past that, and the rows near the top-K refined), so the lists are
+// sized to make that rare.  Past 64 neighbours in more than 256 dims the K-th distance sits in the bulk of the distance distribution (cfg 3,
 // K = 100: ~1 % of candidates pass, ~2,300 per query with a long tail), so those lists are 8x
 // deeper.  An index with a fine level keeps its base in host memory, where an overflow costs
 // most, so its lists are twice as deep again.
@@ -1443,9 +1442,9 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         b.fine_codes = ix->fine_codes;
         b.fine_qp = ix->fine_qp;
         b.fine_mode = fine ? 1 : 0;
-        b.ovf_max = KP <= 128 ? (int)w.ovf_max : 0;
+        b.ovf_max = (int)w.ovf_max;
         b.ovf_n = w.ovf_n;
-        b.ovf_q = w.ovf_q;
+        b.ovf_q = xb_host ? w.ovf_q : w.ovf_slot;  // [ovf_max] slots, or a list of [B]
         b.ovf_slot = w.ovf_slot;
         b.ovf_done = w.ovf_done;
         b.units = w.units;
@@ -1531,31 +1530,45 @@ int trident_search(const TridentIndexView* ix, const TridentSearchParams* sp, co
         m.use_prev = 0;
         m.out_d = out->topk_d;
         m.out_i = out->topk_i;
-        m.probe_cids = w.probe_cids;
-        m.nprobe = nprobe;
-        m.vec_off = ix->cluster_vec_off;
-        m.xb = ix->xb_sorted;
-        m.xq64 = w.xq64;
-        m.tile_oids = ix->tile_orig_ids;
-        m.tile_off = ix->cluster_tile_off;
-        m.T = ix->tile_size;
-        m.D = ix->D;
-        // an overflowed list is rescanned through the SQ8 bounds (rows near the top-K only)
-        m.ovf_bounds = 1;
-        m.cells = reinterpret_cast<const uint4*>(ix->sq8_cells);
-        m.vmin = ix->vmin;
-        m.delta = ix->delta;
-        m.eps = ix->eps_dim;
-        m.per_cluster = ix->per_cluster_sq8;
-        m.D_pad = ix->D_pad;
-        m.xrot64 = w.xrot64;
-        m.qerr = w.qerr;
-        m.lb_scale = a.lb_scale;
-        m.ub_scale = a.ub_scale;
-        // up to ovf_max overflowed lists are rescanned in parallel, one wave per (query, probe);
-        // without an overflow the launches find no slot and end at once
-        m.ovf_par = KP <= 128 ? 1 : 0;
-        if (m.ovf_par) {
+        if (!b.xb_host) {
+            // overflowed lists are rescanned exactly; without one the blocks end at once
+            b.probe_cids = w.probe_cids;
+            b.nprobe = nprobe;
+            m.ovf_cnt = nprobe * rescan_stride(K);
+            const unsigned rg = (unsigned)std::min<int64_t>((int64_t)B * nprobe, kRescanBlocks);
+            if (K <= 64) {
+                if (ix->D <= 256) rescan_kernel<64, 256><<<rg, kBlock, 0, st>>>(b);
+                else rescan_kernel<64, 1024><<<rg, kBlock, 0, st>>>(b);
+            } else {
+                if (ix->D <= 256) rescan_kernel<128, 256><<<rg, kBlock, 0, st>>>(b);
+                else rescan_kernel<128, 1024><<<rg, kBlock, 0, st>>>(b);
+            }
+            if ((rc = check_launch("rescan_kernel"))) return rc;
+        } else {
+            // ... and over a host base through the SQ8 bounds (rows near the top-K only)
+            m.probe_cids = w.probe_cids;
+            m.nprobe = nprobe;
+            m.vec_off = ix->cluster_vec_off;
+            m.xb = ix->xb_sorted;
+            m.xq64 = w.xq64;
+            m.tile_oids = ix->tile_orig_ids;
+            m.tile_off = ix->cluster_tile_off;
+            m.T = ix->tile_size;
+            m.D = ix->D;
+            m.ovf_bounds = 1;
+            m.cells = reinterpret_cast<const uint4*>(ix->sq8_cells);
+            m.vmin = ix->vmin;
+            m.delta = ix->delta;
+            m.eps = ix->eps_dim;
+            m.per_cluster = ix->per_cluster_sq8;
+            m.D_pad = ix->D_pad;
+            m.xrot64 = w.xrot64;
+            m.qerr = w.qerr;
+            m.lb_scale = a.lb_scale;
+            m.ub_scale = a.ub_scale;
+            // up to ovf_max overflowed lists are rescanned in parallel, one wave per (query, probe);
+            // without an overflow the launches find no slot and end at once
+            m.ovf_par = 1;
             m.ovf_max = (int)w.ovf_max;
             m.ovf_n = w.ovf_n;
             m.ovf_q = w.ovf_q;

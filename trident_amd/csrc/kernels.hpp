@@ -59,8 +59,9 @@ struct MergeArgs {
     int64_t* out_i;
     float* tau_sq_out;    // [B] or null
     // A query whose candidate list overflowed `cap` (only the batched routes append without a
-    // per-pair cap).  Mode 10's refine has replaced its list by ovf_cnt entries (the best of each
-    // probe); the cascade rescans it here through the SQ8 bounds (ovf_bounds below).
+    // per-pair cap): its list has been replaced by ovf_cnt entries, the best of each probe
+    // (rescan_lists), or, the cascade over a host base, it is rescanned here through the SQ8
+    // bounds (ovf_bounds below).
     int ovf_cnt;
     const int32_t* probe_cids;  // [B, nprobe], ovf_bounds only, as the rest
     int nprobe;
@@ -71,7 +72,7 @@ struct MergeArgs {
     const int32_t* tile_off;
     int T, D;
     unsigned long long* host_rows;  // [1] rows read by the rescan (host-mapped base), or null
-    // Bounded rescan (ovf_bounds = 1, the batched cascade route): the overflowed query's probed
+    // Bounded rescan (ovf_bounds = 1, the batched cascade route over a host base): the overflowed query's probed
     // rows get their Stage X / Y bounds from the SQ8 code cells and the per-dim parameters
     // below; only rows whose lower bound passes the K-th smallest upper bound are read and
     // refined.
@@ -210,12 +211,11 @@ struct BatchArgs {
     const uint16_t* fine_codes; // [N, D_pad] or null
     const float* fine_qp;       // [N, 4] (offset, step, rho, 0)
     int fine_mode;              // 1: seeds bounded and survivors filtered with the fine level
-    // refine_survivors_kernel gives up to ovf_max overflowed lists a slot of the parallel rescan
-    // (MergeArgs); 0: none
+    // Queries whose list overflowed.  Cascade over a host base: refine_survivors_kernel gives up
+    // to ovf_max of them a slot of the parallel rescan (MergeArgs).  Else they are listed in ovf_q
+    // [B], by fine_tau_kernel (mode 10, probe_cids not null) or the refine, for rescan_lists.
     int ovf_max;
     int32_t *ovf_n, *ovf_q, *ovf_slot, *ovf_done;
-    // mode 10 (probe_cids not null): fine_tau_kernel lists the queries whose list overflowed in
-    // ovf_q [B], and the refine's launch rescans their probes
     const int32_t* probe_cids;  // [B, nprobe]
     int nprobe;
     int cm_emit;                // cm_scan_kernel: 1 lists rows, 0 only lowers the thresholds
@@ -563,9 +563,11 @@ __global__ void lb_scan_wide_kernel(BatchArgs a);  // 4 < KS <= 16
 
 template <bool HOST, int DQ, int KP>
 __global__ void refine_survivors_kernel(BatchArgs a, int B);
-// Blocks of mode 10's refine that wait for overflowed lists (two a CU).
+template <int KP, int DQ>
+__global__ void rescan_kernel(BatchArgs a);
+// Blocks that wait for overflowed lists (two a CU).
 constexpr int kRescanBlocks = 512;
-// Entries per probe that a rescanned list of mode 10 holds (cand_cap_min gives a list the room).
+// Entries per probe that a list rescanned by rescan_lists holds (cand_cap_min gives a list the room).
 __host__ __device__ constexpr int rescan_stride(int K) { return K < 64 ? 64 : K; }
 
 // Mode 10's matrix-core scan up to 256 dims: eight waves a workgroup, 16 queries of the unit each

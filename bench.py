@@ -382,7 +382,7 @@ def measure_variant(w, nprobe, K, mode, ub, route, steps, warmup, rounds, label=
            "pruning": {"candidates": stats[0], "survivors": stats[2], "refined_kept": stats[3]}}
     if w.xb_host:
         D = w.cfg["D"]
-        # the exact refines read the base's uint8 copy when it has one (the rescan of an
+        # the exact refines read the base's uint8 copy when it has one (the cascade's rescan of an
         # overflowed candidate list reads float32 rows)
         u8 = getattr(w.st, "xb_sorted_u8", None) is not None
         rb = D if u8 else 4 * D

@@ -253,8 +253,14 @@ __device__ __forceinline__ void split3(const float (&x)[2 * N], uint32_t (&part)
 // rows, loads waited for where they were issued, and some 20 operations a pair.  Here a pair costs six
 // operations until it passes a test that every listed row passes (base against t plus a bound of
 // E), listed rows are queued in LDS and appended with one atomic per query and flush, and the
-// thresholds are read a block ahead and selected once a block: 1910 us -> 780 there, 275 -> 177 for 40
-// queries on 1e6 rows (nprobe 64), which are bound by the rows' 480 MB.
+// thresholds are read a block ahead and selected once a block: 1957 us -> 817 there (warm-up and main
+// pass), 275 -> 178 for 40 queries on 1e6 rows (nprobe 64).
+//
+// What bounds it now (10,000 queries, nprobe 64, counters): the vector unit issues in 0.56 of the slots
+// (conversion, first test, norms), the matrix cores are busy for 0.36 (828 TFLOP/s, padding of tiles
+// included), waves wait for half of their cycles at the two barriers of a block and its loads.  The 40
+// queries read 480 MB at 2.7 TB/s, half of a copy's rate: with one 16-query tile the eight waves share a
+// block's four tiles, so half of them only convert.
 template <int D4>
 __global__ __launch_bounds__(kCmThreads, D4 <= 32 ? 4 : 2) void cm_scan_kernel(BatchArgs a) {
     constexpr int DP = 4 * D4;  // D_pad
